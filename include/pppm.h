@@ -105,10 +105,10 @@ pppm_status pppm_get_device_bytes(const pppm_ctx *ctx, size_t *bytes);
 pppm_status pppm_set_graphs(pppm_ctx *ctx, int32_t on);
 /* Order in which the near field walks the sorted points (no counterpart in
  * the reference, whose near field takes one thread per point in sort order).
- * PPPM_NEAR_ORDER_AUTO (default): renumbered in super-blocks of 8x4x4 cells
- * when there are at least 4,096 points and a quarter as many as x segments,
- * and the near field's sources and cell tables (32 B a source, 8 B a cell)
- * exceed 64 MiB; in the sort's order otherwise.  _SORT: always the sort's
+ * PPPM_NEAR_ORDER_AUTO (default): the sort's order (the potential-flow near
+ * fields: renumbered in super-blocks of 8x4x4 cells when there are at least
+ * 4,096 points and a quarter as many as x segments, and the near field's
+ * sources and cell tables, 32 B a source and 8 B a cell, exceed 64 MiB).  _SORT: always the sort's
  * order.  _SUPER_BLOCKS: always renumbered.  On grids of more than 2^29
  * cells (sort keys without the octant) the order is the sort's in every
  * mode.  The orders differ in FP32 summation order only. */

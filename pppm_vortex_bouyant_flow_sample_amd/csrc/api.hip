@@ -1072,23 +1072,25 @@ struct NearOverride {
 };
 
 // Evaluation slot -> sorted point in super-block order (nearfield.hip),
-// written into the sort's spare index buffer: when the sort keys carry the
-// octant (so the spare buffer is free) and, in the automatic order, the
-// points are many enough for the slot pass to pay (at least a quarter of the
-// slots, and 4,096) and what the near field gathers (positions and
-// strengths, 32 B a source, and the cell tables, 8 B a cell) is more than
-// twice the chip's L2 (8 XCDs x 4 MiB).  Below that the sort's own order
-// keeps each XCD's gathers in its L2 and the renumbering only spreads them
-// (1M sources on 128^3: 7% slower near field).  Null otherwise: the slots
-// follow the sort.
-static pppm_status super_block_order(pppm_ctx* c, const uint32_t* keys, uint32_t m, uint32_t* spare,
+// written into the sort's spare index buffer, when the sort keys carry the
+// octant (so the spare buffer is free).  Null otherwise: the slots follow the
+// sort.  The automatic order renumbers for the potential-flow near fields only,
+// and where it pays there: points many enough for the slot pass (at least a
+// quarter of the slots, and 4,096) and more gathered bytes (positions and
+// strengths, 32 B a source, and the cell tables, 8 B a cell) than twice the
+// chip's L2 (8 XCDs x 4 MiB); at 1M sources on 128^3 the sort's order is 7%
+// faster.  The vortex near field, whose waves split a union box that wraps
+// around a row or plane, is faster in the sort's order at every size: 11.6
+// against 12.9 ms at the 8M plume on 256^3, 30.3 against 34.4 at 33.5M on
+// 512^3, 1.43 against 1.62 at 1M on 128^3.
+static pppm_status super_block_order(pppm_ctx* c, const uint32_t* keys, uint32_t m, uint32_t* spare, bool potential,
                                      uint32_t** perm) {
     *perm = nullptr;
     if (!c->octant_keys() || m == 0 || c->near_order == PPPM_NEAR_ORDER_SORT) return PPPM_OK;
     if (c->near_order == PPPM_NEAR_ORDER_AUTO) {
         constexpr size_t kSbMinGather = (size_t)64 << 20;
         const size_t gather = 32 * (size_t)c->n + 8 * c->G;
-        if (m < 4096 || m < c->sbg.nslots / 4 || gather <= kSbMinGather) return PPPM_OK;
+        if (!potential || m < 4096 || m < c->sbg.nslots / 4 || gather <= kSbMinGather) return PPPM_OK;
     }
     TRY(launch_sb_order(keys, 3u, m, c->sbg, SbBuffers{c->sb_start, c->sb_len, c->sb_pre, c->sb_scr}, spare, c->st));
     *perm = spare;
@@ -1144,7 +1146,7 @@ extern "C" pppm_status pppm_evaluate_self(pppm_ctx* c, void* ux, void* uy, void*
         perm = spare;
         TRY(launch_octant_order(c->vs.ks, c->spos, c->n, c->pg.invh, perm, c->st));
     } else {
-        TRY(super_block_order(c, c->vs.ks, c->n, spare, &perm));
+        TRY(super_block_order(c, c->vs.ks, c->n, spare, false, &perm));
     }
     return near_common(c, c->n, c->spos, nullptr, c->vs.vs, perm, ux, uy, uz, u_stride, u_dtype);
 }
@@ -1206,7 +1208,7 @@ static pppm_status eval_points(pppm_ctx* c, uint32_t m, const float* eval_pos4, 
         perm = spare;
         TRY(launch_octant_order(c->es.ks, c->epos, m, c->pg.invh, perm, st));
     } else {
-        TRY(super_block_order(c, c->es.ks, m, spare, &perm));
+        TRY(super_block_order(c, c->es.ks, m, spare, ov != nullptr, &perm));
     }
     return near_common(c, m, c->epos, other_end4 ? c->eoth : nullptr, c->es.vs, perm, ux, uy, uz, u_stride,
                        u_dtype, ov);

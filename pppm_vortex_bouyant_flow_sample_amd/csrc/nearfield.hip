@@ -3,6 +3,7 @@
 // (GPU_kernel.cu:2886-2964 BiotSavartInterpolate_far_field_kernel2,
 //  2262-2436 BiotSavartPPCorrScaleMN_kernel, BiotSavartSolverImp.cpp:452-484).
 #include "pppm_internal.hpp"
+#include <cstdlib>
 
 namespace pppm {
 
@@ -13,31 +14,33 @@ struct NearConst {
     float inv4pi;      // 1 / (4 pi) with the reference's 4 pi
     float kexp2;       // -log2(e) / a^3: exp(-(r/a)^3) = exp2(kexp2 r^3)
     float r3_series;   // 0.1 a^3: below it (x = (r/a)^3 < 0.1) the series form
-    float sc[5];       // series coefficients of (1 - e^-x) / x, times 1 / (4 pi)
+    float sc[5];       // series coefficients of (1 - e^-x) / x, times 1 / a^3
     // potential-flow kernels: core radius, the coefficient inside it
     // (1 / (4 pi a^3) for the gradient, 1 / (4 pi a) for the potential) and
     // G times the direction
     float pa, pc, pg;
 };
 
-// q(rho) / (4 pi r^3) for the expcubic core, q = 1 - exp(-(r/a)^3)
-// (GPU_kernel.cu:2389-2402), with a series for x = (r/a)^3 < 0.1 to avoid
-// cancellation.  1 / (4 pi) is folded into q (q' = q / (4 pi)), so the
-// coefficient is rinv^3 q'.  Pairs that close are rare: every lane takes the
-// exponential form, and the series runs only in waves where some lane needs
-// it (a wave-uniform branch, so other waves issue none of its instructions).
-__device__ inline float coeff_expcubic(float r2, const NearConst& nc) {
+// q(rho) / r^3 for the expcubic core, q = 1 - exp(-(r/a)^3)
+// (GPU_kernel.cu:2389-2402), 1 / (4 pi) left to the caller.  For x = (r/a)^3 <
+// 0.1 a series of (1 - e^-x) / x avoids the cancellation.  Pairs that close
+// are rare: every lane takes the exponential form (r^-3 - e r^-3 as one fused
+// multiply-add), and the series runs only in waves where some lane needs it (a
+// wave-uniform branch, so other waves issue none of its instructions).
+__device__ inline float coeff_expcubic_4pi(float r2, const NearConst& nc) {
     const float rinv = __frsqrt_rn(r2);
     const float r3 = r2 * (r2 * rinv);
-    float q = fmaf(-nc.inv4pi, __builtin_amdgcn_exp2f(nc.kexp2 * r3), nc.inv4pi);
+    const float e = __builtin_amdgcn_exp2f(nc.kexp2 * r3);
+    const float ri3 = rinv * rinv * rinv;
+    float c = fmaf(-e, ri3, ri3);
     const bool small = r3 < nc.r3_series;
     if (__ballot(small) != 0) {
         __asm__ volatile("");  // not speculated: keeps the branch a branch
         const float x = r3 * nc.inv_a3;
-        const float qs = x * (nc.sc[0] + x * (nc.sc[1] + x * (nc.sc[2] + x * (nc.sc[3] + x * nc.sc[4]))));
-        if (small) q = qs;
+        if (small)
+            c = fmaf(x, fmaf(x, fmaf(x, fmaf(x, nc.sc[4], nc.sc[3]), nc.sc[2]), nc.sc[1]), nc.sc[0]);
     }
-    return q * (rinv * rinv * rinv);
+    return c;
 }
 
 // Gaussian core: q = erf(rho/sqrt2) - sqrt(2/pi) rho exp(-rho^2/2)
@@ -169,7 +172,7 @@ __global__ void __launch_bounds__(256) k_m2p_points(const float4* __restrict__ e
     uz[dst] = (TO)sz;
 }
 
-// Cluster form: one wave takes kNearTI consecutive sorted evaluation points
+// Potential-flow near fields, in clusters: one wave takes kNearTI consecutive sorted evaluation points
 // (usually one hash cell) and splits the vortices among kNearSJ lanes per
 // point (lane = point + kNearTI * slice).  It scans the hash rows covering the
 // union of the points' boxes (consecutive x cells of a row are consecutive
@@ -180,7 +183,9 @@ __global__ void __launch_bounds__(256) k_m2p_points(const float4* __restrict__ e
 // test passes.  The point's M2P interpolation (k_m2p_points' corners and
 // weights, corner c on slice c) joins the partial sums, which are reduced
 // over the slices at the end (fixed order, deterministic).  All loop bounds
-// are wave-uniform.
+// are wave-uniform.  The vortex kernels have a layout of their own
+// (k_m2p_near); the potential's FP64 outputs hold these FP32 sums and keep
+// this order of summation.
 constexpr int kNearTI = 4;
 constexpr int kNearSJ = 64 / kNearTI;
 static_assert(kNearTI == 4, "the union box is a min / max over a quad of lanes (quad_min, quad_max)");
@@ -188,8 +193,8 @@ static_assert(kNearTI == 4, "the union box is a min / max over a quad of lanes (
 // WIDE: 64-bit vortex addressing; otherwise (fewer than 2^28 vortices) a
 // vortex's byte offset fits 32 bits and the loads take a scalar base plus a
 // 32-bit lane offset.
-template <int KERNEL, bool SEGMENT, typename TO, bool WIDE>
-__global__ void __launch_bounds__(256) k_m2p_near(const float4* __restrict__ epos, const float4* __restrict__ eoth,
+template <int KERNEL, typename TO, bool WIDE>
+__global__ void __launch_bounds__(256) k_pot_near(const float4* __restrict__ epos,
                                                   const uint32_t* __restrict__ eidx, uint32_t m,
                                                   const uint32_t* __restrict__ off, const float4* __restrict__ spos,
                                                   const float4* __restrict__ somg, const float* __restrict__ far,
@@ -250,8 +255,6 @@ __global__ void __launch_bounds__(256) k_m2p_near(const float4* __restrict__ epo
         auto sb = [&](int j) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sbnd), j)); };
         const float lox = sb(0), loy = sb(1), loz = sb(2), hix = sb(3), hiy = sb(4), hiz = sb(5);
         const uint32_t nsrc = off[G];
-        float4 bpos = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (SEGMENT) bpos = eoth[t];
         const int ny_ = yhi - ylo + 1;
         const int nrows = (xlo <= xhi && ylo <= yhi && zlo <= zhi) ? (zhi - zlo + 1) * ny_ : 0;
         // row r -> (z, y) = (r / ny_, r % ny_) through a float reciprocal
@@ -272,21 +275,13 @@ __global__ void __launch_bounds__(256) k_m2p_near(const float4* __restrict__ epo
                 const uint32_t q = sj + qq * kNearSJ;
                 const float4 s = sv[qq];
                 const float dx = a.x - s.x, dy = a.y - s.y, dz = a.z - s.z;
-                // vortex kernels: r^2 carries 1e-24, so a coincident pair has
-                // a finite coefficient and adds omega x 0 = 0 (the reference
-                // zeroes r < 1e-12) with no compare per pair
-                constexpr bool kOffset = KERNEL == PPPM_KERNEL_EXPCUBIC || KERNEL == PPPM_KERNEL_GAUSSIAN;
-                const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, kOffset ? 1e-24f : 0.f)));
+                const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, 0.f)));
                 // |d|inf <= rbox as one max3 of absolute values; a point
                 // past the end of the evaluation set (tv false) computes on
                 // a copy of its cluster's first point and is not stored
                 // (the potential keeps coincident masses: they add G m 1e-14)
-                bool acc = q < n && fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz)) <= rbox &&
-                           (kOffset || KERNEL == kNearPotScalar || r2 >= 1e-24f);
-                if (SEGMENT) {
-                    const float ex = bpos.x - s.x, ey = bpos.y - s.y, ez = bpos.z - s.z;
-                    acc = acc && ex * ex + ey * ey + ez * ez >= 1e-24f;
-                }
+                const bool acc = q < n && fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz)) <= rbox &&
+                                 (KERNEL == kNearPotScalar || r2 >= 1e-24f);
                 if (acc) {
                     const float4 o = ring[w][1][wh + q];
                     if constexpr (KERNEL == kNearPotGrad) {
@@ -298,18 +293,12 @@ __global__ void __launch_bounds__(256) k_m2p_near(const float4* __restrict__ epo
                         vx = fmaf(-c, dx, vx);
                         vy = fmaf(-c, dy, vy);
                         vz = fmaf(-c, dz, vz);
-                    } else if constexpr (KERNEL == kNearPotScalar) {
+                    } else {
                         // Potential_PPCorrMNScalar_kernel (GPU_kernel.cu:1301-1419):
                         // G m / (4 pi max(r, a)), G m 1e-14 for r < 1e-12
                         const float rinv = __frsqrt_rn(r2);
                         const float c = r2 < 1e-24f ? 1e-14f : (r2 * rinv > nc.pa ? nc.inv4pi * rinv : nc.pc);
                         vx = fmaf(nc.pg * o.x, c, vx);
-                    } else {
-                        const float cf = KERNEL == PPPM_KERNEL_GAUSSIAN ? coeff_gaussian(r2, nc)
-                                                                        : coeff_expcubic(r2, nc);
-                        vx += (o.y * dz - o.z * dy) * cf;
-                        vy += (o.z * dx - o.x * dz) * cf;
-                        vz += (o.x * dy - o.y * dx) * cf;
                     }
                 }
             }
@@ -463,23 +452,403 @@ __global__ void __launch_bounds__(256) k_m2p_near(const float4* __restrict__ epo
     }
 }
 
-template <int KERNEL, bool SEGMENT, bool WIDE>
-static void launch_sized(const NearArgs& a, const NearConst& nc, hipStream_t st) {
-    const uint32_t waves = div_up(a.m, kNearTI);
-    dim3 grid(div_up(waves, 4)), blk(256);
+// ---- vortex near field -----------------------------------------------------
+// min / max over the T points that every T consecutive lanes hold
+template <int T>
+__device__ inline float group_min(float v) {
+    v = quad_min(v);
+    if (T == 8) v = fminf(v, dpp_mov<0x124>(v));
+    return v;
+}
+template <int T>
+__device__ inline float group_max(float v) {
+    v = quad_max(v);
+    if (T == 8) v = fmaxf(v, dpp_mov<0x124>(v));
+    return v;
+}
+// v[0..T) per lane -> in lane l the sum, over the lanes that differ from l in
+// their low log2(T) bits only, of v[l % T].  Each step exchanges half of the
+// values with the lane whose next bit differs (for the third bit the lane four
+// below in the row of 16, whose higher bits are summed over later anyway).
+template <int T>
+__device__ inline float transpose_reduce(float (&v)[T], int lane) {
+#pragma unroll
+    for (int q = 0; q < T / 2; q++) {
+        const bool b = lane & 1;
+        const float keep = b ? v[2 * q + 1] : v[2 * q], give = b ? v[2 * q] : v[2 * q + 1];
+        v[q] = keep + dpp_mov<0xB1>(give);
+    }
+#pragma unroll
+    for (int q = 0; q < T / 4; q++) {
+        const bool b = lane & 2;
+        const float keep = b ? v[2 * q + 1] : v[2 * q], give = b ? v[2 * q] : v[2 * q + 1];
+        v[q] = keep + dpp_mov<0x4E>(give);
+    }
+    if (T == 8) {
+        const bool b = lane & 4;
+        const float keep = b ? v[1] : v[0], give = b ? v[0] : v[1];
+        v[0] = keep + dpp_mov<0x124>(give);
+    }
+    return v[0];
+}
+
+// One wave takes T consecutive sorted evaluation points.  Their coordinates
+// sit in scalar registers and the sources in lanes: the hash rows covering the
+// union of the points' boxes are packed into one stream of sources (), those inside the union box are compacted into a ring of
+// 128, and every full window of 64 is read back one source a lane and tested
+// against the T points in turn.  A source is read from LDS once for T points
+// (one read per pair in k_pot_near's point-by-slice layout), and a point
+// whose box holds few of a window's sources costs little, since the sources of
+// a window follow the hash rows and the lanes that fail the box test come in
+// runs.  What bounds it is the vector issue rate: 6 instructions a source and
+// point, 20 more where some lane passes.
+// A union box of more than vlim cells (points around the end of a grid row or
+// plane, or far apart in a sparse scene) is given up for two halves of the
+// points, down to single ones: before, one wave at the end of a plane walked
+// all of its rows and ran on alone (0.79 -> 0.45 ms at 700,001 uniform
+// vortices on 96^3).
+// Measured, ms a launch, k_pot_near -> here (same box, in the sort's order):
+// 8M plume 256^3 16.4 -> 11.6, 33.5M plume 512^3 45.9 -> 30.3, 2M ring 128^3
+// 28.8 -> 22.6, 1M plume 128^3 1.87 -> 1.43, 700k uniform 96^3 0.79 -> 0.37,
+// 65,536 uniform 32^3 0.153 -> 0.073.  T = 16 needs 96 VGPRs: 12.4 ms at the
+// 8M plume.
+template <int KERNEL, bool SEGMENT, typename TO, bool WIDE, int T>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T == 8 ? 7 : 8)))
+k_m2p_near(const float4* __restrict__ epos, const float4* __restrict__ eoth, const uint32_t* __restrict__ eidx, uint32_t m,
+       const uint32_t* __restrict__ off, const float4* __restrict__ spos, const float4* __restrict__ somg,
+       const float* __restrict__ far, uint32_t g, double invh, NearConst nc, int vlim, TO* __restrict__ ux,
+       TO* __restrict__ uy, TO* __restrict__ uz, uint32_t u_stride, const uint32_t* __restrict__ tperm) {
+    static_assert(T == 4 || T == 8, "group_min, group_max and transpose_reduce");
+    __shared__ float4 ring[4][2][128];
+    const int lane0 = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // groups of 256 consecutive workgroups per XCD, so each L2 serves one run
+    // of points whose boxes share most of their hash rows
+    const uint32_t wg = xcd_group<256>(blockIdx.x, gridDim.x);
+    const uint32_t t0 = (wg * 4 + w) * T;
+    if (t0 >= m) return;  // the whole wave leaves together; no block barriers below
+    const uint32_t slot = t0 + lane0 % T;
+    const bool tv = slot < m;
+    // evaluation slot -> sorted point; a slot past the end takes the first
+    // slot's point and is neither in a group nor stored
+    const uint32_t t = tperm ? tperm[tv ? slot : t0] : (tv ? slot : t0);
+    const float4 a0 = epos[t];
+    const int gi = (int)g;
+    const size_t G = (size_t)g * g * g;
+    auto lanef = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+    const double rb = (double)nc.rbox;
+    const float rbox = nc.rbox;
+    // the points' y and z (and other ends), in scalar registers
+    constexpr int TS = SEGMENT ? T : 1;
+    float py[T], pz[T], qx[TS], qy[TS], qz[TS];
+#pragma unroll
+    for (int p = 0; p < T; p++) {
+        py[p] = lanef(a0.y, p);
+        pz[p] = lanef(a0.z, p);
+    }
+    if (SEGMENT) {
+        const float4 bp = eoth[t];
+#pragma unroll
+        for (int p = 0; p < TS; p++) {
+            qx[p] = lanef(bp.x, p);
+            qy[p] = lanef(bp.y, p);
+            qz[p] = lanef(bp.z, p);
+        }
+    }
+    const uint32_t nsrc = off[G];
+    int sz = T;
+    for (int s0 = 0; s0 < T; s0 += sz) {
+        // group [s0, s0 + sz) of the points; after the first, aligned powers
+        // of two
+        if (s0 > 0) sz = s0 & -s0;
+        // opaque in every pass, so that nothing of a pass is kept in registers
+        // for the next (there is one pass in most waves)
+        float4 a = a0;
+        int lane = lane0;
+        __asm__ volatile("" : "+v"(a.x), "+v"(a.y), "+v"(a.z), "+v"(lane));
+        const int ti = lane % T, sj = lane / T;
+        // ---- union of the group's boxes -> scanned cell range (wave-uniform).
+        // A NaN coordinate stays out of the union (all-NaN: an empty range).
+        // Lane j < 6 computes one axis's bounds (j = axis: lower, 3 + axis:
+        // upper): the cell range and the staging bound.  Every vortex the box
+        // test can accept lies strictly inside the staging bounds: the test
+        // keeps fl(|p - s|) <= rbox, so |p - s| <= rbox (1 + 2^-23) exactly, and
+        // s > min - rbox (1 + 2^-21) >= lo, with lo that bound rounded down (hi:
+        // max + rbox (1 + 2^-21) rounded up).
+        int xlo, ylo, zlo, xhi, yhi, zhi, ny_, nrows;
+        float lox, loy, loz, hix, hiy, hiz;
+        for (;;) {
+            const bool in = tv && ti >= s0 && ti < s0 + sz;
+            const bool okx = in && a.x == a.x, oky = in && a.y == a.y, okz = in && a.z == a.z;
+            const float mnx = group_min<T>(okx ? a.x : 3.0e38f), mny = group_min<T>(oky ? a.y : 3.0e38f),
+                        mnz = group_min<T>(okz ? a.z : 3.0e38f);
+            const float mxx = group_max<T>(okx ? a.x : -3.0e38f), mxy = group_max<T>(oky ? a.y : -3.0e38f),
+                        mxz = group_max<T>(okz ? a.z : -3.0e38f);
+            const int bj = lane < 6 ? lane : 0;
+            const bool bup = bj >= 3;
+            const int bax = bup ? bj - 3 : bj;
+            const float bvv = bax == 0 ? (bup ? mxx : mnx) : bax == 1 ? (bup ? mxy : mny) : (bup ? mxz : mnz);
+            const int cbnd = near_cell_bound(bvv, rb, invh, gi, bup);
+            xlo = __builtin_amdgcn_readlane(cbnd, 0);
+            ylo = __builtin_amdgcn_readlane(cbnd, 1);
+            zlo = __builtin_amdgcn_readlane(cbnd, 2);
+            xhi = __builtin_amdgcn_readlane(cbnd, 3);
+            yhi = __builtin_amdgcn_readlane(cbnd, 4);
+            zhi = __builtin_amdgcn_readlane(cbnd, 5);
+            ny_ = yhi - ylo + 1;
+            nrows = (xlo <= xhi && ylo <= yhi && zlo <= zhi) ? (zhi - zlo + 1) * ny_ : 0;
+            if (sz > 1 && nrows * (xhi - xlo + 1) > vlim) {
+                sz >>= 1;
+                continue;
+            }
+            const float sbnd = near_stage_bound(bvv, rb * (1.0 + 0x1p-21), bup);
+            lox = lanef(sbnd, 0);
+            loy = lanef(sbnd, 1);
+            loz = lanef(sbnd, 2);
+            hix = lanef(sbnd, 3);
+            hiy = lanef(sbnd, 4);
+            hiz = lanef(sbnd, 5);
+            break;
+        }
+        // row r -> (z, y) = (r / ny_, r % ny_) through a float reciprocal
+        // (within 1 ulp): exact while r < 2^21 (nrows <= g^2 <= 2^20)
+        const float inv_ny = __builtin_amdgcn_rcpf((float)max(ny_, 1));
+        // x of the points, -inf outside the group: no source passes their box
+        // test (a lane past the window's end holds +inf in all coordinates)
+        float px[T], vx[T], vy[T], vz[T];
+#pragma unroll
+        for (int p = 0; p < T; p++) {
+            px[p] = p >= s0 && p < s0 + sz ? lanef(a.x, p) : -__builtin_inff();
+            vx[p] = vy[p] = vz[p] = 0.f;
+        }
+        // Evaluate the window [wh, wh + n) of the ring (wh is 0 or 64).
+        auto evaluate = [&](uint32_t wh, uint32_t n) {
+            float4 s = ring[w][0][wh + lane];
+            const float4 o = ring[w][1][wh + lane];
+            if ((uint32_t)lane >= n) s.x = s.y = s.z = __builtin_inff();
+#pragma unroll
+            for (int p = 0; p < T; p++) {
+                const float dx = px[p] - s.x, dy = py[p] - s.y, dz = pz[p] - s.z;
+                // |d|inf <= rbox as one max3 of absolute values
+                bool acc = fmaxf(fmaxf(fabsf(dx), fabsf(dy)), fabsf(dz)) <= rbox;
+                if (SEGMENT) {
+                    const int ps = SEGMENT ? p : 0;
+                    const float ex = qx[ps] - s.x, ey = qy[ps] - s.y, ez = qz[ps] - s.z;
+                    acc = acc && ex * ex + ey * ey + ez * ez >= 1e-24f;
+                }
+                if (acc) {
+                    // r^2 carries 1e-24, so a coincident pair has a finite
+                    // coefficient and adds omega x 0 = 0 (the reference zeroes
+                    // r < 1e-12) with no compare per pair
+                    const float r2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, 1e-24f)));
+                    const float cf =
+                        KERNEL == PPPM_KERNEL_GAUSSIAN ? coeff_gaussian(r2, nc) : coeff_expcubic_4pi(r2, nc);
+                    vx[p] += (o.y * dz - o.z * dy) * cf;
+                    vy[p] += (o.z * dx - o.x * dz) * cf;
+                    vz[p] += (o.x * dy - o.y * dx) * cf;
+                }
+            }
+            // the next staging may overwrite these entries
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        };
+        // ring state (wave-uniform): window head (0 or 64) and entries held
+        uint32_t qh = 0, qn = 0;
+        for (int r0 = 0; r0 < nrows; r0 += 64) {
+            // lane l holds the vortex range [lp0, lp1) of row r0 + l (z outer,
+            // y inner), loaded in one pass
+            uint32_t lp0 = 0, lp1 = 0;
+            if (r0 + lane < nrows) {
+                const int r = r0 + lane;
+                const int rz = (int)(((float)r + 0.5f) * inv_ny);
+                const uint32_t kk = (uint32_t)(zlo + rz), jj = (uint32_t)(ylo + r - rz * ny_);
+                const uint32_t rowc = (kk * g + jj) * g;
+                lp0 = off[rowc + xlo];
+                lp1 = min(off[rowc + xhi + 1], nsrc);
+            }
+            const int rn = min(64, nrows - r0);
+            // The rows are packed into one stream of vortices: chunk c holds
+            // stream positions 64 c .. 64 c + 63 across row boundaries.  pre
+            // is a row's first stream position (exclusive prefix of the row
+            // lengths), roff maps stream position to vortex index.
+            const uint32_t len = lp1 > lp0 ? lp1 - lp0 : 0u;
+            const uint32_t incl = wave_inclusive_scan(len);
+            const uint32_t pre = incl - len, roff = lp0 - pre;
+            const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
+            // vortex index of this lane's position in the chunk at S0; rcur
+            // (wave-uniform) is a row at or before the one holding S0 and is
+            // advanced to the last row starting at or before S0 + 64
+            auto locate = [&](uint32_t S0, int& rcur) {
+                const uint32_t S = S0 + (uint32_t)lane;
+                uint32_t mo = __builtin_amdgcn_readlane(roff, rcur);
+                int rnext = rcur;
+                for (int rr = rcur + 1; rr < rn; rr++) {
+                    const uint32_t p = __builtin_amdgcn_readlane(pre, rr);
+                    if (p > S0 + 64) break;
+                    rnext = rr;
+                    if (S >= p) mo = __builtin_amdgcn_readlane(roff, rr);
+                }
+                rcur = rnext;
+                return S + mo;
+            };
+            int rc = 0;
+            // The next chunk is loaded into registers while this one is
+            // staged.  Slots past the end of the stream (pin false) read
+            // vortex 0 and are not staged.
+            float4 pp = make_float4(0.f, 0.f, 0.f, 0.f), po = pp;
+            float lxl = __builtin_inff();
+            auto load = [&](uint32_t S0) {
+                const uint32_t vi = locate(S0, rc);
+                const bool pin = S0 + (uint32_t)lane < total;
+                lxl = pin ? lox : __builtin_inff();  // a slot past the end fails the filter
+                const uint32_t v = pin ? vi : 0u;
+                if (WIDE) {
+                    pp = spos[v];
+                    po = somg[v];
+                } else {
+                    const uint32_t ob = v << 4;
+                    pp = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(spos) + ob);
+                    po = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(somg) + ob);
+                }
+            };
+            if (total > 0) load(0u);
+            for (uint32_t S0 = 0; S0 < total; S0 += 64) {
+                // Stage only the vortices inside the staging bounds on every
+                // axis: the lane masks of the six compares (ordered: NaN
+                // fails) ANDed on the scalar unit, then the mask as the
+                // predicate
+                const uint64_t bal =
+                    __builtin_amdgcn_fcmpf(pp.x, lxl, 2) & __builtin_amdgcn_fcmpf(pp.x, hix, 4) &
+                    __builtin_amdgcn_fcmpf(pp.y, loy, 2) & __builtin_amdgcn_fcmpf(pp.y, hiy, 4) &
+                    __builtin_amdgcn_fcmpf(pp.z, loz, 2) & __builtin_amdgcn_fcmpf(pp.z, hiz, 4);
+                const bool use = __builtin_amdgcn_inverse_ballot_w64(bal);
+                // ring slot: the head plus the kept lanes below this one
+                const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)bal, qh + qn));
+                if (use) {
+                    const uint32_t e = at & 127u;
+                    ring[w][0][e] = pp;
+                    ring[w][1][e] = po;
+                }
+                qn += (uint32_t)__popcll(bal);
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                if (S0 + 64 < total) load(S0 + 64);
+                // a full window: evaluate it and move the head to the other
+                if (qn >= 64) {
+                    evaluate(qh, 64u);
+                    qh ^= 64u;
+                    qn -= 64u;
+                }
+            }
+        }
+        if (qn > 0) evaluate(qh, qn);  // the last, partial window
+        // ---- lane l: point l % T.  1 / (4 pi) is applied here, once a point
+        // (the Gaussian coefficient holds it)
+        float rx = transpose_reduce<T>(vx, lane), ry = transpose_reduce<T>(vy, lane),
+              rz = transpose_reduce<T>(vz, lane);
+        if (KERNEL != PPPM_KERNEL_GAUSSIAN) {
+            rx *= nc.inv4pi;
+            ry *= nc.inv4pi;
+            rz *= nc.inv4pi;
+        }
+        // ---- M2P: the point's 8 interpolation corners, corner sj on slice sj
+        // (the weights and validity of k_m2p_points), into the sums
+        if (sj < 8 && tv) {
+            const int i = cell_of(a.x, invh), j = cell_of(a.y, invh), k = cell_of(a.z, invh);
+            const bool fin = a.x == a.x && a.y == a.y && a.z == a.z;
+            if (fin && i >= 0 && i < gi && j >= 0 && j < gi && k >= 0 && k < gi) {
+                const double xh = (double)a.x * invh - 0.5, yh = (double)a.y * invh - 0.5,
+                             zh = (double)a.z * invh - 0.5;
+                const int i0 = (int)floor(xh), j0 = (int)floor(yh), k0 = (int)floor(zh);
+                const float fx = (float)(xh - i0), fy = (float)(yh - j0), fz = (float)(zh - k0);
+                const int a2 = sj & 1, b2 = (sj >> 1) & 1, c2 = sj >> 2;
+                const bool ok =
+                    (a2 ? i0 + 1 < gi : i0 >= 0) && (b2 ? j0 + 1 < gi : j0 >= 0) && (c2 ? k0 + 1 < gi : k0 >= 0);
+                if (ok) {
+                    const uint32_t q = (((uint32_t)k0 + (uint32_t)c2) * g + (uint32_t)j0 + (uint32_t)b2) * g +
+                                       (uint32_t)i0 + (uint32_t)a2;
+                    const float wgt = (a2 ? fx : 1.f - fx) * (b2 ? fy : 1.f - fy) * (c2 ? fz : 1.f - fz);
+                    rx = fmaf(wgt, far[q], rx);
+                    ry = fmaf(wgt, far[G + q], ry);
+                    rz = fmaf(wgt, far[2 * G + q], rz);
+                }
+            }
+        }
+        // ---- the lanes of a point (a fixed order)
+        if (T == 4) {
+            rx += dpp_mov<0x124>(rx);
+            ry += dpp_mov<0x124>(ry);
+            rz += dpp_mov<0x124>(rz);
+        }
+        rx += dpp_mov<0x128>(rx);
+        ry += dpp_mov<0x128>(ry);
+        rz += dpp_mov<0x128>(rz);
+        for (int o = 16; o < 64; o <<= 1) {
+            rx += __shfl_xor(rx, o, 64);
+            ry += __shfl_xor(ry, o, 64);
+            rz += __shfl_xor(rz, o, 64);
+        }
+        if (lane < T && tv && lane >= s0 && lane < s0 + sz) {
+            const uint32_t dt = eidx[t];
+            if (dt < m) {
+                const size_t dst = (size_t)dt * u_stride;
+                ux[dst] = (TO)rx;
+                uy[dst] = (TO)ry;
+                uz[dst] = (TO)rz;
+            }
+        }
+    }
+}
+
+template <int KERNEL, bool SEGMENT, bool WIDE, int T>
+static void launch_near_sized(const NearArgs& a, const NearConst& nc, hipStream_t st) {
+    // A group's union box: at most five times a single point's cells (a box
+    // of 2K + 1 cells, one more where it straddles).  Limits of 2, 3, 5, 7 and
+    // 12 boxes: 0.71, 0.55, 0.37, 0.36 and 0.37 ms at 700,001 uniform vortices
+    // on 96^3; 16.3, 15.5 at the 8M plume (2, 3), then unchanged; 65,536
+    // uniform on 32^3: 0.073 ms at 5, 0.083 at 7.
+    const int vlim = 5 * (2 * a.K + 2) * (2 * a.K + 2) * (2 * a.K + 2);
+    dim3 grid(div_up(div_up(a.m, T), 4)), blk(256);
     if (a.u_dtype == PPPM_F64)
-        hipLaunchKernelGGL((k_m2p_near<KERNEL, SEGMENT, double, WIDE>), grid, blk, 0, st, a.epos, a.eoth, a.eidx,
-                           a.m, a.off, a.spos, a.somg, a.far, a.g, a.K, a.invh, nc, (double*)a.ux, (double*)a.uy,
+        hipLaunchKernelGGL((k_m2p_near<KERNEL, SEGMENT, double, WIDE, T>), grid, blk, 0, st, a.epos, a.eoth, a.eidx, a.m,
+                           a.off, a.spos, a.somg, a.far, a.g, a.invh, nc, vlim, (double*)a.ux, (double*)a.uy,
                            (double*)a.uz, a.u_stride, a.tperm);
     else
-        hipLaunchKernelGGL((k_m2p_near<KERNEL, SEGMENT, float, WIDE>), grid, blk, 0, st, a.epos, a.eoth, a.eidx,
-                           a.m, a.off, a.spos, a.somg, a.far, a.g, a.K, a.invh, nc, (float*)a.ux, (float*)a.uy,
+        hipLaunchKernelGGL((k_m2p_near<KERNEL, SEGMENT, float, WIDE, T>), grid, blk, 0, st, a.epos, a.eoth, a.eidx, a.m,
+                           a.off, a.spos, a.somg, a.far, a.g, a.invh, nc, vlim, (float*)a.ux, (float*)a.uy,
                            (float*)a.uz, a.u_stride, a.tperm);
 }
 template <int KERNEL, bool SEGMENT>
-static void launch_typed(const NearArgs& a, const NearConst& nc, hipStream_t st) {
-    if (a.nsrc >= (1u << 28)) launch_sized<KERNEL, SEGMENT, true>(a, nc, st);
-    else launch_sized<KERNEL, SEGMENT, false>(a, nc, st);
+static void launch_near(const NearArgs& a, const NearConst& nc, hipStream_t st) {
+    // Eight points a wave once that is two rounds of resident waves (256 CUs
+    // x 28); below, four points keep more waves in flight (10,007 points:
+    // 0.031 against 0.050 ms; 65,536: 0.073 against 0.079; 1M: 1.57 against
+    // 1.43).
+    const bool t8 = a.m > 8u * 2u * 256u * 28u;
+    const bool wide = a.nsrc >= (1u << 28);
+    if (t8 && wide) launch_near_sized<KERNEL, SEGMENT, true, 8>(a, nc, st);
+    else if (t8) launch_near_sized<KERNEL, SEGMENT, false, 8>(a, nc, st);
+    else if (wide) launch_near_sized<KERNEL, SEGMENT, true, 4>(a, nc, st);
+    else launch_near_sized<KERNEL, SEGMENT, false, 4>(a, nc, st);
+}
+
+template <int KERNEL, bool WIDE>
+static void launch_pot_sized(const NearArgs& a, const NearConst& nc, hipStream_t st) {
+    const uint32_t waves = div_up(a.m, kNearTI);
+    dim3 grid(div_up(waves, 4)), blk(256);
+    if (a.u_dtype == PPPM_F64)
+        hipLaunchKernelGGL((k_pot_near<KERNEL, double, WIDE>), grid, blk, 0, st, a.epos, a.eidx, a.m, a.off, a.spos, a.somg, a.far, a.g, a.K, a.invh, nc, (double*)a.ux, (double*)a.uy,
+                           (double*)a.uz, a.u_stride, a.tperm);
+    else
+        hipLaunchKernelGGL((k_pot_near<KERNEL, float, WIDE>), grid, blk, 0, st, a.epos, a.eidx, a.m, a.off, a.spos, a.somg, a.far, a.g, a.K, a.invh, nc, (float*)a.ux, (float*)a.uy,
+                           (float*)a.uz, a.u_stride, a.tperm);
+}
+template <int KERNEL>
+static void launch_pot(const NearArgs& a, const NearConst& nc, hipStream_t st) {
+    if (a.nsrc >= (1u << 28)) launch_pot_sized<KERNEL, true>(a, nc, st);
+    else launch_pot_sized<KERNEL, false>(a, nc, st);
 }
 
 // ---- evaluation order in super-blocks ------------------------------------
@@ -487,11 +856,11 @@ static void launch_typed(const NearArgs& a, const NearConst& nc, hipStream_t st)
 // renumbered so that consecutive evaluation slots walk one super-block of
 // kSbX x kSbY x kSbZ cells (its rows z, then y, each an x segment of kSbX
 // cells) before the next super-block (blocks in z, y, x order).  Consecutive
-// clusters go to one XCD in groups of 256 workgroups, about 4,096 points, and
-// in this order such a run is a compact region whose hash rows fit that XCD's
-// L2: at 8M/256^3 the near field's HBM traffic falls from 8.4 to 3.7 GB per
-// launch and its time from 17.4 to 14.5 ms (blocks of 4x4x4 and 16x4x4 run
-// the same, 8x2x2 16.8 ms, 8x8x8 17.9 ms).
+// clusters go to one XCD in groups of 256 workgroups, about 4,096 points of
+// k_pot_near, and in this order such a run is a compact region whose hash rows
+// fit that XCD's L2 (17.4 -> 14.5 ms at 8M/256^3 for waves of four points that
+// do not split their union box; blocks of 4x4x4 and 16x4x4 the same, 8x2x2
+// 16.8 ms, 8x8x8 17.9 ms).
 constexpr uint32_t kSbX = 8, kSbY = 4, kSbZ = 4;
 
 SbGeom sb_geom(uint32_t g) {
@@ -619,7 +988,7 @@ pppm_status launch_m2p_near(const NearArgs& a, hipStream_t st) {
     nc.r3_series = (float)(0.1 * a.core_a * a.core_a * a.core_a);
     {
         const double c[5] = {1.0, -0.5, 1.0 / 6.0, -1.0 / 24.0, 1.0 / 120.0};
-        for (int k = 0; k < 5; k++) nc.sc[k] = (float)(c[k] / kRefFourPi);
+        for (int k = 0; k < 5; k++) nc.sc[k] = (float)(c[k] / (a.core_a * a.core_a * a.core_a));
     }
     (void)h;
     if (a.K < 0) {
@@ -642,17 +1011,17 @@ pppm_status launch_m2p_near(const NearArgs& a, hipStream_t st) {
         nc.pc = (float)(a.kernel == kNearPotGrad ? 1.0 / (kRefFourPi * ca * ca * ca) : 1.0 / (kRefFourPi * ca));
         nc.pg = (float)a.pot_g;
         if (seg) return PPPM_ERR_INVALID;
-        if (a.kernel == kNearPotGrad) launch_typed<kNearPotGrad, false>(a, nc, st);
-        else launch_typed<kNearPotScalar, false>(a, nc, st);
+        if (a.kernel == kNearPotGrad) launch_pot<kNearPotGrad>(a, nc, st);
+        else launch_pot<kNearPotScalar>(a, nc, st);
         PPPM_LAUNCH_CHECK();
         return PPPM_OK;
     }
     if (a.kernel == PPPM_KERNEL_GAUSSIAN) {
-        if (seg) launch_typed<PPPM_KERNEL_GAUSSIAN, true>(a, nc, st);
-        else launch_typed<PPPM_KERNEL_GAUSSIAN, false>(a, nc, st);
+        if (seg) launch_near<PPPM_KERNEL_GAUSSIAN, true>(a, nc, st);
+        else launch_near<PPPM_KERNEL_GAUSSIAN, false>(a, nc, st);
     } else {
-        if (seg) launch_typed<PPPM_KERNEL_EXPCUBIC, true>(a, nc, st);
-        else launch_typed<PPPM_KERNEL_EXPCUBIC, false>(a, nc, st);
+        if (seg) launch_near<PPPM_KERNEL_EXPCUBIC, true>(a, nc, st);
+        else launch_near<PPPM_KERNEL_EXPCUBIC, false>(a, nc, st);
     }
     PPPM_LAUNCH_CHECK();
     return PPPM_OK;
