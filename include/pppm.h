@@ -322,7 +322,10 @@ pppm_status pppm_mg_smooth(pppm_mg *mg, void *x, const void *b, int32_t iters, d
  * prolongation. */
 pppm_status pppm_mg_set_blocked(pppm_mg *mg, int32_t blocked);
 /* Levels with at least this many cells per component take the blocked
- * passes in PPPM_F32 V-cycles (default 256K: 64^3 and larger). */
+ * passes in PPPM_F32 V-cycles (default 512K: 81^3 and larger); smaller ones
+ * of even dimensions take tile passes (two red-black iterations with the
+ * residual or the prolongation in one launch), others one launch per
+ * half-sweep. */
 pppm_status pppm_mg_set_blocked_min_cells(pppm_mg *mg, uint64_t cells);
 /* PPPM_F32 V-cycles: one_launch = 1 (the default) runs the level above the
  * coarsest (when it is below that threshold and has at most 4096 cells, as

@@ -35,22 +35,28 @@ __device__ inline T nb_sum(const T* __restrict__ x, size_t t, int i, int j, int 
     return r;
 }
 
-// SOR update of cell (i, j, k) of one component: x from its neighbours and
-// bscale times the cell's right-hand side bv (k_rbgs, and k_vtail on a level
-// held in LDS).
+// Relaxation factor over the diagonal 6 - beta nout of a cell with nout
+// neighbours outside and a ghost factor beta; 0 stands for omega / 6.
+template <typename T>
+__device__ inline T rbgs_weight(int nout, T omega, T beta) {
+    return beta == (T)0 || nout == 0 ? (T)0 : omega / ((T)6 - beta * (T)nout);
+}
+// SOR update of a cell: x from the sum r of its neighbours, bscale times its
+// right-hand side bv and its rbgs_weight w (k_rbgs; k_vtail on a level held in
+// LDS, which forms w once for all its half-sweeps).
+template <typename T>
+__device__ inline T rbgs_value(T x, T r, T bv, T bscale, T w, T omega) {
+    r -= bscale * bv;
+    const T s = w != (T)0 ? w * r : omega * r * (T)(1.0 / 6.0);
+    return ((T)1 - omega) * x + s;
+}
 template <typename T>
 __device__ inline void rbgs_point(T* xc, T bv, T bscale, int i, int j, int k, int nx, int ny, int nz, T omega,
                                   T beta) {
     const size_t t = ((size_t)k * ny + j) * nx + i;
     int nout;
-    T r = nb_sum(xc, t, i, j, k, nx, ny, nz, nout);
-    r -= bscale * bv;
-    T xn;
-    if (beta == (T)0 || nout == 0)
-        xn = ((T)1 - omega) * xc[t] + omega * r * (T)(1.0 / 6.0);
-    else
-        xn = ((T)1 - omega) * xc[t] + omega * r / ((T)6 - beta * (T)nout);
-    xc[t] = xn;
+    const T r = nb_sum(xc, t, i, j, k, nx, ny, nz, nout);
+    xc[t] = rbgs_value(xc[t], r, bv, bscale, rbgs_weight(nout, omega, beta), omega);
 }
 
 // One colour of red-black SOR.  color 1 = (i+j+k) odd (swept first, as the
@@ -779,11 +785,277 @@ __global__ void __launch_bounds__(256) k_prolong(T* __restrict__ x, const T* __r
         prolong_point(xc + (size_t)comp * Gc, i, j, k, nx, ny, nz, cx, cy, cz, mode, betac);
 }
 
+// ---- small levels: up to two red-black iterations of a 3-D tile in LDS -------
+// One launch does what used to take a launch per half-sweep (and one each for
+// the zero fill, the residual with its restriction and the prolongation): on
+// levels of up to a million cells such launches are latency (4 to 5 us each
+// for a level of 32^3, whatever it holds).  A workgroup loads its TI^3 tile
+// with an H-cell halo (H = one cell per half-sweep, one more for the residual;
+// clipped at the grid), applies the half-sweeps in LDS with the halo
+// recomputed, and writes its tile: out of place, as the halos are other
+// workgroups' tiles.  A cell at distance d from a side of the loaded region
+// that is not a grid boundary is right for the first d half-sweeps.
+//
+// LDS holds the two colours apart: colour c of plane z, row y has at index m
+// the colour-c cell of the pair (2m, 2m + 1), x counted from the region's even
+// lower corner, with one zero row, plane and index around it for the ghosts
+// (and for what a region side that is no boundary reads: those cells are in
+// the discarded halo).  A thread owns the pairs (m, y) of a run of planes, in
+// registers with their right-hand sides.  Of the six neighbours of a cell,
+// all of the other colour, the pair's other cell and the same cell of the
+// planes above and below are the thread's own; the other x neighbour and the
+// two in y come from LDS (three reads and a write an update, at immediate
+// offsets from three registers).  Vector issue and LDS are about even.
+//
+// us of one V(2,2) cycle's level, three components, before -> here: 32^3 50
+// (11 launches) -> 16.5 (2), 64^3 51 (k_rbc) -> 34; FP64, one component: V(4,4)
+// at 64^3 and below 19 launches of 4.2 -> 4 of 11.  96^3: 92 against 83 with
+// k_rbc, so the line to the blocked passes lies at 512K cells.  1024 threads
+// take a 16^3 tile, 576 an 8^3 one.
+template <typename T>
+struct TileArgs {
+    const T* xin;  // level before the pass (null: zero)
+    T* x;          // level after the pass (another buffer)
+    const T* b;
+    T bscale;
+    int nx, ny, nz;
+    size_t G;
+    T omega, beta;
+    int iters;  // 1 or 2
+    int tx, ty, tz;
+    // residual restricted into bn (null: none), coarse dims n / 2
+    T* bn;
+    int cx, cy, cz;
+    size_t Gc;
+    // x += prolongation of xc on load (null: none)
+    const T* xc;
+    T betac;
+    int mode;
+};
+
+constexpr int tile_threads(int TI) { return TI == 16 ? 1024 : 576; }
+
+template <typename T, int TI, bool BETA>
+__global__ void __launch_bounds__(tile_threads(TI)) k_tile(TileArgs<T> a) {
+    constexpr int NT = tile_threads(TI);
+    constexpr int HP = TI / 2 + 6;                // pairs per row: TI + 5 above, TI - 6 below, even
+    constexpr int RY = TI + 10;                   // rows and planes
+    constexpr int PX = HP + 1, PY = RY + 2, PZ = PY * PX;
+    constexpr int PC = (RY + 2) * PZ + 1;         // a colour, with the ghosts
+    constexpr int NGMIN = NT / (HP * RY);         // column groups when the region is largest
+    constexpr int KQ = (RY + NGMIN - 1) / NGMIN;  // planes per thread
+    constexpr int CW = TI / 2 + 6;                // coarse window per axis
+    constexpr int RW = TI / 2;
+    constexpr int AUX = CW * CW * CW > TI * TI * RW ? CW * CW * CW : TI * TI * RW;
+    __shared__ T xs[2 * PC];
+    __shared__ T aux[AUX];  // coarse window while loading, pair residuals at the end
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const int bx = blockIdx.x % a.tx, by = (blockIdx.x / a.tx) % a.ty, bz = blockIdx.x / (a.tx * a.ty);
+    const int comp = blockIdx.y;
+    const int H = 2 * a.iters + (a.bn ? 1 : 0);
+    const int t0x = bx * TI, t0y = by * TI, t0z = bz * TI;
+    const int x0 = max(t0x - H, 0) & ~1, x1 = min(t0x + TI + H, nx);
+    const int y0 = max(t0y - H, 0), y1 = min(t0y + TI + H, ny);
+    const int z0 = max(t0z - H, 0), z1 = min(t0z + TI + H, nz);
+    const int hp = (x1 - x0 + 1) >> 1, ry = y1 - y0, rz = z1 - z0;
+    const T* xin = a.xin ? a.xin + (size_t)comp * a.G : nullptr;
+    const T* b = a.b + (size_t)comp * a.G;
+    const int tid = threadIdx.x;
+    // thread -> column (m, yy), planes zb .. zb + nq - 1 of the region
+    const int ncol = hp * ry, NG = NT / ncol;    // NG >= NGMIN
+    const int kq = (rz + NG - 1) / NG;           // <= KQ
+    const int col = tid % ncol, grp = tid / ncol;
+    const int m = col % hp, yy = col / hp;
+    const int zb = grp * kq;
+    const int nq = grp < NG ? min(kq, rz - zb) : 0;  // <= 0: no planes
+    const int gi = x0 + 2 * m, gj = y0 + yy, gk0 = z0 + zb;
+    const bool two = gi + 1 < x1;  // the pair's second cell exists
+    // colour of the first cell of plane zb + q: p ^ (q & 1)
+    const int p = (gj + gk0) & 1;
+
+    // right-hand sides and starting values by colour, all loads in flight
+    // together (a pair that does not exist reads the component's first cells)
+    T bc[2][KQ], xr[2][KQ];
+    const int o1 = two ? 1 : 0;
+#pragma unroll
+    for (int q = 0; q < KQ; q++) {
+        const bool ok = q < nq;
+        const size_t t = ok ? ((size_t)(gk0 + q) * ny + gj) * nx + gi : 0;
+        bc[0][q] = b[t];
+        bc[1][q] = b[t + (ok ? o1 : 0)];
+    }
+    if (xin) {
+#pragma unroll
+        for (int q = 0; q < KQ; q++) {
+            const bool ok = q < nq;
+            const size_t t = ok ? ((size_t)(gk0 + q) * ny + gj) * nx + gi : 0;
+            xr[0][q] = xin[t];
+            xr[1][q] = xin[t + (ok ? o1 : 0)];
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < KQ; q++) xr[0][q] = xr[1][q] = (T)0;
+    }
+    for (int q = tid; q < 2 * PC; q += NT) xs[q] = (T)0;
+    const int c0x = (x0 >> 1) - 1, c0y = (y0 >> 1) - 1, c0z = (z0 >> 1) - 1;
+    if (a.xc) {
+        // window c0 .. of the coarse level; a cell outside holds its nearest
+        // in-grid cell, betac times per axis for the trilinear transfer
+        const T* xc = a.xc + (size_t)comp * a.Gc;
+        const T gb = a.mode == PROLONG_TRILINEAR ? a.betac : (T)1;
+        constexpr int NC = (CW * CW * CW + NT - 1) / NT;
+        T cv[NC];
+#pragma unroll
+        for (int u = 0; u < NC; u++) {
+            const int q = min(tid + NT * u, CW * CW * CW - 1);
+            const int cx_ = c0x + q % CW, cy_ = c0y + (q / CW) % CW, cz_ = c0z + q / (CW * CW);
+            const int ix = min(max(cx_, 0), a.cx - 1), iy = min(max(cy_, 0), a.cy - 1), iz = min(max(cz_, 0), a.cz - 1);
+            const T f = (ix != cx_ ? gb : (T)1) * (iy != cy_ ? gb : (T)1) * (iz != cz_ ? gb : (T)1);
+            cv[u] = f * xc[((size_t)iz * a.cy + iy) * a.cx + ix];
+        }
+#pragma unroll
+        for (int u = 0; u < NC; u++) aux[min(tid + NT * u, CW * CW * CW - 1)] = cv[u];
+    }
+    __syncthreads();
+    // index of the pair in a plane of one colour; a thread without planes
+    // stays at the first ghost row, which it neither reads nor writes
+    T* const X = xs + (nq > 0 ? (zb + 1) * PZ + (yy + 1) * PX + m + 1 : PZ + 1);
+#pragma unroll
+    for (int q = 0; q < KQ; q++) {
+        if (q >= nq) continue;
+        if (a.xc) {
+            const int px = (gi >> 1) - c0x, py = (gj >> 1) - c0y, gk = gk0 + q, pz = (gk >> 1) - c0z;
+            if (a.mode == PROLONG_CONSTANT) {
+                const T v = aux[(pz * CW + py) * CW + px];
+                xr[0][q] += v;
+                xr[1][q] += v;
+            } else {
+                // 3/4 the parent, 1/4 its neighbour on the cell's side
+                const int qy = py + ((gj & 1) ? 1 : -1), qz = pz + ((gk & 1) ? 1 : -1);
+                T ye[2], yo[2];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const T* r0 = aux + ((h ? qz : pz) * CW + py) * CW + px;
+                    const T* r1 = aux + ((h ? qz : pz) * CW + qy) * CW + px;
+                    ye[h] = (T)0.75 * ((T)0.75 * r0[0] + (T)0.25 * r0[-1]) +
+                            (T)0.25 * ((T)0.75 * r1[0] + (T)0.25 * r1[-1]);
+                    yo[h] = (T)0.75 * ((T)0.75 * r0[0] + (T)0.25 * r0[1]) +
+                            (T)0.25 * ((T)0.75 * r1[0] + (T)0.25 * r1[1]);
+                }
+                xr[0][q] += (T)0.75 * ye[0] + (T)0.25 * ye[1];
+                xr[1][q] += (T)0.75 * yo[0] + (T)0.25 * yo[1];
+            }
+        }
+        // first, second cell -> colour 0, 1; a second cell that does not
+        // exist stays 0 (its relaxation factor is 0)
+        const T u0 = xr[0][q], u1 = two ? xr[1][q] : (T)0, d0 = a.bscale * bc[0][q], d1 = a.bscale * bc[1][q];
+        const bool sw = (p ^ (q & 1)) != 0;
+        xr[0][q] = sw ? u1 : u0;
+        xr[1][q] = sw ? u0 : u1;
+        bc[0][q] = sw ? d1 : d0;
+        bc[1][q] = sw ? d0 : d1;
+        X[q * PZ] = xr[0][q];
+        X[PC + q * PZ] = xr[1][q];
+    }
+    __syncthreads();
+    // The colour-c cell of plane q is the pair's cell e = p ^ c ^ (q & 1): its
+    // x neighbour outside the pair is the other colour's at index e ? + 1 : - 1.
+    // Xn[v]: that index for e = p ^ v.
+    const T* const Xn[2] = {X + (p ? 1 : -1), X + (p ? -1 : 1)};
+    // relaxation factor over the diagonal of cell e = p ^ v: w / 6, and with a
+    // ghost factor beta (nout neighbours outside) w / (6 - beta nout), wz in
+    // the first and last grid plane
+    const int nout_y = (gj == 0) + (gj == ny - 1);
+    T w[2], wz[2];
+#pragma unroll
+    for (int v = 0; v < 2; v++) {
+        const int e = p ^ v, i = gi + e;
+        const int no = nout_y + (i == 0) + (i == nx - 1);
+        const T om = e == 0 || two ? a.omega : (T)0;
+        w[v] = BETA ? om / ((T)6 - a.beta * (T)no) : om * (T)(1.0 / 6.0);
+        wz[v] = BETA ? om / ((T)6 - a.beta * (T)(no + 1)) : w[v];
+    }
+    const int qlo = -gk0, qhi = nz - 1 - gk0;  // plane indices of the z boundaries
+    const T om1 = (T)1 - a.omega;
+    for (int h = 0; h < 2 * a.iters; h += 2) {
+#pragma unroll
+        for (int c = 1; c >= 0; c--) {  // odd colour first
+            const T* const O = X + (1 - c) * PC;
+            // the run's end neighbours in z
+            T zlo = (T)0, zhi = (T)0;
+            if (nq > 0) {
+                zlo = O[-PZ];
+                zhi = O[nq * PZ];
+            }
+#pragma unroll
+            for (int q = 0; q < KQ; q++) {
+                if (q >= nq) continue;
+                const int v = c ^ (q & 1);
+                const T zm = q == 0 ? zlo : xr[1 - c][q > 0 ? q - 1 : 0];
+                const T zp = q == nq - 1 ? zhi : (q + 1 < KQ ? xr[1 - c][q + 1 < KQ ? q + 1 : q] : zhi);
+                T r = xr[1 - c][q] + Xn[v][(1 - c) * PC + q * PZ];
+                r += O[q * PZ + PX] + O[q * PZ - PX];
+                r += zm + zp;
+                r -= bc[c][q];
+                const T wq = BETA && (q == qlo || q == qhi) ? wz[v] : w[v];
+                xr[c][q] = om1 * xr[c][q] + wq * r;
+                X[c * PC + q * PZ] = xr[c][q];
+            }
+            __syncthreads();
+        }
+    }
+    T* x = a.x + (size_t)comp * a.G;
+    const bool own = nq > 0 && gi >= t0x && gi < t0x + TI && gj >= t0y && gj < t0y + TI;
+    const bool res = a.bn && two && (gi >> 1) < a.cx;
+#pragma unroll
+    for (int q = 0; q < KQ; q++) {
+        const int gk = gk0 + q;
+        if (!own || q >= nq || gk < t0z || gk >= t0z + TI) continue;
+        const bool sw = (p ^ (q & 1)) != 0;
+        const size_t t = ((size_t)gk * ny + gj) * nx + gi;
+        x[t] = sw ? xr[1][q] : xr[0][q];
+        if (two) x[t + 1] = sw ? xr[0][q] : xr[1][q];
+        if (!res) continue;
+        // residual of the pair, summed
+        T part = (T)0;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const T* const O = X + (1 - c) * PC;
+            const int v = c ^ (q & 1);
+            T r = xr[1 - c][q] + Xn[v][(1 - c) * PC + q * PZ];
+            r += O[q * PZ + PX] + O[q * PZ - PX];
+            r += O[q * PZ - PZ] + O[q * PZ + PZ];
+            r -= (T)6 * xr[c][q];
+            if (BETA) {
+                const int i = gi + (p ^ v);
+                const int no = nout_y + (i == 0) + (i == nx - 1) + (gk == 0) + (gk == nz - 1);
+                r += a.beta * (T)no * xr[c][q];
+            }
+            part += bc[c][q] - r;
+        }
+        aux[((gk - t0z) * TI + (gj - t0y)) * RW + ((gi - t0x) >> 1)] = part;
+    }
+    if (a.bn) {
+        __syncthreads();
+        T* bn = a.bn + (size_t)comp * a.Gc;
+        for (int q = tid; q < RW * RW * RW; q += NT) {
+            const int I = q % RW, J = (q / RW) % RW, K = q / (RW * RW);
+            const int ci = (t0x >> 1) + I, cj = (t0y >> 1) + J, ck = (t0z >> 1) + K;
+            if (ci >= a.cx || cj >= a.cy || ck >= a.cz) continue;
+            const T* r = aux + ((2 * K) * TI + 2 * J) * RW + I;
+            bn[((size_t)ck * a.cy + cj) * a.cx + ci] =
+                ((r[0] + r[RW]) + (r[TI * RW] + r[TI * RW + RW])) * (T)0.5;
+        }
+    }
+}
+
 // Exact solve of the <= 512-cell coarsest level in the separable eigenbasis,
 // FP64: v holds bscale b on entry (t < n = nx ny nz; every thread of the
 // workgroup calls it, as it synchronises), thread t < n gets x at cell t.
-__device__ inline double coarse_solve(double* v, double* w, const double* __restrict__ tab, int nx, int ny, int nz,
-                                      int t) {
+// N > 0: nx = ny = nz = N, the loops unrolled; N = 0: any dimensions.
+template <int N>
+__device__ inline double coarse_solve_n(double* v, double* w, const double* tab, int nx_, int ny_, int nz_, int t) {
+    const int nx = N ? N : nx_, ny = N ? N : ny_, nz = N ? N : nz_;
     const int n = nx * ny * nz;
     const double* Ex = tab;
     const double* Ey = Ex + nx * nx;
@@ -792,43 +1064,52 @@ __device__ inline double coarse_solve(double* v, double* w, const double* __rest
     const double* ly = lx + nx;
     const double* lz = ly + ny;
     const int i = t % nx, j = (t / nx) % ny, k = t / (nx * ny);
+    auto dot = [](int n_, auto term) {
+        double s = 0;
+        if (N) {
+#pragma unroll
+            for (int q = 0; q < N; q++) s += term(q);
+        } else {
+            for (int q = 0; q < n_; q++) s += term(q);
+        }
+        return s;
+    };
     __syncthreads();
     // forward: v <- E v along x, y, z
-    if (t < n) {
-        double s = 0;
-        for (int q = 0; q < nx; q++) s += Ex[i * nx + q] * v[(k * ny + j) * nx + q];
-        w[t] = s;
-    }
+    if (t < n) w[t] = dot(nx, [&](int q) { return Ex[i * nx + q] * v[(k * ny + j) * nx + q]; });
     __syncthreads();
-    if (t < n) {
-        double s = 0;
-        for (int q = 0; q < ny; q++) s += Ey[j * ny + q] * w[(k * ny + q) * nx + i];
-        v[t] = s;
-    }
+    if (t < n) v[t] = dot(ny, [&](int q) { return Ey[j * ny + q] * w[(k * ny + q) * nx + i]; });
     __syncthreads();
-    if (t < n) {
-        double s = 0;
-        for (int q = 0; q < nz; q++) s += Ez[k * nz + q] * v[(q * ny + j) * nx + i];
-        w[t] = s / (lx[i] + ly[j] + lz[k]);
-    }
+    if (t < n)
+        w[t] = dot(nz, [&](int q) { return Ez[k * nz + q] * v[(q * ny + j) * nx + i]; }) / (lx[i] + ly[j] + lz[k]);
     __syncthreads();
     // backward: v <- E^T v along x, y, z
-    if (t < n) {
-        double s = 0;
-        for (int q = 0; q < nx; q++) s += Ex[q * nx + i] * w[(k * ny + j) * nx + q];
-        v[t] = s;
-    }
+    if (t < n) v[t] = dot(nx, [&](int q) { return Ex[q * nx + i] * w[(k * ny + j) * nx + q]; });
     __syncthreads();
-    if (t < n) {
-        double s = 0;
-        for (int q = 0; q < ny; q++) s += Ey[q * ny + j] * v[(k * ny + q) * nx + i];
-        w[t] = s;
-    }
+    if (t < n) w[t] = dot(ny, [&](int q) { return Ey[q * ny + j] * v[(k * ny + q) * nx + i]; });
     __syncthreads();
     double s = 0;
-    if (t < n)
-        for (int q = 0; q < nz; q++) s += Ez[q * nz + k] * w[(q * ny + j) * nx + i];
+    if (t < n) s = dot(nz, [&](int q) { return Ez[q * nz + k] * w[(q * ny + j) * nx + i]; });
     return s;
+}
+
+// The eigenbasis tables of levels whose edges add up to little (8^3: 216
+// numbers) are first copied to LDS: the six products of a solve read them one
+// after another, at L2's latency (k_vtail 18 -> 15 us with the level in LDS by colours).
+constexpr int kCoarseTab = 1024;
+__device__ inline int coarse_tab_size(int nx, int ny, int nz) { return nx * nx + ny * ny + nz * nz + nx + ny + nz; }
+// ltab: kCoarseTab doubles of LDS, filled here (before coarse_solve, which
+// synchronises)
+__device__ inline void coarse_stage(double* ltab, const double* __restrict__ tab, int nx, int ny, int nz) {
+    const int n = coarse_tab_size(nx, ny, nz);
+    if (n <= kCoarseTab)
+        for (int q = threadIdx.x; q < n; q += blockDim.x) ltab[q] = tab[q];
+}
+__device__ inline double coarse_solve(double* v, double* w, const double* ltab, const double* __restrict__ tab, int nx,
+                                      int ny, int nz, int t) {
+    if (nx == 8 && ny == 8 && nz == 8) return coarse_solve_n<8>(v, w, ltab, nx, ny, nz, t);
+    if (coarse_tab_size(nx, ny, nz) <= kCoarseTab) return coarse_solve_n<0>(v, w, ltab, nx, ny, nz, t);
+    return coarse_solve_n<0>(v, w, tab, nx, ny, nz, t);
 }
 
 // Exact solve of the coarsest level, one workgroup per component.
@@ -837,136 +1118,202 @@ __global__ void __launch_bounds__(512) k_coarse(T* __restrict__ x, const T* __re
                                                 int nz, size_t G, const double* __restrict__ tab) {
     __shared__ double v[512];
     __shared__ double w[512];
+    __shared__ double ltab[kCoarseTab];
     const int comp = blockIdx.x;
     const int n = nx * ny * nz;
     const int t = threadIdx.x;
+    coarse_stage(ltab, tab, nx, ny, nz);
     if (t < n) v[t] = (double)bscale * (double)b[(size_t)comp * G + t];
-    const double s = coarse_solve(v, w, tab, nx, ny, nz, t);
+    const double s = coarse_solve(v, w, ltab, tab, nx, ny, nz, t);
     if (t < n) x[(size_t)comp * G + t] = (T)s;
 }
 
-// The two smallest levels of a fused V-cycle in one launch: level l0 (at
-// most 4096 cells, 16^3) and the coarsest below it, one component per
-// workgroup, the iterates in LDS and level l0's right-hand side in registers
-// (it comes from the restriction above), the same operations in the same
-// order as the launches they replace: zero x, nu1 red-black iterations,
-// residual and restriction, the exact coarsest solve, trilinear
-// prolongation, nu2 iterations, and X of level l0 written for the level
-// above.  A barrier separates the phases (a half-sweep reads only the other
-// colour, so its cells update in any order).  Larger levels stay on the
-// per-launch kernels: one compute unit per component sweeps 32^3 in about
-// 115 us, against about 50 us as launches over the whole device.
+// The two smallest levels of a V-cycle in one launch: level l0 (at most 4096
+// cells, 16^3) and the coarsest below it, one component per workgroup, the
+// iterate in LDS, the same operations in the same order as the launches they
+// replace: the starting x, nu1 red-black iterations, residual and restriction,
+// the exact coarsest solve, prolongation, nu2 iterations, and x of level l0
+// written for the level above.  A barrier separates the phases (a half-sweep
+// reads only the other colour, so its cells update in any order).  Larger
+// levels stay on launches over the whole device: one compute unit per
+// component sweeps 32^3 in about 115 us.  LDS issue bounds it (eight accesses
+// an update); x by colours with ghosts and the relaxation factors formed once
+// took the four half-sweeps from 8.9 to 6.1 thousand cycles, the residuals
+// through LDS the restriction from 5.8 to 4.1.
 constexpr int kTailMax = 4096;
 constexpr int kTailThreads = 1024;
 // cell pairs (2 i2, 2 i2 + 1) per thread on level l0
 constexpr int kTailPairs = 4;
+template <typename T>
 struct TailArgs {
-    float* x0;            // level l0 iterate out [ncomp][G0]
-    const float* b0;      // level l0 right-hand side [ncomp][G0]
-    float* b1;            // coarsest right-hand side [ncomp][G1] (written)
+    const T* xin;         // level l0 iterate before (null: zero)
+    T* x0;                // level l0 iterate out [ncomp][G0]
+    const T* b0;          // level l0 right-hand side [ncomp][G0]
+    T* b1;                // coarsest right-hand side [ncomp][G1] (written)
+    T bscale;             // times b0
     int d0[3], d1[3];     // dims of level l0 and of the coarsest
     size_t G0, G1;
-    float beta0, beta1;   // ghost factors of the two levels
+    T beta0, beta1;       // ghost factors of the two levels
+    int mode;             // prolongation
     int nu1, nu2;
-    float omega;
-    const double* tab;    // coarsest eigenbasis (consistent ghosts)
+    T omega;
+    const double* tab;    // coarsest eigenbasis
 };
 
-// Threads to cells on level l0: thread t owns the cell pairs (2 i2, 2 i2 + 1)
-// of column (i2, j) = t mod P (P = ceil(nx / 2) ny columns) at planes
-// k0 + R m (R = threads / P, k0 = t / P), so no loop divides.
-struct TailMap {
-    int nx, ny, nz, R, i2, j, k0;
-    bool act;
-    __device__ TailMap(const int* d) : nx(d[0]), ny(d[1]), nz(d[2]) {
-        const int hx = (nx + 1) / 2, P = hx * ny;
-        R = kTailThreads / P;
-        const int t = threadIdx.x;
-        act = t < R * P;
-        const int c = t % P;
-        i2 = c % hx;
-        j = c / hx;
-        k0 = t / P;
-    }
-};
-// the fit test of level l0 (host side)
+// Level l0 in LDS by colours, as a tile of k_tile with the whole level as its
+// region: pair (m, y) of plane z at index ((z + 1) (ny + 2) + y + 1) (hx + 1) +
+// m + 1 of each colour, hx = ceil(nx / 2), zeros around.
+constexpr int kTailLds = 4096;
+inline int tail_pairs(const int* d) { return ((d[0] + 1) / 2 + 1) * (d[1] + 2) * (d[2] + 2) + 1; }
+// the fit test of level l0 (host side): thread t owns column (m, y) = t mod P
+// (P = hx ny columns) at kq = ceil(nz / (threads / P)) planes
 inline bool tail_fits(const int* d) {
     const int P = ((d[0] + 1) / 2) * d[1];
-    if (P > kTailThreads) return false;
+    if (P > kTailThreads || tail_pairs(d) > kTailLds) return false;
     const int R = kTailThreads / P;
     return (d[2] + R - 1) / R <= kTailPairs;
 }
 
-// be / bo: the right-hand sides of the thread's even and odd cells (two
-// arrays with constant indices, so they stay in registers)
-__device__ inline void tail_smooth(float* x, const float (&be)[kTailPairs], const float (&bo)[kTailPairs],
-                                   const TailMap& m, float omega, float beta, int iters) {
-    for (int it = 0; it < iters; it++)
-        for (int color = 1; color >= 0; color--) {
-#pragma unroll
-            for (int q = 0; q < kTailPairs; q++) {
-                const int k = m.k0 + m.R * q;
-                if (m.act && k < m.nz) {
-                    const int e = (m.j + k + color) & 1, i = 2 * m.i2 + e;
-                    if (i < m.nx) rbgs_point(x, e ? bo[q] : be[q], 1.0f, i, m.j, k, m.nx, m.ny, m.nz, omega, beta);
-                }
-            }
-            __syncthreads();
-        }
-}
-
-__global__ void __launch_bounds__(kTailThreads) k_vtail(TailArgs a) {
-    __shared__ float xa[kTailMax];
-    __shared__ float xc[512];
-    __shared__ double cv[512], cw[512];
-    const int comp = blockIdx.x;
-    const int n0 = a.d0[0] * a.d0[1] * a.d0[2], n1 = a.d1[0] * a.d1[1] * a.d1[2];
-    const float* b0 = a.b0 + (size_t)comp * a.G0;
-    float* b1 = a.b1 + (size_t)comp * a.G1;
-    const TailMap m(a.d0);
-    // the thread's right-hand sides into registers; x = 0
-    float be[kTailPairs], bo[kTailPairs];
+template <typename T>
+__global__ void __launch_bounds__(kTailThreads) k_vtail(TailArgs<T> a) {
+    __shared__ T xa[2][kTailLds];
+    __shared__ T rs[kTailMax];  // residuals of level l0, in grid order
+    __shared__ T xc[512];
+    __shared__ double cv[512], cw[512], ltab[kCoarseTab];
+    const int comp = blockIdx.x, tid = threadIdx.x;
+    const int nx = a.d0[0], ny = a.d0[1], nz = a.d0[2];
+    const int cx = a.d1[0], cy = a.d1[1], cz = a.d1[2];
+    const int n1 = cx * cy * cz;
+    const T* b0 = a.b0 + (size_t)comp * a.G0;
+    const T* xi = a.xin ? a.xin + (size_t)comp * a.G0 : nullptr;
+    T* b1 = a.b1 + (size_t)comp * a.G1;
+    // thread -> pair column (m, j), planes k0 .. k0 + nq - 1
+    const int hx = (nx + 1) >> 1, P = hx * ny, R = kTailThreads / P;
+    const int kq = (nz + R - 1) / R;
+    const int col = tid % P, grp = tid / P;
+    const int m = col % hx, j = col / hx, i = 2 * m, k0 = grp * kq;
+    const int nq = grp < R ? min(kq, nz - k0) : 0;  // <= 0: no planes
+    const bool two = i + 1 < nx;
+    const int p = (j + k0) & 1;  // colour of the first cell in plane k0
+    const int PX = hx + 1, PZ = PX * (ny + 2);
+    // the thread's right-hand sides and starting x into registers, by cell
+    // (first, second); planes past nq read the first cells
+    T be[kTailPairs], bo[kTailPairs], xe[kTailPairs], xo[kTailPairs];
 #pragma unroll
     for (int q = 0; q < kTailPairs; q++) {
-        const int k = m.k0 + m.R * q, i = 2 * m.i2;
-        be[q] = bo[q] = 0.f;
-        if (m.act && k < m.nz) {
-            const size_t t = ((size_t)k * m.ny + m.j) * m.nx + i;
-            be[q] = b0[t];
-            if (i + 1 < m.nx) bo[q] = b0[t + 1];
-        }
+        const size_t t = q < nq ? ((size_t)(k0 + q) * ny + j) * nx + i : 0;
+        const size_t t1 = t + (q < nq && two ? 1 : 0);
+        be[q] = b0[t];
+        bo[q] = b0[t1];
+        xe[q] = xi ? xi[t] : (T)0;
+        xo[q] = xi ? xi[t1] : (T)0;
     }
-    for (int q = threadIdx.x; q < n0; q += blockDim.x) xa[q] = 0.f;
+    coarse_stage(ltab, a.tab, cx, cy, cz);
+    const int nl = PZ * (nz + 2) + 1;
+    for (int q = tid; q < nl; q += kTailThreads) xa[0][q] = xa[1][q] = (T)0;
     __syncthreads();
-    tail_smooth(xa, be, bo, m, a.omega, a.beta0, a.nu1);
-    // residual and restriction into the coarsest right-hand side (rounded to
-    // float as the global store of the per-launch path), then its exact solve
-    for (int q = threadIdx.x; q < n1; q += blockDim.x) {
-        const int ci = q % a.d1[0], cj = (q / a.d1[0]) % a.d1[1], ck = q / (a.d1[0] * a.d1[1]);
-        const float r = restrict_point(xa, b0, 1.0f, ci, cj, ck, a.d0[0], a.d0[1], a.d0[2], a.beta0);
+    const int o0 = nq > 0 ? (k0 + 1) * PZ + (j + 1) * PX + m + 1 : 0;
+#pragma unroll
+    for (int q = 0; q < kTailPairs; q++)
+        if (q < nq) {
+            const int s = p ^ (q & 1), o = o0 + q * PZ;
+            xa[s][o] = xe[q];
+            if (two) xa[1 - s][o] = xo[q];
+        }
+    __syncthreads();
+    // sum of the neighbours of cell e of the pair at o (colour c), added as
+    // nb_sum does
+    auto nbr = [&](int c, int o, int e) {
+        const T* O = xa[1 - c];
+        T r = O[o - 1 + e] + O[o + e];
+        r += O[o + PX] + O[o - PX];
+        r += O[o - PZ] + O[o + PZ];
+        return r;
+    };
+    const int nout_y = (j == 0) + (j == ny - 1);
+    auto outside = [&](int e, int k) {
+        return (i + e == 0) + (i + e == nx - 1) + nout_y + (k == 0) + (k == nz - 1);
+    };
+    T we[kTailPairs], wo[kTailPairs];
+#pragma unroll
+    for (int q = 0; q < kTailPairs; q++) {
+        we[q] = rbgs_weight(outside(0, k0 + q), a.omega, a.beta0);
+        wo[q] = rbgs_weight(outside(1, k0 + q), a.omega, a.beta0);
+    }
+    auto smooth = [&](int iters) {
+        for (int h = 0; h < iters; h++)
+#pragma unroll
+            for (int c = 1; c >= 0; c--) {  // odd colour first
+#pragma unroll
+                for (int q = 0; q < kTailPairs; q++) {
+                    const int e = p ^ c ^ (q & 1), o = o0 + q * PZ;
+                    if (q < nq && (e == 0 || two))
+                        xa[c][o] = rbgs_value(xa[c][o], nbr(c, o, e), e ? bo[q] : be[q], a.bscale,
+                                              e ? wo[q] : we[q], a.omega);
+                }
+                __syncthreads();
+            }
+    };
+    smooth(a.nu1);
+    // residuals (residual_at), then their sums over the children of each
+    // coarse cell in restrict_point's order: the coarsest right-hand side
+#pragma unroll
+    for (int q = 0; q < kTailPairs; q++)
+        if (q < nq) {
+            const int o = o0 + q * PZ, t = ((k0 + q) * ny + j) * nx + i;
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int c = p ^ e ^ (q & 1);
+                if (e == 1 && !two) continue;
+                const T xv = xa[c][o];
+                T r = nbr(c, o, e);
+                r -= (T)6 * xv;
+                const int no = outside(e, k0 + q);
+                if (a.beta0 != (T)0 && no) r += a.beta0 * (T)no * xv;
+                rs[t + e] = a.bscale * (e ? bo[q] : be[q]) - r;
+            }
+        }
+    __syncthreads();
+    for (int q = tid; q < n1; q += kTailThreads) {
+        const int ci = q % cx, cj = (q / cx) % cy, ck = q / (cx * cy);
+        const bool hi = 2 * ci + 1 < nx, hj = 2 * cj + 1 < ny, hk = 2 * ck + 1 < nz;
+        const T* f = rs + ((2 * ck) * ny + 2 * cj) * nx + 2 * ci;
+        T r = 0;
+        r += f[0];
+        if (hi) r += f[1];
+        if (hj) r += f[nx];
+        if (hi && hj) r += f[nx + 1];
+        if (hk) r += f[nx * ny];
+        if (hi && hk) r += f[nx * ny + 1];
+        if (hj && hk) r += f[nx * ny + nx];
+        if (hi && hj && hk) r += f[nx * ny + nx + 1];
+        r *= (T)0.5;
         b1[q] = r;
         cv[q] = (double)1.0f * (double)r;
     }
-    const double s = coarse_solve(cv, cw, a.tab, a.d1[0], a.d1[1], a.d1[2], threadIdx.x);
-    if ((int)threadIdx.x < n1) xc[threadIdx.x] = (float)s;
+    const double s = coarse_solve(cv, cw, ltab, a.tab, cx, cy, cz, tid);
+    if (tid < n1) xc[tid] = (T)s;
     __syncthreads();
     // prolongation of the coarse correction, then nu2 iterations
 #pragma unroll
-    for (int q = 0; q < kTailPairs; q++) {
-        const int k = m.k0 + m.R * q;
-        if (m.act && k < m.nz)
-            for (int e = 0; e < 2; e++) {
-                const int i = 2 * m.i2 + e;
-                if (i < m.nx)
-                    xa[((size_t)k * m.ny + m.j) * m.nx + i] +=
-                        prolong_point((const float*)xc, i, m.j, k, m.nx, m.ny, m.nz, a.d1[0], a.d1[1], a.d1[2],
-                                      (int)PROLONG_TRILINEAR, a.beta1);
-            }
-    }
+    for (int q = 0; q < kTailPairs; q++)
+        if (q < nq) {
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                if (e == 0 || two)
+                    xa[p ^ e ^ (q & 1)][o0 + q * PZ] +=
+                        prolong_point((const T*)xc, i + e, j, k0 + q, nx, ny, nz, cx, cy, cz, a.mode, a.beta1);
+        }
     __syncthreads();
-    tail_smooth(xa, be, bo, m, a.omega, a.beta0, a.nu2);
-    float* xo = a.x0 + (size_t)comp * a.G0;
-    for (int q = threadIdx.x; q < n0; q += blockDim.x) xo[q] = xa[q];
+    smooth(a.nu2);
+    T* x = a.x0 + (size_t)comp * a.G0;
+#pragma unroll
+    for (int q = 0; q < kTailPairs; q++)
+        if (q < nq) {
+            const int sc = p ^ (q & 1), o = o0 + q * PZ, t = ((k0 + q) * ny + j) * nx + i;
+            x[t] = xa[sc][o];
+            if (two) x[t + 1] = xa[1 - sc][o];
+        }
 }
 
 template <typename T>
@@ -1221,7 +1568,7 @@ template <typename T>
 size_t MGHier<T>::bytes_for(int nx, int ny, int nz, int ncomp) {
     size_t b = 0, cells = (size_t)nx * ny * nz;
     int x = nx, y = ny, z = nz, L = 1;
-    if (std::is_same<T, float>::value) b += cells * ncomp * sizeof(T);
+    if (has_temp(cells)) b += cells * ncomp * sizeof(T);
     while ((long)x * y * z > 512 && L < 16) {
         x = x / 2 > 0 ? x / 2 : 1;
         y = y / 2 > 0 ? y / 2 : 1;
@@ -1229,7 +1576,7 @@ size_t MGHier<T>::bytes_for(int nx, int ny, int nz, int ncomp) {
         L++;
         cells = (size_t)x * y * z;
         b += 2 * cells * ncomp * sizeof(T);
-        if (std::is_same<T, float>::value) b += cells * ncomp * sizeof(T);
+        if (has_temp(cells)) b += cells * ncomp * sizeof(T);
     }
     // coarse tables (two bases, <= 3 * 512^2 doubles each at most) and norm partials
     b += 2 * (size_t)(x * x + y * y + z * z + x + y + z) * sizeof(double);
@@ -1266,10 +1613,11 @@ pppm_status MGHier<T>::init(int nx, int ny, int nz, int ncomp) {
     b_.assign(L_, nullptr);
     t_.assign(L_, nullptr);
     bytes_ = 0;
-    if (std::is_same<T, float>::value) {
-        rbc_prime();
-        // out-of-place targets of the blocked smoother, every level
+    {
+        if (std::is_same<T, float>::value) rbc_prime();
+        // out-of-place targets of the blocked passes
         for (int l = 0; l < L_; l++) {
+            if (!has_temp(cells(l))) continue;
             size_t n = cells(l) * ncomp_;
             if (hipMalloc(&t_[l], n * sizeof(T)) != hipSuccess) {
                 release_locked();
@@ -1571,7 +1919,7 @@ pppm_status MGHier<T>::coarse(T* x, const T* b, T bscale, bool consistent, hipSt
 
 template <typename T>
 int MGHier<T>::tail_level() const {
-    if (!std::is_same<T, float>::value || !tail_ || L_ < 3) return -1;
+    if (!tb_ || !tail_ || L_ < 3) return -1;
     // the level above the coarsest, below the blocked levels
     const int l0 = L_ - 2;
     if (cells(l0) >= tb_min_cells_ || cells(l0) > (size_t)kTailMax || cells(L_ - 1) > 512 || !tail_fits(d_[l0]))
@@ -1580,56 +1928,176 @@ int MGHier<T>::tail_level() const {
 }
 
 template <typename T>
-pppm_status MGHier<T>::tail(int, int, int, T, hipStream_t) {
-    return PPPM_ERR_INVALID;
-}
-template <>
-pppm_status MGHier<float>::tail(int l0, int nu1, int nu2, float omega, hipStream_t st) {
-    TailArgs a{};
-    a.x0 = x_[l0];
-    a.b0 = b_[l0];
-    a.b1 = b_[l0 + 1];
+pppm_status MGHier<T>::tail(const T* xin, T* x, const T* b, T* b1, T bscale, int nu1, int nu2, T omega,
+                            bool consistent, hipStream_t st) {
+    const int l0 = L_ - 2;
+    TailArgs<T> a{};
+    a.xin = xin;
+    a.x0 = x;
+    a.b0 = b;
+    a.b1 = b1;
+    a.bscale = bscale;
     for (int c = 0; c < 3; c++) {
         a.d0[c] = d_[l0][c];
         a.d1[c] = d_[l0 + 1][c];
     }
     a.G0 = cells(l0);
     a.G1 = cells(l0 + 1);
-    a.beta0 = (float)mg_beta(l0);
-    a.beta1 = (float)mg_beta(l0 + 1);
+    a.beta0 = consistent ? (T)mg_beta(l0) : (T)0;
+    a.beta1 = consistent ? (T)mg_beta(l0 + 1) : (T)0;
+    a.mode = consistent ? PROLONG_TRILINEAR : PROLONG_CONSTANT;
     a.nu1 = nu1;
     a.nu2 = nu2;
     a.omega = omega;
-    a.tab = tab_cons_;
-    hipLaunchKernelGGL(k_vtail, dim3(ncomp_), dim3(kTailThreads), 0, st, a);
+    a.tab = consistent ? tab_cons_ : tab_ref_;
+    hipLaunchKernelGGL(k_vtail<T>, dim3(ncomp_), dim3(kTailThreads), 0, st, a);
     PPPM_LAUNCH_CHECK();
     return PPPM_OK;
 }
 
-// MultiGrid.cpp:128-201 (m_Vcycle)
+template <typename T>
+bool MGHier<T>::tile_level(int l, bool consistent) const {
+    if (!tb_ || l >= L_ - 1 || !has_temp(cells(l)) || cells(l) >= std::min(tb_min_cells_, kTileCells)) return false;
+    for (int c = 0; c < 3; c++)
+        // without the one launch of the smallest levels the one above the
+        // coarsest runs a launch per half-sweep, with bitwise its results
+        if (d_[l][c] < 2 || (!tail_ && l == L_ - 2) || (consistent && (d_[l][c] & 1))) return false;  // trilinear parents are i / 2
+    return true;
+}
+
+template <typename T>
+pppm_status MGHier<T>::tile(int l, const T* xin, T* x, const T* b, T bscale, int iters, T omega, T beta, T* bnext,
+                            const T* xc, int mode, T betac, hipStream_t st) {
+    if (iters < 1 || iters > 2 || (bnext && xc) || xin == x) return PPPM_ERR_INVALID;
+    const int* d = d_[l];
+    const int* c = d_[l + 1];
+    TileArgs<T> a{};
+    a.xin = xin;
+    a.x = x;
+    a.b = b;
+    a.bscale = bscale;
+    a.nx = d[0];
+    a.ny = d[1];
+    a.nz = d[2];
+    a.G = cells(l);
+    a.omega = omega;
+    a.beta = beta;
+    a.iters = iters;
+    a.bn = bnext;
+    a.cx = c[0];
+    a.cy = c[1];
+    a.cz = c[2];
+    a.Gc = cells(l + 1);
+    a.xc = xc;
+    a.betac = betac;
+    a.mode = mode;
+    // 16^3 tiles recompute less halo (26^3 cells against 18^3 for an eighth
+    // of the tile) where they still fill the chip; doubles of them do not fit
+    // LDS with a second workgroup
+    const bool big = std::is_same<T, float>::value && cells(l) * (size_t)ncomp_ >= kTile16Cells;
+    const int TI = big ? 16 : 8;
+    a.tx = (d[0] + TI - 1) / TI;
+    a.ty = (d[1] + TI - 1) / TI;
+    a.tz = (d[2] + TI - 1) / TI;
+    dim3 grid(a.tx * a.ty * a.tz, ncomp_);
+    if constexpr (std::is_same<T, float>::value) {
+        if (big) {
+            if (beta != 0.f) hipLaunchKernelGGL((k_tile<float, 16, true>), grid, dim3(tile_threads(16)), 0, st, a);
+            else hipLaunchKernelGGL((k_tile<float, 16, false>), grid, dim3(tile_threads(16)), 0, st, a);
+            PPPM_LAUNCH_CHECK();
+            return PPPM_OK;
+        }
+    }
+    if (beta != (T)0) hipLaunchKernelGGL((k_tile<T, 8, true>), grid, dim3(tile_threads(8)), 0, st, a);
+    else hipLaunchKernelGGL((k_tile<T, 8, false>), grid, dim3(tile_threads(8)), 0, st, a);
+    PPPM_LAUNCH_CHECK();
+    return PPPM_OK;
+}
+
+// A tile level of a V-cycle on the way down: nu1 iterations, two a launch,
+// from src (null: zero; else X[l] itself), the last launch with the residual
+// and its restriction; fold (with more than two iterations): coarse iterate
+// whose prolongation is added first.  The launches alternate between X and the
+// level's temporary so that the nu2 iterations on the way up end in X (a start
+// from X itself and an odd number of launches ends in the temporary, copied
+// by tile_up).
+template <typename T>
+static pppm_status tile_down(MGHier<T>& m, int l, T* X, const T* src, const T* b, T bs, int nu1, int nu2, T omega,
+                             T beta, T* bnext, const T* fold, int mode, T betac, T** cur, hipStream_t st) {
+    const int np1 = (nu1 + 1) / 2, total = np1 + (nu2 + 1) / 2;
+    T* dst = (!src && (total & 1)) ? X : m.temp(l);
+    for (int q = 0; q < np1; q++) {
+        const bool last = q == np1 - 1;
+        pppm_status s = m.tile(l, src, dst, b, bs, last ? nu1 - 2 * q : 2, omega, beta, last ? bnext : nullptr,
+                               q == 0 ? fold : nullptr, mode, betac, st);
+        if (s != PPPM_OK) return s;
+        src = dst;
+        dst = dst == X ? m.temp(l) : X;
+    }
+    *cur = const_cast<T*>(src);
+    return PPPM_OK;
+}
+// ... and on the way up: the prolongation of xc, then nu2 iterations, into X.
+template <typename T>
+static pppm_status tile_up(MGHier<T>& m, int l, T* X, T* cur, const T* b, T bs, int nu2, T omega, T beta, const T* xc,
+                           int mode, T betac, hipStream_t st) {
+    for (int done = 0; done < nu2; done += 2) {
+        T* dst = cur == X ? m.temp(l) : X;
+        pppm_status s = m.tile(l, cur, dst, b, bs, std::min(2, nu2 - done), omega, beta, nullptr,
+                               done == 0 ? xc : nullptr, mode, betac, st);
+        if (s != PPPM_OK) return s;
+        cur = dst;
+    }
+    return cur == X ? PPPM_OK : m.copy(X, cur, m.cells(l) * m.ncomp(), st);
+}
+
+// MultiGrid.cpp:128-201 (m_Vcycle) from level l0 on X[l0]; fold: level l0 + 1
+// iterate whose (constant) prolongation is added to X[l0] first.
 template <typename T>
 static pppm_status vcycle_from(MGHier<T>& m, std::vector<T*>& X, std::vector<T*>& B, int l0, T bscale0, int nu1,
-                               int nu2, T omega, bool consistent, hipStream_t st) {
-    const int L = m.levels();
+                               int nu2, T omega, bool consistent, hipStream_t st, const T* fold = nullptr) {
+    const int L = m.levels(), mode = consistent ? PROLONG_TRILINEAR : PROLONG_CONSTANT;
+    const bool relax = nu1 > 0 && nu2 > 0;
+    const int lt = m.tail_level();
+    const bool tail = lt >= l0 && lt >= 0;
+    const int lend = tail ? lt : L - 1;
+    std::vector<T*> cur(L, nullptr);
     pppm_status s;
-    for (int l = l0; l < L - 1; l++) {
-        T beta = consistent ? (T)mg_beta(l) : (T)0;
-        T bs = l == 0 ? bscale0 : (T)1;
+    auto beta_of = [&](int l) { return consistent ? (T)mg_beta(l) : (T)0; };
+    if (fold && !(l0 < lend && relax && nu1 > 2 && m.tile_level(l0, consistent))) {
+        if ((s = m.prolong(l0, X[l0], fold, mode, beta_of(l0 + 1), st)) != PPPM_OK) return s;
+        fold = nullptr;
+    }
+    for (int l = l0; l < lend; l++) {
+        const T beta = beta_of(l), bs = l == 0 ? bscale0 : (T)1;
+        if (relax && m.tile_level(l, consistent)) {
+            if ((s = tile_down(m, l, X[l], l > l0 ? (const T*)nullptr : (const T*)X[l], (const T*)B[l], bs, nu1, nu2,
+                               omega, beta, B[l + 1], l == l0 ? fold : (const T*)nullptr, mode, beta_of(l + 1), &cur[l],
+                               st)) != PPPM_OK)
+                return s;
+            continue;
+        }
         if (l > l0 && (s = m.fill(X[l], m.cells(l) * m.ncomp(), st)) != PPPM_OK) return s;
         if ((s = m.smooth(l, X[l], B[l], bs, nu1, omega, beta, st)) != PPPM_OK) return s;
         if ((s = m.residual_restrict(l, X[l], B[l], bs, beta, B[l + 1], st)) != PPPM_OK) return s;
     }
-    {
+    if (tail) {
+        if ((s = m.tail(lt > l0 ? (const T*)nullptr : (const T*)X[lt], X[lt], B[lt], B[lt + 1],
+                        lt == 0 ? bscale0 : (T)1, nu1, nu2, omega, consistent, st)) != PPPM_OK)
+            return s;
+    } else {
         T bs = (L - 1) == 0 ? bscale0 : (T)1;
         if ((s = m.coarse(X[L - 1], B[L - 1], bs, consistent, st)) != PPPM_OK) return s;
     }
-    for (int l = L - 2; l >= l0; l--) {
-        T beta = consistent ? (T)mg_beta(l) : (T)0;
-        T bs = l == 0 ? bscale0 : (T)1;
-        T betac = consistent ? (T)mg_beta(l + 1) : (T)0;
-        if ((s = m.prolong(l, X[l], X[l + 1], consistent ? PROLONG_TRILINEAR : PROLONG_CONSTANT, betac, st)) !=
-            PPPM_OK)
-            return s;
+    for (int l = lend - 1; l >= l0; l--) {
+        const T beta = beta_of(l), betac = beta_of(l + 1), bs = l == 0 ? bscale0 : (T)1;
+        if (cur[l]) {
+            if ((s = tile_up(m, l, X[l], cur[l], (const T*)B[l], bs, nu2, omega, beta, (const T*)X[l + 1], mode, betac,
+                             st)) != PPPM_OK)
+                return s;
+            continue;
+        }
+        if ((s = m.prolong(l, X[l], X[l + 1], mode, betac, st)) != PPPM_OK) return s;
         if ((s = m.smooth(l, X[l], B[l], bs, nu2, omega, beta, st)) != PPPM_OK) return s;
     }
     return PPPM_OK;
@@ -1668,8 +2136,9 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
         return a;
     };
     // Blocked passes pay a fixed latency per plane that small levels cannot
-    // amortise: levels below the hierarchy's threshold run the
-    // one-launch-per-colour kernels in place instead.
+    // amortise: levels below the hierarchy's threshold run the tile passes
+    // (k_tile), or with odd dimensions the one-launch-per-colour kernels in
+    // place.
     auto blocked = [&](int l) { return m.cells(l) >= m.blocked_min_cells(); };
     // the small levels in one launch where they fit (l0 >= 1: X and B of
     // those levels are the hierarchy's own)
@@ -1679,6 +2148,14 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
     // ping-ponging with the level's temporary; the last pass also restricts
     std::vector<float*> cur(L, nullptr);
     for (int l = 0; l < lend; l++) {
+        if (m.tile_level(l, true)) {
+            const bool zero = l > 0 || x0_zero;
+            if ((s = tile_down(m, l, X[l], zero ? (const float*)nullptr : (const float*)X[l], (const float*)B[l],
+                               l == 0 ? bscale0 : 1.0f, nu1, nu2, omega, (float)mg_beta(l), B[l + 1],
+                               (const float*)nullptr, (int)PROLONG_TRILINEAR, 0.f, &cur[l], st)) != PPPM_OK)
+                return s;
+            continue;
+        }
         if (!blocked(l)) {
             const float bs = l == 0 ? bscale0 : 1.0f, beta = (float)mg_beta(l);
             if ((l > 0 || x0_zero) && (s = m.fill(X[l], m.cells(l) * nc, st)) != PPPM_OK) return s;
@@ -1709,13 +2186,20 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
         cur[l] = src;
     }
     if (l0 > 0) {
-        if ((s = m.tail(l0, nu1, nu2, omega, st)) != PPPM_OK) return s;
+        if ((s = m.tail(nullptr, X[l0], B[l0], B[l0 + 1], 1.0f, nu1, nu2, omega, true, st)) != PPPM_OK) return s;
         cur[l0] = X[l0];
     } else if ((s = m.coarse(X[L - 1], B[L - 1], L == 1 ? bscale0 : 1.0f, true, st)) != PPPM_OK) {
         return s;
     }
     // up: nu2 passes per level, the first adds the prolonged correction on load
     for (int l = l0 > 0 ? l0 - 1 : L - 2; l >= 0; l--) {
+        if (m.tile_level(l, true)) {
+            if ((s = tile_up(m, l, X[l], cur[l], (const float*)B[l], l == 0 ? bscale0 : 1.0f, nu2, omega,
+                             (float)mg_beta(l), (const float*)X[l + 1], (int)PROLONG_TRILINEAR, (float)mg_beta(l + 1),
+                             st)) != PPPM_OK)
+                return s;
+            continue;
+        }
         if (!blocked(l)) {
             const float bs = l == 0 ? bscale0 : 1.0f, beta = (float)mg_beta(l);
             if ((s = m.prolong(l, X[l], X[l + 1], PROLONG_TRILINEAR, (float)mg_beta(l + 1), st)) != PPPM_OK)
@@ -1779,8 +2263,8 @@ pppm_status MGHier<T>::ref_fmg(T* x0, const T* b0, T bscale0, int nu1, int nu2, 
     }
     if ((s = coarse(X[L_ - 1], B[L_ - 1], L_ == 1 ? bscale0 : (T)1, false, st)) != PPPM_OK) return s;
     for (int l = L_ - 2; l >= 0; l--) {
-        if ((s = prolong(l, X[l], X[l + 1], PROLONG_CONSTANT, (T)0, st)) != PPPM_OK) return s;
-        if ((s = vcycle_from(*this, X, B, l, bscale0, nu1, nu2, omega, false, st)) != PPPM_OK) return s;
+        if ((s = vcycle_from(*this, X, B, l, bscale0, nu1, nu2, omega, false, st, (const T*)X[l + 1])) != PPPM_OK)
+            return s;
     }
     return vcycle_from(*this, X, B, 0, bscale0, nu1, nu2, omega, false, st);
 }

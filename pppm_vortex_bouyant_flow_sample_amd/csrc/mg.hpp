@@ -71,8 +71,12 @@ class MGHier {
     pppm_status coarse(T* x, const T* b, T bscale, bool consistent, hipStream_t st);
     pppm_status fill(T* p, size_t n, hipStream_t st);
     pppm_status copy(T* d, const T* s, size_t n, hipStream_t st);
-    // out-of-place target of the blocked smoother at level l (float only)
+    // out-of-place target of the blocked passes at level l (null where
+    // has_temp is false)
     T* temp(int l) { return t_[l]; }
+    // levels with an out-of-place target: every float level (blocked
+    // smoother, tile passes), the double ones that take the tile passes
+    static bool has_temp(size_t cells) { return sizeof(T) == 4 || cells < kTileCells; }
     double* partials() { return part_; }
     // the reduced norms, 2 per component (||r||^2, ||b||^2), after the partials
     double* norm_out() { return part_ + (size_t)kNormBlocks * ncomp_ * 2; }
@@ -91,17 +95,26 @@ class MGHier {
     void set_blocked_smoother(int kind) { tb_ = kind; }
     int blocked_smoother() const { return tb_; }
     // V-cycles run the blocked passes on levels with at least this many cells
-    // per component, one launch per colour below
+    // per component, the tile passes below
     void set_blocked_min_cells(size_t n) { tb_min_cells_ = n; }
     size_t blocked_min_cells() const { return tb_min_cells_; }
-    // float V-cycles: the level above the coarsest and the coarsest solve in
-    // one launch (k_vtail) where they fit, or one launch per half-sweep
+    // V-cycles: the level above the coarsest and the coarsest solve in one
+    // launch (k_vtail) where they fit, or apart
     void set_small_one_launch(bool on) { tail_ = on; }
     bool small_one_launch() const { return tail_; }
-    // the level l0 = L - 2 of that launch, or -1 where it does not apply
+    // the level L - 2 of that launch, or -1 where it does not apply
     int tail_level() const;
-    // the launch (levels l0 and l0 + 1) on the hierarchy's own level arrays
-    pppm_status tail(int l0, int nu1, int nu2, T omega, hipStream_t st);
+    // that launch, on that level's iterate x (xin: its start, null: zero),
+    // its right-hand side b (times bscale) and the coarsest one's b1 (written)
+    pppm_status tail(const T* xin, T* x, const T* b, T* b1, T bscale, int nu1, int nu2, T omega, bool consistent,
+                     hipStream_t st);
+    // whether level l of a V-cycle takes the tile passes (k_tile)
+    bool tile_level(int l, bool consistent) const;
+    // one tile pass, xin (null: zero) -> x: the prolongation of xc added
+    // (null: none), 1 or 2 red-black iterations, the residual restricted into
+    // bnext (null: none; not with xc)
+    pppm_status tile(int l, const T* xin, T* x, const T* b, T bscale, int iters, T omega, T beta, T* bnext,
+                     const T* xc, int mode, T betac, hipStream_t st);
 
    private:
     void release_locked();  // release() with runtime_mutex() already held
@@ -115,7 +128,11 @@ class MGHier {
     double* hnorm_ = nullptr;     // pinned host copy of the reduced norms
     size_t bytes_ = 0;
     int tb_ = 2;
-    size_t tb_min_cells_ = (size_t)1 << 18;
+    // Tile passes below kTileCells cells a component, in 16^3 tiles from
+    // kTile16Cells cells over all components.
+    static constexpr size_t kTileCells = (size_t)1 << 19;
+    static constexpr size_t kTile16Cells = (size_t)1 << 19;
+    size_t tb_min_cells_ = (size_t)1 << 19;
     bool tail_ = true;
 };
 
