@@ -125,23 +125,34 @@ PathGeom make_geom(const pppm_params& p) {
 }
 
 // dir table of the far-field correction (GPU_kernel.cu:2646-2677), FP64 on the
-// host, stored as float3 rows in ((dz+K)(2K+1)+(dy+K))(2K+1)+(dx+K) order.
+// host, stored as float3 rows in ((dz+M)(2M+1)+(dy+M))(2M+1)+(dx+M) order, M =
+// max(K, 1).  The curl of the diagonal term c h^2 w (1976-2001), central
+// differences over the face neighbours, is part of the table: +- c / (2 h^2)
+// in component a at +- e_a (the kernel scales by h^3).
 std::vector<float> far_dir_table(int K, double h) {
-    const int W = 2 * K + 1;
+    const int M = K < 1 ? 1 : K;
+    const int W = 2 * M + 1;
     std::vector<float> out((size_t)W * W * W * 3, 0.f);
     auto R = [](double ax, double ay, double az, double bx, double by, double bz) {
         double r2 = (ax - bx) * (ax - bx) + (ay - by) * (ay - by) + (az - bz) * (az - bz);
         return r2 > 1e-12 ? kRefFourPi * std::sqrt(r2) : 1e24;
     };
-    for (int kk = -K; kk <= K; kk++)
-        for (int jj = -K; jj <= K; jj++)
-            for (int ii = -K; ii <= K; ii++) {
+    const double diag = 0.5 * kRefDiagPsi / (h * h);
+    for (int kk = -M; kk <= M; kk++)
+        for (int jj = -M; jj <= M; jj++)
+            for (int ii = -M; ii <= M; ii++) {
                 if (ii == 0 && jj == 0 && kk == 0) continue;
                 double px = (ii + 0.5) * h, py = (jj + 0.5) * h, pz = (kk + 0.5) * h, X = 0.5 * h;
                 double dx = 0.5 * ((1.0 / R(X + h, X, X, px, py, pz)) - (1.0 / R(X - h, X, X, px, py, pz))) / h;
                 double dy = 0.5 * ((1.0 / R(X, X + h, X, px, py, pz)) - (1.0 / R(X, X - h, X, px, py, pz))) / h;
                 double dz = 0.5 * ((1.0 / R(X, X, X + h, px, py, pz)) - (1.0 / R(X, X, X - h, px, py, pz))) / h;
-                size_t o = 3 * (size_t)(((kk + K) * W + (jj + K)) * W + (ii + K));
+                if (K < 1) dx = dy = dz = 0;  // the diagonal term alone
+                if (std::abs(ii) + std::abs(jj) + std::abs(kk) == 1) {
+                    dx += ii * diag;
+                    dy += jj * diag;
+                    dz += kk * diag;
+                }
+                size_t o = 3 * (size_t)(((kk + M) * W + (jj + M)) * W + (ii + M));
                 out[o] = (float)dx;
                 out[o + 1] = (float)dy;
                 out[o + 2] = (float)dz;

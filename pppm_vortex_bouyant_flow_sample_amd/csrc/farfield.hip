@@ -9,32 +9,273 @@
 // grid_U and its per-call host table upload are gone: dir[] is built once per
 // (K, h) and read with wave-uniform (scalar) loads.
 #include "pppm_internal.hpp"
+#include <algorithm>
+#include <type_traits>
 
 namespace pppm {
 
-template <typename TP>
-__device__ inline double ld(const TP* p, size_t i) {
-    return (double)p[i];
+// What each plane of the grid vorticity w adds to the sum is formed once, when
+// the plane arrives, for the 2K+1 output planes it reaches (their sums sit in
+// registers while a workgroup marches along z), so LDS holds one plane and the
+// next.  dir[D] has component a odd in D_a and even in the other two (a central
+// difference along a of 1/(4 pi |r|)), so the (2K+1)^2 neighbours of a plane are
+// folded to sums and differences over +-y and +-x first and the planes at +-dz
+// share their products: 191 vector instructions a cell at K = 2 where the sum
+// over neighbour pairs took 650, and 45 8-byte LDS reads for two cells where it
+// took 372 4-byte ones a cell.  The curl of the diagonal term, differences over
+// the six face neighbours, is part of the same sum: dir[+-e_a]_a carries
+// +- diag / h^3, and the clamp to the edge (the sum reads zero outside) adds the
+// cell's own w back on the faces of the grid.
+// A thread owns two cells along x.  The curl of psi reads global memory at the
+// end of a plane.  Bound by vector issue and the loads of psi; us a launch, sum
+// over pairs with a ring of 2K+1 planes -> here: 32^3
+// (FP64 psi) 80 -> 17, 64^3 85 -> 20, 96^3 88 -> 44, 128^3 101 -> 68, 256^3 504
+// -> 331 (FP32 psi 483 -> 295).  Held to 3 or 4 waves per SIMD the compiler
+// spills: 1.0 ms at 256^3.
+constexpr int kCfThreads = 256;
+
+template <typename TP, typename TC, int K, int TX, bool EVEN>
+__global__ void __launch_bounds__(kCfThreads) k_curl_far(const TP* __restrict__ psi, const float* __restrict__ wg,
+                                                         float* __restrict__ far, const float* __restrict__ dir,
+                                                         uint32_t g, float h3, TC half_invh, float diag_h3, int zc) {
+    constexpr bool kSum = K >= 0;           // else the grid velocity alone
+    constexpr int KC = K < 1 ? 1 : K;       // reach of the sum with the diagonal term
+    constexpr int KE = KC + (KC & 1);       // x halo, even
+    constexpr int W = 2 * KC + 1;
+    constexpr int TXT = TX / 2, TY = kCfThreads / TXT;
+    constexpr int LX = TX + 2 * KE, LY = TY + 2 * KC, PL = LX * LY, NV = 2 + 2 * KE;
+    constexpr int NL = (3 * PL + kCfThreads - 1) / kCfThreads;
+    __shared__ float2 pl[2][kSum ? 3 * PL / 2 : 1];
+    const int gi = (int)g, tid = threadIdx.x;
+    const size_t G = (size_t)g * g * g;
+    const int tilesx = (gi + TX - 1) / TX;
+    const int bx = blockIdx.x % tilesx, by = blockIdx.x / tilesx;
+    const int z0 = blockIdx.y * zc, z1 = min(z0 + zc, gi);
+    const int tx = tid % TXT, ty = tid / TXT;
+    const int i = bx * TX + 2 * tx, j = by * TY + ty;
+    const int gx0 = bx * TX - KE, gy0 = by * TY - KC;
+    auto at = [&](int a, int b, int c) { return ((size_t)c * g + (size_t)b) * g + (size_t)a; };
+
+    float acc[W][3][2];
+#pragma unroll
+    for (int s = 0; s < W; s++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) acc[s][c][0] = acc[s][c][1] = 0.f;
+
+    // plane p of w into registers (zero outside the grid), then LDS
+    float ld[NL];
+    auto fetch = [&](int p) {
+#pragma unroll
+        for (int u = 0; u < NL; u++) {
+            const int q = tid + kCfThreads * u, c = q / PL, r = q - c * PL, yy = r / LX, xx = r - yy * LX;
+            const int ii = gx0 + xx, jj = gy0 + yy;
+            const bool ok = c < 3 && p >= 0 && p < gi && ii >= 0 && ii < gi && jj >= 0 && jj < gi;
+            ld[u] = ok ? wg[c * G + at(ii, jj, p)] : 0.f;
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < NL; u++)
+            if (tid + kCfThreads * u < 3 * PL) reinterpret_cast<float*>(pl[buf])[tid + kCfThreads * u] = ld[u];
+    };
+    // component a of dir at (dx, dy, dz) >= 0, the diagonal term included
+    auto coef = [&](int a, int dx, int dy, int dz) { return dir[3 * (((dz + KC) * W + dy + KC) * W + dx + KC) + a]; };
+    // outputs z0 .. z1 - 1; plane p = z0 - KC + s, output p - KC complete
+    // after it.  Slot of output k: (k - z0 + KC) mod W.
+    const int steps = (kSum ? z1 - z0 + 2 * KC : z1 - z0);
+    if (kSum) {
+        fetch(z0 - KC);
+        store(0);
+        __syncthreads();
+    }
+    for (int s0 = 0; s0 < steps; s0 += W) {
+#pragma unroll
+        for (int sj = 0; sj < W; sj++) {
+            const int s = s0 + sj;
+            if (s >= steps) continue;
+            const int p = kSum ? z0 - KC + s : z0 + s;
+            const int k = kSum ? p - KC : p;  // the output that ends here
+            if (kSum) {
+                if (s + 1 < steps) fetch(p + 1);
+                if (p >= 0 && p < gi) {
+                    float ctr[3][2];  // the cells' own w
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        // rows of component c, folded over +-y
+                        float E[KC + 1][NV], O[KC + 1][NV];
+#pragma unroll
+                        for (int r = 0; r <= KC; r++) {
+                            const float2* up = &pl[s & 1][(c * PL + (ty + KC + r) * LX) / 2 + tx];
+                            const float2* dn = &pl[s & 1][(c * PL + (ty + KC - r) * LX) / 2 + tx];
+#pragma unroll
+                            for (int q = 0; q < NV / 2; q++) {
+                                const float2 a = up[q];
+                                if (r == 0) {
+                                    E[0][2 * q] = a.x;
+                                    E[0][2 * q + 1] = a.y;
+                                } else {
+                                    const float2 b = dn[q];
+                                    E[r][2 * q] = a.x + b.x;
+                                    E[r][2 * q + 1] = a.y + b.y;
+                                    O[r][2 * q] = a.x - b.x;
+                                    O[r][2 * q + 1] = a.y - b.y;
+                                }
+                            }
+                        }
+#pragma unroll
+                        for (int e = 0; e < 2; e++) {
+                            const int m = KE + e;
+                            ctr[c][e] = E[0][m];
+                            // sums over the plane for |dz| = 0 .. KC: with
+                            // dir_2 (even in x and y; odd in z, so none at
+                            // dz = 0), dir_0 (odd in x), dir_1 (odd in y)
+                            float s2[KC + 1], s0_[KC + 1], s1[KC + 1];
+#pragma unroll
+                            for (int dz = 0; dz <= KC; dz++) s2[dz] = s0_[dz] = s1[dz] = 0.f;
+#pragma unroll
+                            for (int dy = 0; dy <= KC; dy++)
+#pragma unroll
+                                for (int dx = 0; dx <= KC; dx++) {
+                                    const float ee = dx == 0 ? E[dy][m] : E[dy][m + dx] + E[dy][m - dx];
+                                    const float oe = dx == 0 ? 0.f : E[dy][m + dx] - E[dy][m - dx];
+                                    const float eo = dy == 0   ? 0.f
+                                                     : dx == 0 ? O[dy][m]
+                                                               : O[dy][m + dx] + O[dy][m - dx];
+#pragma unroll
+                                    for (int dz = 0; dz <= KC; dz++) {
+                                        if (K < 1 && dx + dy + dz != 1) continue;  // no local correction
+                                        if (c != 2 && dz > 0) s2[dz] = fmaf(coef(2, dx, dy, dz), ee, s2[dz]);
+                                        if (c != 0 && dx > 0) s0_[dz] = fmaf(coef(0, dx, dy, dz), oe, s0_[dz]);
+                                        if (c != 1 && dy > 0) s1[dz] = fmaf(coef(1, dx, dy, dz), eo, s1[dz]);
+                                    }
+                                }
+                            // dir x w: x = d1 wz - d2 wy, y = d2 wx - d0 wz,
+                            // z = d0 wy - d1 wx, of outputs p - dz (D_z = dz)
+                            // and p + dz (dir_2 turned round)
+#pragma unroll
+                            for (int dz = 0; dz <= KC; dz++) {
+                                const int sl = (sj - dz + W) % W, sh = (sj + dz) % W;
+                                if (c == 0) {
+                                    acc[sl][1][e] += s2[dz];
+                                    acc[sl][2][e] -= s1[dz];
+                                    if (dz > 0) {
+                                        acc[sh][1][e] -= s2[dz];
+                                        acc[sh][2][e] -= s1[dz];
+                                    }
+                                } else if (c == 1) {
+                                    acc[sl][0][e] -= s2[dz];
+                                    acc[sl][2][e] += s0_[dz];
+                                    if (dz > 0) {
+                                        acc[sh][0][e] += s2[dz];
+                                        acc[sh][2][e] += s0_[dz];
+                                    }
+                                } else {
+                                    acc[sl][0][e] += s1[dz];
+                                    acc[sl][1][e] -= s0_[dz];
+                                    if (dz > 0) {
+                                        acc[sh][0][e] += s1[dz];
+                                        acc[sh][1][e] -= s0_[dz];
+                                    }
+                                }
+                            }
+                        }
+                    }
+                    // the diagonal term's differences clamp to the edge
+                    if (p == 0 || p == gi - 1 || j == 0 || j == gi - 1 || i == 0 || i + 2 >= gi) {
+#pragma unroll
+                        for (int e = 0; e < 2; e++) {
+                            const float fx = diag_h3 * ((i + e == gi - 1 ? 1.f : 0.f) - (i + e == 0 ? 1.f : 0.f));
+                            const float fy = diag_h3 * ((j == gi - 1 ? 1.f : 0.f) - (j == 0 ? 1.f : 0.f));
+                            const float fz = diag_h3 * ((p == gi - 1 ? 1.f : 0.f) - (p == 0 ? 1.f : 0.f));
+                            acc[sj][0][e] += fy * ctr[2][e] - fz * ctr[1][e];
+                            acc[sj][1][e] += fz * ctr[0][e] - fx * ctr[2][e];
+                            acc[sj][2][e] += fx * ctr[1][e] - fy * ctr[0][e];
+                        }
+                    }
+                }
+            }
+            constexpr int KO = kSum ? KC : 0;
+            const int so = (sj - KO + W) % W;
+            if (k >= z0 && k < z1 && i < gi && j < gi) {
+                const int jm = j > 0 ? j - 1 : 0, jp = j < gi - 1 ? j + 1 : gi - 1;
+                const int km = k > 0 ? k - 1 : 0, kp = k < gi - 1 ? k + 1 : gi - 1;
+                const TP* Px = psi;
+                const TP* Py = psi + G;
+                const TP* Pz = psi + 2 * G;
+                // psi at the pair's neighbours; pairs in one access when the rows
+                // keep them aligned (g even)
+                const bool have1 = i + 1 < gi;
+                TC zp_[2], zm_[2], xp_[2], xm_[2], yzm[2], yzp[2], xzm[2], xzp[2], zx[4], yx[4];
+                auto pair = [&](const TP* P, size_t t, TC* v) {
+                    if (EVEN) {
+                        struct alignas(2 * sizeof(TP)) P2 { TP a, b; };
+                        const P2 q = *reinterpret_cast<const P2*>(P + t);
+                        v[0] = (TC)q.a;
+                        v[1] = (TC)q.b;
+                    } else {
+                        v[0] = (TC)P[t];
+                        v[1] = (TC)P[t + (have1 ? 1 : 0)];
+                    }
+                };
+                pair(Pz, at(i, jp, k), zp_);
+                pair(Pz, at(i, jm, k), zm_);
+                pair(Py, at(i, j, km), yzm);
+                pair(Py, at(i, j, kp), yzp);
+                pair(Px, at(i, j, kp), xzp);
+                pair(Px, at(i, j, km), xzm);
+                pair(Px, at(i, jm, k), xm_);
+                pair(Px, at(i, jp, k), xp_);
+                pair(Pz, at(i, j, k), zx + 1);
+                pair(Py, at(i, j, k), yx + 1);
+                const size_t tl = at(i > 0 ? i - 1 : 0, j, k), tr = at(min(i + 2, gi - 1), j, k);
+                zx[0] = (TC)Pz[tl];
+                zx[3] = (TC)Pz[tr];
+                yx[0] = (TC)Py[tl];
+                yx[3] = (TC)Py[tr];
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    if (e == 1 && !have1) continue;
+                    // curl(psi), GPU_kernel.cu:1770-1786 (evaluation order kept)
+                    const TC ux = half_invh * (zp_[e] - zm_[e] + yzm[e] - yzp[e]);
+                    const TC uy = half_invh * (xzp[e] - xzm[e] + zx[e] - zx[e + 2]);
+                    const TC uz = half_invh * (yx[e + 2] - yx[e] + xm_[e] - xp_[e]);
+                    const size_t c = at(i + e, j, k);
+                    far[c] = (float)((double)ux - (double)(acc[so][0][e] * h3));
+                    far[G + c] = (float)((double)uy - (double)(acc[so][1][e] * h3));
+                    far[2 * G + c] = (float)((double)uz - (double)(acc[so][2][e] * h3));
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 3; c++) acc[so][c][0] = acc[so][c][1] = 0.f;  // output p + KC + 1 takes the slot
+            if (kSum) {
+                if (s + 1 < steps) store((s + 1) & 1);
+                __syncthreads();
+            }
+        }
+    }
 }
 
+// K = 4: the sums of nine planes do not fit the registers of k_curl_far (1.0 to
+// 1.7 ms at 128^3 against 0.64 here), so the sum runs over pairs of neighbours.
 // A workgroup owns a 32 x 8 tile of cells and a run of z planes.  The grid
 // vorticity streams through an LDS ring of 2K+1 planes with a K-cell halo
 // (zero outside the grid, which is the reference's in-grid-only sum), so the
-// (2K+1)^3 local correction and the curl of the diagonal term read LDS; the
-// curl of psi reads global memory (12 loads, mostly L2 hits).
-constexpr int kCfTX = 32, kCfTY = 8, kCfZC = 16;
+// (2K+1)^3 sum reads LDS; the curl of psi reads global memory (12 loads,
+// mostly L2 hits).
+constexpr int kCfTX = 32, kCfTY = 8;
 
 template <typename TP, typename TC, int K>
-__global__ void __launch_bounds__(256) k_curl_far(const TP* __restrict__ psi, const float* __restrict__ wg,
+__global__ void __launch_bounds__(256) k_curl_far_pairs(const TP* __restrict__ psi, const float* __restrict__ wg,
                                                   float* __restrict__ far, const float* __restrict__ dir, uint32_t g,
-                                                  float h3, TC half_invh, float cdiag_half_invh) {
+                                                  float h3, TC half_invh, float diag_h3,
+                                                  int zc) {
     constexpr int W = 2 * K + 1, LXW = kCfTX + 2 * K, LYW = kCfTY + 2 * K, PLW = LXW * LYW;
-    __shared__ float ring[W > 0 ? W : 1][3][PLW];
+    __shared__ float ring[W][3][PLW];
     const uint32_t G = g * g * g;
     const int gi = (int)g;
     const int tilesx = (gi + kCfTX - 1) / kCfTX, tilesy = (gi + kCfTY - 1) / kCfTY;
     const int bx = blockIdx.x % tilesx, by = blockIdx.x / tilesx;
-    const int z0 = blockIdx.y * kCfZC, z1 = min(z0 + kCfZC, gi);
+    const int z0 = blockIdx.y * zc, z1 = min(z0 + zc, gi);
     const int lx = threadIdx.x % kCfTX, ly = threadIdx.x / kCfTX;
     const int i = bx * kCfTX + lx, j = by * kCfTY + ly;
     const int gx0 = bx * kCfTX - K, gy0 = by * kCfTY - K;
@@ -59,10 +300,9 @@ __global__ void __launch_bounds__(256) k_curl_far(const TP* __restrict__ psi, co
             rp[2 * PLW + q] = vz;
         }
     };
-    if (K >= 0)
-        for (int kk = z0 - K; kk < z0 + K; kk++) load_plane(kk);
+    for (int kk = z0 - K; kk < z0 + K; kk++) load_plane(kk);
     for (int k = z0; k < z1; k++) {
-        if (K >= 0) load_plane(k + K);
+        load_plane(k + K);
         __syncthreads();
         if (i < gi && j < gi) {
             const int im = i > 0 ? i - 1 : 0, ip = i < gi - 1 ? i + 1 : gi - 1;
@@ -78,27 +318,21 @@ __global__ void __launch_bounds__(256) k_curl_far(const TP* __restrict__ psi, co
                                  (TC)Pz[at(ip, j, k)]);
             TC uz = half_invh * ((TC)Py[at(ip, j, k)] - (TC)Py[at(im, j, k)] + (TC)Px[at(i, jm, k)] -
                                  (TC)Px[at(i, jp, k)]);
-            // diagonal term: curl of 0.2505806 h^2 w with the same clamped
-            // stencil; for K >= 1 the ring holds the neighbours (the clamp
-            // reads the edge cell itself, which the ring holds too)
-            float dx, dy, dz;
-            if (K >= 1) {
-                auto wr = [&](int comp, int ii, int jj, int kk) {
-                    return ring[((kk % W) + W) % W][comp][(jj - gy0) * LXW + (ii - gx0)];
-                };
-                dx = cdiag_half_invh * (wr(2, i, jp, k) - wr(2, i, jm, k) + wr(1, i, j, km) - wr(1, i, j, kp));
-                dy = cdiag_half_invh * (wr(0, i, j, kp) - wr(0, i, j, km) + wr(2, im, j, k) - wr(2, ip, j, k));
-                dz = cdiag_half_invh * (wr(1, ip, j, k) - wr(1, im, j, k) + wr(0, i, jm, k) - wr(0, i, jp, k));
-            } else {
-                dx = cdiag_half_invh * (Wz[at(i, jp, k)] - Wz[at(i, jm, k)] + Wy[at(i, j, km)] - Wy[at(i, j, kp)]);
-                dy = cdiag_half_invh * (Wx[at(i, j, kp)] - Wx[at(i, j, km)] + Wz[at(im, j, k)] - Wz[at(ip, j, k)]);
-                dz = cdiag_half_invh * (Wy[at(ip, j, k)] - Wy[at(im, j, k)] + Wx[at(i, jm, k)] - Wx[at(i, jp, k)]);
-            }
             // local correction over the (2K+1)^3 block.  dir is odd,
             // dir[-D] = -dir[D] (a central difference of the even 1/(4 pi |r|),
             // computed so in FP64 and rounded), so D and -D are taken
             // together: dir[D] x (w[c+D] - w[c-D]); h^3 is applied once.
             float vx = 0.f, vy = 0.f, vz = 0.f;
+            if (k == 0 || k == gi - 1 || j == 0 || j == gi - 1 || i == 0 || i == gi - 1) {
+                // the diagonal term's differences clamp to the edge
+                const float* c = &ring[((k % W) + W) % W][0][(ly + K) * LXW + lx + K];
+                const float fx = diag_h3 * ((i == gi - 1 ? 1.f : 0.f) - (i == 0 ? 1.f : 0.f));
+                const float fy = diag_h3 * ((j == gi - 1 ? 1.f : 0.f) - (j == 0 ? 1.f : 0.f));
+                const float fz = diag_h3 * ((k == gi - 1 ? 1.f : 0.f) - (k == 0 ? 1.f : 0.f));
+                vx = fy * c[2 * PLW] - fz * c[PLW];
+                vy = fz * c[0] - fx * c[2 * PLW];
+                vz = fx * c[PLW] - fy * c[0];
+            }
 #pragma unroll
             for (int a = 0; a <= K; a++) {
                 const float* rp = &ring[(((k + a) % W) + W) % W][0][0];
@@ -125,26 +359,37 @@ __global__ void __launch_bounds__(256) k_curl_far(const TP* __restrict__ psi, co
             vy *= h3;
             vz *= h3;
             const size_t c = at(i, j, k);
-            far[c] = (float)((double)ux - (double)vx - (double)dx);
-            far[(size_t)G + c] = (float)((double)uy - (double)vy - (double)dy);
-            far[2 * (size_t)G + c] = (float)((double)uz - (double)vz - (double)dz);
+            far[c] = (float)((double)ux - (double)vx);
+            far[(size_t)G + c] = (float)((double)uy - (double)vy);
+            far[2 * (size_t)G + c] = (float)((double)uz - (double)vz);
         }
         __syncthreads();  // the next plane load reuses the slot of plane k - K
     }
 }
 
-template <typename TP, typename TC>
+template <typename TP, typename TC, int TX, bool EVEN>
 static void launch_curl_far_k(const TP* psi, const float* wgrid, float* far, const float* dir, uint32_t g, int K,
                               float h3, TC half_invh, float cd, hipStream_t st) {
-    const uint32_t tiles = div_up(g, kCfTX) * div_up(g, kCfTY);
-    dim3 grid(tiles, div_up(g, kCfZC)), blk(256);
+    constexpr int TY = kCfThreads / (TX / 2);
+    const uint32_t tiles = div_up(g, TX) * div_up(g, TY);
+    // planes per workgroup: about three workgroups per CU in all; longer runs
+    // (up to 32) repeat fewer of the 2K planes around them, shorter ones (down
+    // to 2) keep the chip busy on small grids
+    const int zc = std::max(2, std::min(32, (int)div_up(g * tiles, 768)));
+    dim3 grid(tiles, div_up(g, zc)), blk(kCfThreads);
     switch (K) {
-        case 0: hipLaunchKernelGGL((k_curl_far<TP, TC, 0>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd); break;
-        case 1: hipLaunchKernelGGL((k_curl_far<TP, TC, 1>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd); break;
-        case 2: hipLaunchKernelGGL((k_curl_far<TP, TC, 2>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd); break;
-        case 3: hipLaunchKernelGGL((k_curl_far<TP, TC, 3>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd); break;
-        case 4: hipLaunchKernelGGL((k_curl_far<TP, TC, 4>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd); break;
-        default: hipLaunchKernelGGL((k_curl_far<TP, TC, -1>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd); break;
+        case 0: hipLaunchKernelGGL((k_curl_far<TP, TC, 0, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
+        case 1: hipLaunchKernelGGL((k_curl_far<TP, TC, 1, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
+        case 2: hipLaunchKernelGGL((k_curl_far<TP, TC, 2, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
+        case 3: hipLaunchKernelGGL((k_curl_far<TP, TC, 3, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
+        case 4: {
+            // two workgroups (69 KB of LDS each) a CU
+            const uint32_t t4 = div_up(g, kCfTX) * div_up(g, kCfTY);
+            const int zc4 = std::max(2, std::min(16, (int)div_up(g * t4, 512)));
+            hipLaunchKernelGGL((k_curl_far_pairs<TP, TC, 4>), dim3(t4, div_up(g, zc4)), blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc4);
+            break;
+        }
+        default: hipLaunchKernelGGL((k_curl_far<TP, TC, -1, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
     }
 }
 
@@ -152,12 +397,25 @@ pppm_status launch_curl_far_impl(const void* psi, int psi_dtype, const float* wg
                                  uint32_t g, int K, double h, hipStream_t st) {
     const float h3 = (float)(h * h * h);
     const double half_invh = 0.5 * (1.0 / h);
-    // vortex-in-cell (K < 0): the far-field buffer is the grid velocity itself
-    const float cd = K < 0 ? 0.0f : (float)(kRefDiagPsi * h * h * half_invh);
-    if (psi_dtype == PPPM_F64)
-        launch_curl_far_k<double, double>((const double*)psi, wgrid, far, dir, g, K, h3, half_invh, cd, st);
-    else
-        launch_curl_far_k<float, float>((const float*)psi, wgrid, far, dir, g, K, h3, (float)half_invh, cd, st);
+    // the diagonal term's difference factor over h^3 (the sum is scaled by
+    // h^3); vortex-in-cell (K < 0): the buffer is the grid velocity itself
+    const float cd = K < 0 ? 0.0f : (float)(kRefDiagPsi * h * h * half_invh / (h * h * h));
+    // 64-cell tiles along x, or 32 where they would leave a third of the
+    // threads or more without cells
+    const bool t64 = g % 64 == 0 || g > 128;
+    auto run = [&](auto* ps, auto hi, auto t64_, auto even) {
+        using TP = std::remove_const_t<std::remove_pointer_t<decltype(ps)>>;
+        launch_curl_far_k<TP, TP, decltype(t64_)::value ? 64 : 32, decltype(even)::value>(ps, wgrid, far, dir, g, K, h3,
+                                                                                        hi, cd, st);
+    };
+    auto by_size = [&](auto* ps, auto hi) {
+        using std::true_type;
+        using std::false_type;
+        if (g % 2 == 0) t64 ? run(ps, hi, true_type(), true_type()) : run(ps, hi, false_type(), true_type());
+        else t64 ? run(ps, hi, true_type(), false_type()) : run(ps, hi, false_type(), false_type());
+    };
+    if (psi_dtype == PPPM_F64) by_size((const double*)psi, half_invh);
+    else by_size((const float*)psi, (float)half_invh);
     PPPM_LAUNCH_CHECK();
     return PPPM_OK;
 }
