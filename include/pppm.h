@@ -317,12 +317,12 @@ pppm_status pppm_mg_vcycles(pppm_mg *mg, void *x, const void *b, int32_t nu1, in
 pppm_status pppm_mg_smooth(pppm_mg *mg, void *x, const void *b, int32_t iters, double omega, int32_t blocked,
                            void *hip_stream);
 /* PPPM_F32 V-cycles on levels at or above the blocked threshold (below):
- * blocked = 1..4 (the kinds of pppm_mg_smooth; default 2) use fused blocked
+ * blocked = 1..4 (the kinds of pppm_mg_smooth; default 4) use fused blocked
  * passes, 0 one launch per half-sweep, residual, restriction and
  * prolongation. */
 pppm_status pppm_mg_set_blocked(pppm_mg *mg, int32_t blocked);
 /* Levels with at least this many cells per component take the blocked
- * passes in PPPM_F32 V-cycles (default 512K: 81^3 and larger); smaller ones
+ * passes in PPPM_F32 V-cycles (default 327680: 69^3 and larger); smaller ones
  * of even dimensions take tile passes (two red-black iterations with the
  * residual or the prolongation in one launch), others one launch per
  * half-sweep. */

@@ -362,11 +362,8 @@ __global__ void __launch_bounds__(256) k_rb2(TbArgs a) {
 }
 
 // Colour-split blocked smoother: the pass of k_rb2 (z planes streamed through
-// LDS rings, halos recomputed, out of place) with each LDS plane split by
-// colour, and S half-sweeps per pass (S = 2: one red-black iteration; S = 4:
-// two, which halves the passes over the grid of a V(2,2) cycle's finest
-// levels).  Row ly of colour c holds at
-// index m the colour-c cell of the cell pair (2m, 2m + 1) of that row.  Every
+// LDS rings, halos recomputed, out of place; one red-black iteration) with
+// each LDS plane split by colour.  Row ly of colour c holds at index m the colour-c cell of the cell pair (2m, 2m + 1) of that row.  Every
 // neighbour of a colour-c cell is of colour 1 - c: at index m in the rows
 // above and below and in the planes before and after, and at m + s - 1 and
 // m + s in its own row (s = 1 if the cell is the pair's second), so the reads
@@ -392,10 +389,10 @@ constexpr int kRcTY = 16;
 // alone, which allows two workgroups per CU; they are latency-bound, so their
 // registers are capped for three waves per SIMD (<= 168; no spills), the
 // occupancy their LDS allows.
-template <bool RESTRICT, bool PROLONG, bool XZERO, bool BETA, int NR, int S>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((RESTRICT || PROLONG) && S == 2 ? 3 : 1)))
+template <bool RESTRICT, bool PROLONG, bool XZERO, bool BETA, int NR>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RESTRICT || PROLONG ? 3 : 1)))
 k_rbc(TbArgs a) {
-    static_assert(S == 2 || S == 4, "one or two red-black iterations per pass");
+    constexpr int S = 2;                         // half-sweeps
     constexpr int H = S + (RESTRICT ? 1 : 0);    // halo: one cell per half-sweep, +1 for the residual
     constexpr int HXC = H + (H & 1);             // x halo in cells (even)
     constexpr int HY = H;                        // y and z halo
@@ -701,6 +698,331 @@ k_rbc(TbArgs a) {
     }
 }
 
+// Two red-black iterations (four half-sweeps) in one pass over the grid.  A
+// workgroup streams z planes of a 64 x 64 cell region; a thread owns the cell
+// pair m of two rows (2 rg, 2 rg + 1) and keeps its cells and right-hand side
+// of the planes in flight in registers, so that neighbours in z, in the own
+// pair and in the other row are registers, the neighbouring pair is a lane
+// shift, and only the rows above and below come through LDS: one cell of one
+// colour a row and half-sweep.  In step k plane k arrives (state 0) and
+// half-sweep t updates plane k - t, t ascending.  What half-sweep t reads of
+// other threads (plane k - t after t - 1) was written in step k - 1, and
+// what it reads of its own thread's planes k - t + 1 (after t - 1, this step)
+// and k - t - 1 (before t + 1) is in program order: one barrier a plane, where
+// k_rbc needs one or two a half-sweep.  The region's outer cells become wrong
+// by one cell a half-sweep (and one for the residual): a halo of 4 cells, 6
+// (5, even) for the residual from a start that is not zero; a zero start is
+// exact beyond the region, which saves one.  Planes outside the grid are
+// zero and stay so, as cells outside it in x and y.  Needs nx even.
+//
+// Sums are formed in k_rbc's order.  One workgroup of 16 waves a CU, bound
+// by its planes' loads and by vector issue at once.  256^3 x 3, V(2,2) (us):
+// down from zero 107 + 179 (two k_rbc passes) -> 128, up 203 + 151 -> 205;
+// 96^3 x 3: 39 -> 18, 41 -> 22.
+constexpr int kR4Region = 64;
+
+template <bool RESTRICT, bool PROLONG, bool XZERO, bool BETA>
+__global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
+    constexpr bool kWide = RESTRICT && !XZERO;
+    constexpr int HXY = kWide ? 6 : 4, HZ = kWide ? 5 : 4;
+    constexpr int TW = kR4Region - 2 * HXY;  // tile
+    constexpr int NR = RESTRICT ? 8 : 6;     // planes in flight
+    constexpr int ES = 34 * 32;              // row groups -1 .. 32 of one row parity
+    // exchanged rows: state t of plane k - t, stored in step j, goes to slot
+    // xslot(t, j); states 0 .. 3 are read one step later (two buffers), the
+    // residual also reads state 4 one step and state 3 two steps later (four)
+    constexpr int NE = RESTRICT ? 12 : 8;
+    auto xslot = [](int t, int j) {
+        return t < 3 ? 2 * t + (j & 1) : t == 3 ? 6 + (j & (RESTRICT ? 3 : 1)) : 10 + (j & 1);
+    };
+    constexpr int CW = 34;  // coarse window of the prolongation
+    __shared__ float ex[NE][2][ES];
+    __shared__ float cw[PROLONG ? 3 : 1][PROLONG ? CW * CW : 1];
+    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const uint32_t tile = xcd_block(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
+                                    gridDim.x * gridDim.y * gridDim.z);
+    const int bx = (int)(tile % gridDim.x), by = (int)((tile / gridDim.x) % gridDim.y);
+    const int bz = (int)(tile / (gridDim.x * gridDim.y));
+    const int gx0 = bx * TW - HXY, gy0 = by * TW - HXY;
+    const int nzc = (nz + a.zc - 1) / a.zc;
+    const int comp = bz / nzc, zi = bz - comp * nzc;
+    const int z0 = zi * a.zc, z1 = min(z0 + a.zc, nz);
+    const float* xsrc = XZERO ? nullptr : a.xin + (size_t)comp * a.G;
+    float* xdst = a.x + (size_t)comp * a.G;
+    const float* bcp = a.b + (size_t)comp * a.G;
+    const float* xcoarse = PROLONG ? a.xc + (size_t)comp * a.Gc : nullptr;
+    float* bnext = RESTRICT ? a.bn + (size_t)comp * a.Gc : nullptr;
+    const int klo = max(z0 - HZ, 0), khi = min(z1 + HZ, nz);
+    const int kend = z1 + 4 + (RESTRICT ? 1 : 0);
+    const int kbeg = klo & ~1;  // ring slots and plane parities by the step count
+    const size_t plane = (size_t)nx * ny;
+    const float omega = a.omega, beta = a.beta, bscale = a.bscale;
+    const int tid = threadIdx.x, m = tid & 31, rg = tid >> 5;
+    const int i0 = gx0 + 2 * m;
+    const bool xin = i0 >= 0 && i0 < nx;
+    for (int q = tid; q < NE * 2 * ES; q += 1024) (&ex[0][0][0])[q] = 0.f;
+
+    // Planes are read and written as buffers of plane bytes (0 bytes: none),
+    // so that loads off the grid give zero and stores outside the tile are
+    // dropped without a branch: a step is straight-line code, and its loads
+    // are waited for a whole step later.
+    constexpr uint32_t kOff = 0x80000000u;  // beyond any plane
+    const uint32_t pbytes = (uint32_t)(plane * sizeof(float));
+    uint32_t lofs[2], sofs[2];
+    bool gin[2];
+    float wr[2];
+    // cells outside the grid next to a cell in the plane, and the diagonal's
+    // reciprocal off and on the first and last plane
+    float nxy[2][2], d0[2][2], d1[2][2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int j = gy0 + 2 * rg + r, ly = 2 * rg + r;
+        gin[r] = xin && j >= 0 && j < ny;
+        lofs[r] = gin[r] ? 4u * (uint32_t)(j * nx + i0) : kOff;
+        wr[r] = gin[r] ? omega : 0.f;
+        sofs[r] = ly >= HXY && ly < HXY + TW && 2 * m >= HXY && 2 * m < HXY + TW ? lofs[r] : kOff;
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int i = i0 + e;
+            nxy[r][e] = (float)((i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1));
+            d0[r][e] = 1.0f / (6.0f - beta * nxy[r][e]);
+            d1[r][e] = 1.0f / (6.0f - beta * (nxy[r][e] + (nz == 1 ? 2.f : 1.f)));
+        }
+    }
+    const int gI = i0 >> 1, gJ = (gy0 >> 1) + rg;
+    const uint32_t cofs = RESTRICT && sofs[0] != kOff && gI < a.cx && gJ < a.cy ? 4u * (uint32_t)(gJ * a.cx + gI) : kOff;
+    auto buffer = [](const void* p, uint32_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
+    };
+
+    // [slot][row][pair cell]
+    float X[NR][2][2], B[NR][2][2];
+    uint2 px[2], pb[2];
+    float pc[2], pf = 0.f, rsum[2] = {0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < NR; q++)
+#pragma unroll
+        for (int r = 0; r < 2; r++) X[q][r][0] = X[q][r][1] = B[q][r][0] = B[q][r][1] = 0.f;
+    auto fetch = [&](int k) {
+        k = __builtin_amdgcn_readfirstlane(k);
+        const bool real = k >= klo && k < khi;
+        const size_t ko = real ? (size_t)k * plane : 0;
+        const auto rb = buffer(bcp + ko, real ? pbytes : 0u);
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            px[r] = make_uint2(0u, 0u);
+            if (!XZERO) {
+                const auto rx = buffer(xsrc + ko, real ? pbytes : 0u);
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(rx, lofs[r], 0, 0);
+                px[r] = make_uint2(v[0], v[1]);
+            }
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rb, lofs[r], 0, 0);
+            pb[r] = make_uint2(v[0], v[1]);
+        }
+    };
+    // the coarse window, ghost-extended as k_rbc's; plane c in slot (c + 3) % 3.
+    // A thread's two cells (the last of them beyond the window: not stored)
+    const int cx0 = (gx0 >> 1) - 1, cy0 = (gy0 >> 1) - 1;
+    uint32_t cq[2];  // byte offsets
+    float cf[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int q = min(tid + 1024 * u, CW * CW - 1);
+        const int ci = cx0 + q % CW, cj = cy0 + q / CW;
+        const int cic = PROLONG ? min(max(ci, 0), a.cx - 1) : 0, cjc = PROLONG ? min(max(cj, 0), a.cy - 1) : 0;
+        cq[u] = 4u * (uint32_t)(cjc * a.cx + cic);
+        cf[u] = (cic != ci ? a.betac : 1.f) * (cjc != cj ? a.betac : 1.f);
+    }
+    auto fetch_coarse = [&](int c) {
+        const int cc = min(max(c, 0), a.cz - 1);
+        pf = cc != c ? a.betac : 1.f;
+        const char* p = reinterpret_cast<const char*>(xcoarse + (size_t)__builtin_amdgcn_readfirstlane(cc) * a.cy * a.cx);
+        pc[0] = *reinterpret_cast<const float*>(p + cq[0]);
+        pc[1] = *reinterpret_cast<const float*>(p + cq[1]);
+    };
+    auto store_coarse = [&](int c) {
+        float* w = cw[(c + 3) % 3];
+        w[tid] = pc[0] * (cf[0] * pf);
+        if (tid + 1024 < CW * CW) w[tid + 1024] = pc[1] * (cf[1] * pf);
+    };
+    if (PROLONG) {
+        // (klo is even: the first step stores plane klo / 2 + 1)
+        for (int c = (klo >> 1) - 1; c <= (klo >> 1); c++) {
+            fetch_coarse(c);
+            store_coarse(c);
+        }
+        fetch_coarse((klo >> 1) + 1);
+    }
+    fetch(kbeg);
+    __syncthreads();
+
+    // the neighbouring pair's cell: lane - 1's (m > 0) or lane + 1's; the
+    // region's edge lanes read a row that is not theirs, inside the halo
+    auto from_left = [](float v) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, false));
+    };
+    auto from_right = [](float v) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, false));
+    };
+    const int lo = rg * 32 + m;  // row group rg - 1 in an exchanged row; rg + 1 at lo + 64
+
+    for (int k0 = kbeg;; k0 += NR) {
+#pragma unroll
+        for (int j = 0; j < NR; j++) {
+            const int k = k0 + j;  // k & 1 == j & 1
+            if (k >= kend) return;
+            // ---- the exchanged rows of this step (with the coarse window's
+            // cells in registers too, spills: the prolongation goes first)
+            float y[4][2];
+            auto exchanged = [&]() {
+#pragma unroll
+                for (int t = XZERO ? 2 : 1; t <= 4; t++) {
+                    y[t - 1][0] = ex[xslot(t - 1, j + 3)][1][lo];
+                    y[t - 1][1] = ex[xslot(t - 1, j + 3)][0][lo + 64];
+                }
+            };
+            // of the residual: [row][colour]; colour 1 was last written by
+            // half-sweep 3, colour 0 by 4
+            float yr[2][2];
+            if (RESTRICT) {
+                yr[0][0] = ex[xslot(3, j + 2)][1][lo];
+                yr[1][0] = ex[xslot(3, j + 2)][0][lo + 64];
+                yr[0][1] = ex[xslot(4, j + 3)][1][lo];
+                yr[1][1] = ex[xslot(4, j + 3)][0][lo + 64];
+            }
+            if (!PROLONG) exchanged();
+            // ---- state 0 of plane k (zero from khi on)
+            {
+                float v[2][2] = {{__uint_as_float(px[0].x), __uint_as_float(px[0].y)},
+                                 {__uint_as_float(px[1].x), __uint_as_float(px[1].y)}};
+                if (PROLONG) {
+                    // trilinear: parent column m + 1 of the window, neighbour m
+                    // (first cell) or m + 2; parent row rg + 1, neighbour rg
+                    // (first row) or rg + 2; parent plane k >> 1, neighbour one
+                    // up (k odd) or down
+                    const int pk = k >> 1, nk = pk + ((j & 1) ? 1 : -1);
+                    float w[2][2][2];
+                    // opaque: the slots repeat with the unrolled steps, and their
+                    // addresses would all be kept in registers (spills)
+                    int c00 = rg * CW + m;
+                    __asm__ volatile("" : "+v"(c00));
+#pragma unroll
+                    for (int z = 0; z < 2; z++) {
+                        const float* c0 = &cw[((z ? nk : pk) + 3) % 3][c00];
+                        float xe[3], xo[3];
+#pragma unroll
+                        for (int q = 0; q < 3; q++) {
+                            const float* c = c0 + q * CW;
+                            xe[q] = 0.75f * c[1] + 0.25f * c[0];
+                            xo[q] = 0.75f * c[1] + 0.25f * c[2];
+                        }
+#pragma unroll
+                        for (int r = 0; r < 2; r++) {
+                            w[z][r][0] = 0.75f * xe[1] + 0.25f * xe[2 * r];
+                            w[z][r][1] = 0.75f * xo[1] + 0.25f * xo[2 * r];
+                        }
+                    }
+                    const bool real = k < khi;
+#pragma unroll
+                    for (int r = 0; r < 2; r++)
+#pragma unroll
+                        for (int e = 0; e < 2; e++) {
+                            const float f = v[r][e] + (0.75f * w[0][r][e] + 0.25f * w[1][r][e]);
+                            v[r][e] = gin[r] && real ? f : v[r][e];
+                        }
+                }
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    X[j][r][0] = v[r][0];
+                    X[j][r][1] = v[r][1];
+                    B[j][r][0] = __uint_as_float(pb[r].x);
+                    B[j][r][1] = __uint_as_float(pb[r].y);
+                    // half-sweep 1 updates colour 1 and reads colour 0
+                    if (!XZERO) ex[xslot(0, j)][r][lo + 32] = X[j][r][(r ^ j) & 1];
+                }
+            }
+            if (PROLONG) {
+                if ((j & 1) == 0) store_coarse((k >> 1) + 1);  // fetched in step k - 1
+                else fetch_coarse(((k + 1) >> 1) + 1);
+            }
+            fetch(k + 1);
+            if (PROLONG) {
+                __builtin_amdgcn_sched_barrier(0);
+                exchanged();
+            }
+            // ---- half-sweep t on plane k - t
+#pragma unroll
+            for (int t = 1; t <= 4; t++) {
+                const int jp = (j - t + NR) % NR, jm = (jp + NR - 1) % NR, jq = (jp + 1) % NR;
+                const int p = k - t, c = t & 1;  // odd colour first, as the reference
+                const bool in = p >= 0 && p < nz, zb = p == 0 || p == nz - 1;
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    const int e = (c ^ r ^ jp) & 1;
+                    float s = 0.f;
+                    if (!(XZERO && t == 1)) {
+                        const float other = X[jp][r][1 - e];
+                        s = e ? other + from_right(X[jp][r][0]) : from_left(X[jp][r][1]) + other;
+                        s += r ? X[jp][0][e] + y[t - 1][1] : y[t - 1][0] + X[jp][1][e];
+                        s += X[jm][r][e] + X[jq][r][e];
+                    }
+                    s = fmaf(-bscale, B[jp][r][e], s);
+                    const float d = BETA ? (zb ? d1[r][e] : d0[r][e]) : 1.0f / 6.0f, xo = X[jp][r][e];
+                    const float xn = xo + (in ? wr[r] : 0.f) * (s * d - xo);
+                    X[jp][r][e] = xn;
+                    if (t < 4 || RESTRICT) ex[xslot(t, j)][r][lo + 32] = xn;
+                }
+            }
+            // ---- plane k - 4 is final
+            {
+                const int jw = (j + NR - 4) % NR, pw = __builtin_amdgcn_readfirstlane(k - 4);
+                const bool mine = pw >= z0 && pw < z1;
+                const auto rd = buffer(xdst + (mine ? (size_t)pw * plane : 0), mine ? pbytes : 0u);
+                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    const u32x2 v = {__float_as_uint(X[jw][r][0]), __float_as_uint(X[jw][r][1])};
+                    __builtin_amdgcn_raw_buffer_store_b64(v, rd, sofs[r], 0, 0);
+                }
+            }
+            // ---- residual of plane k - 5 and its restriction: this thread's
+            // 2 x 2 cells of a plane pair are one coarse cell
+            if (RESTRICT) {
+                const int jr = (j + NR - 5) % NR, jm = (jr + NR - 1) % NR, jq = (jr + 1) % NR, pr = k - 5;
+                const float zb = (float)((pr == 0) + (pr == nz - 1));
+                float part[2];
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    part[r] = 0.f;
+#pragma unroll
+                    for (int c = 0; c < 2; c++) {
+                        const int e = (c ^ r ^ jr) & 1;
+                        const float xo = X[jr][r][e], other = X[jr][r][1 - e];
+                        float s = e ? other + from_right(X[jr][r][0]) : from_left(X[jr][r][1]) + other;
+                        s += r ? X[jr][0][e] + yr[1][c] : yr[0][c] + X[jr][1][e];
+                        s += X[jm][r][e] + X[jq][r][e];
+                        s -= 6.0f * xo;
+                        if (BETA) s += beta * (nxy[r][e] + zb) * xo;
+                        part[r] += fmaf(bscale, B[jr][r][e], -s);
+                    }
+                }
+                if ((jr & 1) == 0) {
+                    rsum[0] = part[0];
+                    rsum[1] = part[1];
+                } else {
+                    const int gK = __builtin_amdgcn_readfirstlane(pr >> 1);
+                    const bool mine = pr >= z0 && pr < z1 && gK < a.cz;
+                    const auto rn = buffer(bnext + (mine ? (size_t)gK * a.cy * a.cx : 0),
+                                           mine ? 4u * (uint32_t)(a.cy * a.cx) : 0u);
+                    __builtin_amdgcn_raw_buffer_store_b32(
+                        __float_as_uint(((rsum[0] + part[0]) + (rsum[1] + part[1])) * 0.5f), rn, cofs, 0, 0);
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
 template <typename T>
 __device__ inline T residual_at(const T* __restrict__ x, const T* __restrict__ b, T bscale, int i, int j, int k,
                                 int nx, int ny, int nz, T beta) {
@@ -809,9 +1131,9 @@ __global__ void __launch_bounds__(256) k_prolong(T* __restrict__ x, const T* __r
 //
 // us of one V(2,2) cycle's level, three components, before -> here: 32^3 50
 // (11 launches) -> 16.5 (2), 64^3 51 (k_rbc) -> 34; FP64, one component: V(4,4)
-// at 64^3 and below 19 launches of 4.2 -> 4 of 11.  96^3: 92 against 83 with
-// k_rbc, so the line to the blocked passes lies at 512K cells.  1024 threads
-// take a 16^3 tile, 576 an 8^3 one.
+// at 64^3 and below 19 launches of 4.2 -> 4 of 11.  In FP32 the blocked passes
+// (k_rb4) are the faster from 72^3 (tb_min_cells_).  1024 threads take a 16^3
+// tile, 576 an 8^3 one.
 template <typename T>
 struct TileArgs {
     const T* xin;  // level before the pass (null: zero)
@@ -1731,11 +2053,11 @@ static int cu_count() {
 // Launch one k_rbc instantiation with z chunks sized so the whole grid is
 // resident at once (one round of workgroups: no tail), when the tiles leave
 // room for at least two chunks; otherwise the caller's chunking.
-template <bool R, bool P, bool Z, bool B, int NR, int S>
+template <bool R, bool P, bool Z, bool B, int NR>
 static int rbc_per_cu() {
     static int per_cu = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(&k_rbc<R, P, Z, B, NR, S>),
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(&k_rbc<R, P, Z, B, NR>),
                                                          256, 0) != hipSuccess ||
             n < 1)
             n = 1;
@@ -1748,33 +2070,27 @@ static int rbc_per_cu() {
 // stream capture.
 static void rbc_prime() {
     (void)cu_count();
-    (void)rbc_per_cu<false, false, false, false, 4, 2>();
-    (void)rbc_per_cu<false, false, false, true, 4, 2>();
-    (void)rbc_per_cu<false, false, true, false, 4, 2>();
-    (void)rbc_per_cu<false, false, true, true, 4, 2>();
-    (void)rbc_per_cu<false, true, false, false, 4, 2>();
-    (void)rbc_per_cu<false, true, false, true, 4, 2>();
-    (void)rbc_per_cu<false, false, false, false, 6, 2>();
-    (void)rbc_per_cu<false, false, false, true, 6, 2>();
-    (void)rbc_per_cu<false, false, true, false, 6, 2>();
-    (void)rbc_per_cu<false, false, true, true, 6, 2>();
-    (void)rbc_per_cu<false, true, false, false, 6, 2>();
-    (void)rbc_per_cu<false, true, false, true, 6, 2>();
-    (void)rbc_per_cu<true, false, false, false, 6, 2>();
-    (void)rbc_per_cu<true, false, false, true, 6, 2>();
-    (void)rbc_per_cu<true, false, true, false, 6, 2>();
-    (void)rbc_per_cu<true, false, true, true, 6, 2>();
-    (void)rbc_per_cu<false, true, false, false, 6, 4>();
-    (void)rbc_per_cu<false, true, false, true, 6, 4>();
-    (void)rbc_per_cu<true, false, false, false, 8, 4>();
-    (void)rbc_per_cu<true, false, false, true, 8, 4>();
-    (void)rbc_per_cu<true, false, true, false, 8, 4>();
-    (void)rbc_per_cu<true, false, true, true, 8, 4>();
+    (void)rbc_per_cu<false, false, false, false, 4>();
+    (void)rbc_per_cu<false, false, false, true, 4>();
+    (void)rbc_per_cu<false, false, true, false, 4>();
+    (void)rbc_per_cu<false, false, true, true, 4>();
+    (void)rbc_per_cu<false, true, false, false, 4>();
+    (void)rbc_per_cu<false, true, false, true, 4>();
+    (void)rbc_per_cu<false, false, false, false, 6>();
+    (void)rbc_per_cu<false, false, false, true, 6>();
+    (void)rbc_per_cu<false, false, true, false, 6>();
+    (void)rbc_per_cu<false, false, true, true, 6>();
+    (void)rbc_per_cu<false, true, false, false, 6>();
+    (void)rbc_per_cu<false, true, false, true, 6>();
+    (void)rbc_per_cu<true, false, false, false, 6>();
+    (void)rbc_per_cu<true, false, false, true, 6>();
+    (void)rbc_per_cu<true, false, true, false, 6>();
+    (void)rbc_per_cu<true, false, true, true, 6>();
 }
 
-template <bool R, bool P, bool Z, bool B, int NR, int S>
+template <bool R, bool P, bool Z, bool B, int NR>
 static void launch_rbc(TbArgs a, int ncomp, hipStream_t st) {
-    const int per_cu = rbc_per_cu<R, P, Z, B, NR, S>();
+    const int per_cu = rbc_per_cu<R, P, Z, B, NR>();
     const int tiles = (int)(div_up(a.nx, kRcTX) * div_up(a.ny, kRcTY)) * ncomp;
     const int chunks = per_cu * cu_count() / tiles;
     if (chunks >= 2) {
@@ -1784,14 +2100,36 @@ static void launch_rbc(TbArgs a, int ncomp, hipStream_t st) {
     }
     const int nzc = (a.nz + a.zc - 1) / a.zc;
     dim3 grid(div_up(a.nx, kRcTX), div_up(a.ny, kRcTY), nzc * ncomp), blk(256);
-    hipLaunchKernelGGL((k_rbc<R, P, Z, B, NR, S>), grid, blk, 0, st, a);
+    hipLaunchKernelGGL((k_rbc<R, P, Z, B, NR>), grid, blk, 0, st, a);
+}
+
+// k_rb4 over all components, one workgroup a CU at a time: the number of z
+// chunks that needs the fewest steps, rounds of workgroups times a chunk's
+// planes with its halo.
+template <bool R, bool P, bool Z, bool B>
+static void launch_rb4(TbArgs a, int ncomp, hipStream_t st) {
+    constexpr int tw = kR4Region - (R && !Z ? 12 : 8), halo = (R && !Z ? 10 : 8) + 4;
+    const int tx = (a.nx + tw - 1) / tw, ty = (a.ny + tw - 1) / tw;
+    const int64_t tiles = (int64_t)tx * ty * ncomp, cus = cu_count();
+    int64_t best = INT64_MAX;
+    for (int c = 1; c <= 64; c++) {
+        int zc = (a.nz + c - 1) / c;
+        zc += zc & 1;
+        const int64_t n = (a.nz + zc - 1) / zc, cost = (tiles * n + cus - 1) / cus * (zc + halo);
+        if (cost < best) {
+            best = cost;
+            a.zc = zc;
+        }
+    }
+    dim3 grid(tx, ty, (a.nz + a.zc - 1) / a.zc * ncomp);
+    hipLaunchKernelGGL((k_rb4<R, P, Z, B>), grid, dim3(1024), 0, st, a);
 }
 
 // One blocked pass over all components: kind 1 = k_rb2, 2 = k_rbc with a
 // four-plane ring, 3 = k_rbc with a six-plane ring (the residual pass always
 // uses six); k_rbc needs nx even, k_rb2 takes any size.
-// two_iter: two red-black iterations in the pass (k_rbc with S = 4; nx even,
-// kind 4 only), else one.
+// two_iter: two red-black iterations in the pass (k_rb4; nx even, kind 4
+// only), else one.
 template <bool R, bool P, bool Z>
 static pppm_status launch_rb2(const TbArgs& a, int ncomp, int kind, hipStream_t st, bool two_iter = false) {
     static_assert(kTbTX == kRcTX && kTbTY == kRcTY, "both blocked kernels use the same tiles");
@@ -1800,17 +2138,16 @@ static pppm_status launch_rb2(const TbArgs& a, int ncomp, int kind, hipStream_t 
     const bool beta = a.beta != 0.f;
     if (two_iter && (kind < 4 || (a.nx & 1) != 0)) return PPPM_ERR_INVALID;
     if (two_iter) {
-        constexpr int NRS4 = R ? 8 : 6;
-        if (beta) launch_rbc<R, P, Z, true, NRS4, 4>(a, ncomp, st);
-        else launch_rbc<R, P, Z, false, NRS4, 4>(a, ncomp, st);
+        if (beta) launch_rb4<R, P, Z, true>(a, ncomp, st);
+        else launch_rb4<R, P, Z, false>(a, ncomp, st);
     } else if (kind >= 2 && (a.nx & 1) == 0) {
-        if (R || kind >= 3) {
-            if (beta) launch_rbc<R, P, Z, true, 6, 2>(a, ncomp, st);
-            else launch_rbc<R, P, Z, false, 6, 2>(a, ncomp, st);
+        if (R || kind == 3) {
+            if (beta) launch_rbc<R, P, Z, true, 6>(a, ncomp, st);
+            else launch_rbc<R, P, Z, false, 6>(a, ncomp, st);
         } else {
             constexpr int NR4 = R ? 6 : 4;
-            if (beta) launch_rbc<R, P, Z, true, NR4, 2>(a, ncomp, st);
-            else launch_rbc<R, P, Z, false, NR4, 2>(a, ncomp, st);
+            if (beta) launch_rbc<R, P, Z, true, NR4>(a, ncomp, st);
+            else launch_rbc<R, P, Z, false, NR4>(a, ncomp, st);
         }
     } else if (beta) {
         hipLaunchKernelGGL((k_rb2<R, P, Z, true>), grid, blk, 0, st, a);
@@ -1957,7 +2294,8 @@ pppm_status MGHier<T>::tail(const T* xin, T* x, const T* b, T* b1, T bscale, int
 
 template <typename T>
 bool MGHier<T>::tile_level(int l, bool consistent) const {
-    if (!tb_ || l >= L_ - 1 || !has_temp(cells(l)) || cells(l) >= std::min(tb_min_cells_, kTileCells)) return false;
+    if (!tb_ || l >= L_ - 1 || !has_temp(cells(l)) || cells(l) >= kTileCells) return false;
+    if (cells(l) >= tb_min_cells_ && !(d_[l][0] & 1)) return false;  // k_rb4, k_rbc
     for (int c = 0; c < 3; c++)
         // without the one launch of the smallest levels the one above the
         // coarsest runs a launch per half-sweep, with bitwise its results
@@ -2139,7 +2477,7 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
     // amortise: levels below the hierarchy's threshold run the tile passes
     // (k_tile), or with odd dimensions the one-launch-per-colour kernels in
     // place.
-    auto blocked = [&](int l) { return m.cells(l) >= m.blocked_min_cells(); };
+    auto blocked = [&](int l) { return m.cells(l) >= m.blocked_min_cells() && m.even(l); };
     // the small levels in one launch where they fit (l0 >= 1: X and B of
     // those levels are the hierarchy's own)
     const int l0 = m.tail_level();
@@ -2229,9 +2567,11 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
 template <typename T>
 pppm_status MGHier<T>::vcycle(T* x0, const T* b0, T bscale0, int nu1, int nu2, T omega, bool consistent,
                               hipStream_t st, bool x0_zero) {
-    bool even = true;  // the blocked prolongation takes parents as i / 2
+    // the blocked prolongation takes parents as i / 2; a small odd level runs
+    // a launch per colour inside the fused cycle
+    bool even = true;
     for (int l = 0; l + 1 < L_; l++)
-        if (cells(l) >= tb_min_cells_) even = even && !(d_[l][0] & 1) && !(d_[l][1] & 1) && !(d_[l][2] & 1);
+        if (cells(l) >= std::max(tb_min_cells_, kTileCells)) even = even && this->even(l);
     if (std::is_same<T, float>::value && consistent && tb_ && (nu1 == 1 || nu1 == 2) && (nu2 == 1 || nu2 == 2) &&
         L_ > 1 && even) {
         std::vector<T*> X = x_, B = b_;
