@@ -649,8 +649,7 @@ extern "C" pppm_status pppm_set_vortices(pppm_ctx* c, uint32_t n, const float* p
     TRY(launch_calc_keys((const float4*)pos4, n, c->pg.hash, c->vs.k0, nullptr, st, osh != 0));
     TRY(radix_sort_pairs(c->vs.k0, c->vs.v0, c->vs.k1, c->vs.v1, n, key_bits_for(c->G) + osh, true, c->vs.scratch,
                          &c->vs.ks, &c->vs.vs, st));
-    TRY(launch_cell_tables(c->vs.ks, n, (uint32_t)c->G, c->cstart, c->cend, st, osh));
-    TRY(cell_offsets_from_tables(c->cstart, c->cend, (uint32_t)c->G, c->coff, c->scan_scr, st));
+    TRY(launch_cell_tables(c->vs.ks, n, (uint32_t)c->G, c->cstart, c->cend, st, osh, c->coff, c->scan_scr));
     TRY(launch_fill_u32(c->d_strays, 1, 0u, st));
     {
         // the sort's spare value buffer holds the inverse permutation

@@ -3,15 +3,27 @@
 // particle_hash/particle_hash/particle_hash_kernel.cu:32-184 and
 // SpaceHashFunctional.cu:53-145 (keys bit-exact; the reference's Thrust sort is
 // replaced by a stable radix sort: order by (key, original index)).
+#include <algorithm>
+
 #include "pppm_internal.hpp"
 
 namespace pppm {
 
 constexpr int kSortThreads = 256;  // 4 wave64s
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kSortThreads * kSortItems;  // 4096 keys per workgroup
 constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
+// Keys per thread of a sort tile: 16 at large, fewer where tiles of 4096 keys
+// leave compute units idle and a pass is the latency of one tile.  us of a
+// 24-bit sort with 4 / 8 / 16: 64K keys 49 / 52 / 62, 262K 55 / 58 / 67, 700K
+// 67 / 65 / 73, 1M 82 / 73 / 77, 1.5M 96 / 79 / 84, 2M 128 / 95 / 89, 8M 363 /
+// 254 / 213.
+constexpr uint32_t kSort4 = 1u << 19, kSort8 = 3u << 19;
+constexpr int sort_items(uint32_t n) { return n <= kSort4 ? 4 : n <= kSort8 ? 8 : 16; }
+inline uint32_t sort_tiles(uint32_t n) { return (uint32_t)div_up64(n, kSortThreads * sort_items(n)); }
+// Cells up to which the offsets are searched for, a thread a cell (us of
+// hashing and reordering, scanned / searched: 64K particles in 64^3 104 / 87,
+// 700K in 96^3 143 / 137, 1M in 128^3 164 / 179, 8M in 256^3 967 / 1238).
+constexpr uint32_t kSearchCells = 1u << 20;
 
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_calc_keys(const float4* __restrict__ pos, uint32_t n, uint32_t g, float hf,
@@ -75,54 +87,90 @@ __device__ inline uint32_t block_scan_256(uint32_t v, uint32_t* lw, uint32_t& to
 }
 
 // Per-workgroup digit histogram, stored digit-major: hist[d * nblocks + b].
+// All of a thread's keys are loaded before the first count (a load a round
+// waits for each: 10 us for one tile).
+template <int ITEMS>
 __global__ void __launch_bounds__(kSortThreads) k_radix_upsweep(const uint32_t* __restrict__ keys, uint32_t n,
                                                                 int shift, uint32_t* __restrict__ hist,
                                                                 uint32_t nblocks) {
     __shared__ uint32_t h[kRadix];
+    const uint32_t base = blockIdx.x * (kSortThreads * ITEMS) + threadIdx.x;
+    uint32_t k[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) k[j] = base + j * kSortThreads < n ? keys[base + j * kSortThreads] : 0u;
     h[threadIdx.x] = 0;
     __syncthreads();
-    const uint32_t base = blockIdx.x * kSortTile;
-    for (int j = 0; j < kSortItems; j++) {
-        uint32_t i = base + j * kSortThreads + threadIdx.x;
-        bool valid = i < n;
-        uint32_t d = valid ? (keys[i] >> shift) & (kRadix - 1) : 0u;
-        uint64_t m = match_digit(d, valid);
-        if (valid && (m & lanemask_lt()) == 0) atomicAdd(&h[d], (uint32_t)__popcll(m));
-    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++)
+        if (base + j * kSortThreads < n) atomicAdd(&h[(k[j] >> shift) & (kRadix - 1)], 1u);
     __syncthreads();
     hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
-// Stable scatter of one 4096-key tile: wave w owns items [w*1024, w*1024+1024)
-// of the tile, in 16 rounds of 64 consecutive items, so (wave, round, lane)
-// order is item order.  Ranks come from ballots; the tile is staged in LDS in
+// Exclusive prefix of each digit's tile counts, in place, and the digit's
+// total: workgroup d takes digit d (the downsweep adds the digits below).
+__global__ void __launch_bounds__(256) k_digit_scan(uint32_t* __restrict__ hist, uint32_t nblocks,
+                                                    uint32_t* __restrict__ total) {
+    constexpr int kItems = 8;
+    __shared__ uint32_t lw[4];
+    uint32_t* row = hist + (size_t)blockIdx.x * nblocks;
+    uint32_t run = 0;
+    for (uint32_t b0 = 0; b0 < nblocks; b0 += 256 * kItems) {
+        const uint32_t i0 = b0 + threadIdx.x * kItems;
+        uint32_t v[kItems], s = 0, tot;
+#pragma unroll
+        for (int q = 0; q < kItems; q++) {
+            v[q] = i0 + q < nblocks ? row[i0 + q] : 0u;
+            s += v[q];
+        }
+        uint32_t at = run + block_scan_256(s, lw, tot);
+#pragma unroll
+        for (int q = 0; q < kItems; q++) {
+            if (i0 + q < nblocks) row[i0 + q] = at;
+            at += v[q];
+        }
+        run += tot;
+    }
+    if (threadIdx.x == 0) total[blockIdx.x] = run;
+}
+
+// Stable scatter of one tile: each of the four waves owns a quarter of it, in
+// ITEMS rounds of 64 consecutive items, so (wave, round, lane) order is item
+// order.  Ranks come from ballots; the tile is staged in LDS in
 // digit order and written out coalesced.
+template <int ITEMS>
 __global__ void __launch_bounds__(kSortThreads) k_radix_downsweep(const uint32_t* __restrict__ kin,
                                                                   const uint32_t* __restrict__ vin,
                                                                   uint32_t* __restrict__ kout,
                                                                   uint32_t* __restrict__ vout, uint32_t n, int shift,
                                                                   const uint32_t* __restrict__ hist_scan,
+                                                                  const uint32_t* __restrict__ total,
                                                                   uint32_t nblocks) {
+    constexpr int kTile = kSortThreads * ITEMS;
     __shared__ uint32_t wcnt[4][kRadix];
     __shared__ uint32_t dstart[kRadix];
     __shared__ uint32_t gbase[kRadix];
-    __shared__ uint32_t sk[kSortTile];
-    __shared__ uint32_t sv[kSortTile];
+    __shared__ uint32_t sk[kTile];
+    __shared__ uint32_t sv[kTile];
     __shared__ uint32_t lw[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int d = tid; d < 4 * kRadix; d += kSortThreads) (&wcnt[0][0])[d] = 0;
     __syncthreads();
 
-    const uint32_t base = blockIdx.x * kSortTile;
-    const uint32_t wbase = base + wave * (kSortTile / 4);
-    uint32_t k[kSortItems], v[kSortItems], rank[kSortItems];
+    const uint32_t base = blockIdx.x * kTile;
+    const uint32_t wbase = base + wave * (kTile / 4);
+    uint32_t k[ITEMS], v[ITEMS], rank[ITEMS];
     const uint64_t lt = lanemask_lt();
 #pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
+    for (int r = 0; r < ITEMS; r++) {
         uint32_t i = wbase + r * 64 + lane;
-        bool valid = i < n;
-        k[r] = valid ? kin[i] : 0u;
-        v[r] = valid ? (vin ? vin[i] : i) : 0u;
+        k[r] = i < n ? kin[i] : 0u;
+        v[r] = i < n ? (vin ? vin[i] : i) : 0u;
+    }
+    const uint32_t gb = hist_scan[(size_t)tid * nblocks + blockIdx.x], gt = total[tid];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        bool valid = wbase + r * 64 + lane < n;
         uint32_t d = (k[r] >> shift) & (kRadix - 1);
         uint64_t m = match_digit(d, valid);
         uint32_t below = (uint32_t)__popcll(m & lt);
@@ -141,23 +189,23 @@ __global__ void __launch_bounds__(kSortThreads) k_radix_downsweep(const uint32_t
         wcnt[2][d] = c0 + c1;
         wcnt[3][d] = c0 + c1 + c2;
         dstart[d] = ex;
-        gbase[d] = hist_scan[(size_t)d * nblocks + blockIdx.x];
+        gbase[d] = gb + block_scan_256(gt, lw, tot_all);
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kSortItems; r++) {
+    for (int r = 0; r < ITEMS; r++) {
         uint32_t i = wbase + r * 64 + lane;
         if (i < n) {
             uint32_t d = (k[r] >> shift) & (kRadix - 1);
             uint32_t lp = dstart[d] + wcnt[wave][d] + rank[r];
-            if (lp < (uint32_t)kSortTile) {
+            if (lp < (uint32_t)kTile) {
                 sk[lp] = k[r];
                 sv[lp] = v[r];
             }
         }
     }
     __syncthreads();
-    const uint32_t nvalid = (n - base) < (uint32_t)kSortTile ? (n - base) : (uint32_t)kSortTile;
+    const uint32_t nvalid = (n - base) < (uint32_t)kTile ? (n - base) : (uint32_t)kTile;
     for (uint32_t j = tid; j < nvalid; j += kSortThreads) {
         uint32_t key = sk[j];
         uint32_t d = (key >> shift) & (kRadix - 1);
@@ -171,10 +219,11 @@ __global__ void __launch_bounds__(kSortThreads) k_radix_downsweep(const uint32_t
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// Histograms of the most tiles that any count up to n has (a buffer kept for
+// n serves smaller sorts), and the digits' totals.
 size_t sort_scratch_bytes(uint32_t n) {
-    uint64_t nb = div_up64(n ? n : 1, kSortTile);
-    uint64_t hw = nb * kRadix;
-    return align256(hw * 4) * 2 + align256(scan_scratch_words(hw) * 4);
+    const uint32_t nb = std::max({sort_tiles(n), sort_tiles(std::min(n, kSort4)), sort_tiles(std::min(n, kSort8))});
+    return align256((size_t)std::max(nb, 1u) * kRadix * 4) + kRadix * 4;
 }
 
 uint32_t key_bits_for(uint64_t ncells) {
@@ -189,26 +238,29 @@ pppm_status radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
     *keys_out = keys;
     *vals_out = vals;
     if (n == 0) return PPPM_OK;
-    const uint32_t nb = div_up(n, kSortTile);
-    const uint64_t hw = (uint64_t)nb * kRadix;
-    if (hw > 0xFFFFFFFFull) return PPPM_ERR_INVALID;
-    uint8_t* sp = (uint8_t*)scratch;
-    uint32_t* hist = (uint32_t*)sp;
-    uint32_t* hscan = (uint32_t*)(sp + align256(hw * 4));
-    uint32_t* sscr = (uint32_t*)(sp + 2 * align256(hw * 4));
+    const uint32_t nb = sort_tiles(n);
+    uint32_t* hist = (uint32_t*)scratch;
+    uint32_t* total = (uint32_t*)((uint8_t*)scratch + align256((size_t)nb * kRadix * 4));
     int passes = (int)div_up(key_bits ? key_bits : 1, kRadixBits);
     uint32_t *ks = keys, *kd = keys_alt;
     uint32_t *vbuf = vals, *vd = vals_alt;
     const uint32_t* vread = vals_identity ? nullptr : vals;  // null: value = item index
+    auto pass = [&](auto up, auto down, int shift) {
+        const dim3 grid(nb), blk(kSortThreads);
+        hipLaunchKernelGGL(up, grid, blk, 0, st, ks, n, shift, hist, nb);
+        PPPM_LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_digit_scan, dim3(kRadix), dim3(256), 0, st, hist, nb, total);
+        PPPM_LAUNCH_CHECK();
+        hipLaunchKernelGGL(down, grid, blk, 0, st, ks, vread, kd, vd, n, shift, hist, total, nb);
+        PPPM_LAUNCH_CHECK();
+        return PPPM_OK;
+    };
     for (int p = 0; p < passes; p++) {
-        int shift = p * kRadixBits;
-        hipLaunchKernelGGL(k_radix_upsweep, dim3(nb), dim3(kSortThreads), 0, st, ks, n, shift, hist, nb);
-        PPPM_LAUNCH_CHECK();
-        pppm_status s = exclusive_scan_u32(hist, (uint32_t)hw, hscan, sscr, st);
+        const int shift = p * kRadixBits;
+        pppm_status s = sort_items(n) == 4   ? pass(k_radix_upsweep<4>, k_radix_downsweep<4>, shift)
+                        : sort_items(n) == 8 ? pass(k_radix_upsweep<8>, k_radix_downsweep<8>, shift)
+                                             : pass(k_radix_upsweep<16>, k_radix_downsweep<16>, shift);
         if (s != PPPM_OK) return s;
-        hipLaunchKernelGGL(k_radix_downsweep, dim3(nb), dim3(kSortThreads), 0, st, ks, vread, kd, vd, n, shift,
-                           hscan, nb);
-        PPPM_LAUNCH_CHECK();
         uint32_t* t = ks;
         ks = kd;
         kd = t;
@@ -254,17 +306,53 @@ pppm_status launch_fill_u32(uint32_t* a, uint64_t n, uint32_t v, hipStream_t st)
     return PPPM_OK;
 }
 
+// start, end and the offsets of every cell from the sorted keys: cell c's
+// first key by bisection.  A chain of log2(n) loads that neighbouring cells
+// mostly share, in one launch in place of two fills, k_cell_bounds and the
+// three of the scan.
+__global__ void __launch_bounds__(256) k_cell_search(const uint32_t* __restrict__ ks, uint32_t n, uint32_t ncells,
+                                                     uint32_t* __restrict__ start, uint32_t* __restrict__ end,
+                                                     uint32_t* __restrict__ off, uint32_t shift) {
+    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+    // first key of a cell at or after `cell`, at or after lo
+    auto first = [&](uint32_t cell, uint32_t lo) {
+        uint32_t hi = n;
+        while (lo < hi) {
+            const uint32_t mid = lo + (hi - lo) / 2;
+            if (ks[mid] >> shift < cell) lo = mid + 1;
+            else hi = mid;
+        }
+        return lo;
+    };
+    const uint32_t f = first(min(c, ncells), 0);
+    // the next cell's: the next lane's, or for the last lane its own search
+    uint32_t next = __shfl_down(f, 1);
+    if ((threadIdx.x & 63) == 63) next = first(min(c + 1, ncells), f);
+    if (c <= ncells) off[c] = f;
+    if (c < ncells) {
+        start[c] = next > f ? f : kEmptyCell;
+        end[c] = next > f ? next : kEmptyCell;
+    }
+}
+
 pppm_status launch_cell_tables(const uint32_t* keys_sorted, uint32_t n, uint32_t ncells, uint32_t* start,
-                               uint32_t* end, hipStream_t st, uint32_t shift) {
+                               uint32_t* end, hipStream_t st, uint32_t shift, uint32_t* off, uint32_t* scan_scratch) {
+    if (off && ncells <= kSearchCells) {
+        hipLaunchKernelGGL(k_cell_search, dim3(div_up(ncells + 1, 256)), dim3(256), 0, st, keys_sorted, n, ncells,
+                           start, end, off, shift);
+        PPPM_LAUNCH_CHECK();
+        return PPPM_OK;
+    }
     pppm_status s = launch_fill_u32(start, ncells, kEmptyCell, st);
     if (s != PPPM_OK) return s;
     s = launch_fill_u32(end, ncells, kEmptyCell, st);
     if (s != PPPM_OK) return s;
-    if (n == 0) return PPPM_OK;
-    hipLaunchKernelGGL(k_cell_bounds, dim3(div_up(n, 256)), dim3(256), 0, st, keys_sorted, n, ncells, start, end,
-                       shift);
-    PPPM_LAUNCH_CHECK();
-    return PPPM_OK;
+    if (n > 0) {
+        hipLaunchKernelGGL(k_cell_bounds, dim3(div_up(n, 256)), dim3(256), 0, st, keys_sorted, n, ncells, start, end,
+                           shift);
+        PPPM_LAUNCH_CHECK();
+    }
+    return off ? cell_offsets_from_tables(start, end, ncells, off, scan_scratch, st) : PPPM_OK;
 }
 
 // ---------------------------------------------------------------------------

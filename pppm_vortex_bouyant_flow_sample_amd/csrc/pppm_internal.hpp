@@ -40,9 +40,11 @@ pppm_status radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt,
                              uint32_t key_bits, bool vals_identity, void* scratch, uint32_t** keys_out,
                              uint32_t** vals_out, hipStream_t st);
 pppm_status launch_fill_u32(uint32_t* a, uint64_t n, uint32_t v, hipStream_t st);
-// cell = key >> shift (3 for octant keys)
+// cell = key >> shift (3 for octant keys); off (null: not wanted): the cells'
+// first keys, ncells + 1, with scan_scratch of scan_scratch_words(ncells)
 pppm_status launch_cell_tables(const uint32_t* keys_sorted, uint32_t n, uint32_t ncells, uint32_t* start,
-                               uint32_t* end, hipStream_t st, uint32_t shift = 0);
+                               uint32_t* end, hipStream_t st, uint32_t shift = 0, uint32_t* off = nullptr,
+                               uint32_t* scan_scratch = nullptr);
 pppm_status launch_gather(const uint32_t* idx, const void* in, void* out, uint32_t stride, int dtype, uint32_t n,
                           hipStream_t st);
 pppm_status launch_scatter(const uint32_t* idx, const void* in, void* out, uint32_t stride, int dtype, uint32_t n,
