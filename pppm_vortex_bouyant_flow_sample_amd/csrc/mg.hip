@@ -78,24 +78,26 @@ __global__ void __launch_bounds__(256) k_rbgs(T* __restrict__ x, const T* __rest
 constexpr int kTbTX = 64;
 constexpr int kTbTY = 16;
 
-struct TbArgs {
-    const float* xin;    // level array before the pass (read only)
-    float* x;            // level array after the pass (a different buffer)
-    const float* b;      // right-hand side (times bscale)
-    float bscale;
+template <typename T>
+struct TbArgsT {
+    const T* xin;    // level array before the pass (read only)
+    T* x;            // level array after the pass (a different buffer)
+    const T* b;      // right-hand side (times bscale)
+    T bscale;
     int nx, ny, nz;
     size_t G;            // cells per component
-    float omega, beta;   // SOR factor, ghost factor of this level
+    T omega, beta;   // SOR factor, ghost factor of this level
     int zc;              // z planes per workgroup chunk (even)
     // RESTRICT: residual restricted into bn (coarse dims cx, cy, cz = n / 2)
-    float* bn;
+    T* bn;
     int cx, cy, cz;
     size_t Gc;
     // PROLONG: x += trilinear(xc) on load (coarse dims cx, cy, cz, fine dims
     // even), ghost betac
-    const float* xc;
-    float betac;
+    const T* xc;
+    T betac;
 };
+using TbArgs = TbArgsT<float>;
 
 // Trilinear prolongation (k_prolong's weights) at fine cell (i, j, k) from a
 // coarse window held in LDS: cw[slot(c)][cy - cy0][cx - cx0] for coarse planes
@@ -721,13 +723,65 @@ k_rbc(TbArgs a) {
 // 96^3 x 3: 39 -> 18, 41 -> 22.
 constexpr int kR4Region = 64;
 
-template <bool RESTRICT, bool PROLONG, bool XZERO, bool BETA>
-__global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
+// 1024 threads take a region of 64 x 64 floats; of doubles 512 threads one of
+// 64 x 32, whose planes in flight need the registers of two waves per SIMD.
+template <typename T>
+constexpr int r4_threads() { return sizeof(T) == 4 ? 1024 : 512; }
+
+__device__ inline float r4_fma(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ inline double r4_fma(double a, double b, double c) { return fma(a, b, c); }
+
+// value of the lane that DPP control C selects (0x130: lane + 1, 0x138: lane - 1)
+template <int C>
+__device__ inline float lane_shift(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), C, 0xf, 0xf, false));
+}
+template <int C>
+__device__ inline double lane_shift(double v) {
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), C, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(v), C, 0xf, 0xf, false));
+}
+
+// A cell pair through a buffer: one 8- or 16-byte access.
+template <typename T>
+struct R4Pair;
+template <>
+struct R4Pair<float> {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    u32x2 v = {0u, 0u};
+    R4Pair() = default;
+    __device__ R4Pair(float a, float b) : v{__float_as_uint(a), __float_as_uint(b)} {}
+    template <typename R>
+    __device__ void load(R r, uint32_t off) { v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0); }
+    template <typename R>
+    __device__ void store(R r, uint32_t off) const { __builtin_amdgcn_raw_buffer_store_b64(v, r, off, 0, 0); }
+    __device__ float first() const { return __uint_as_float(v[0]); }
+    __device__ float second() const { return __uint_as_float(v[1]); }
+};
+template <>
+struct R4Pair<double> {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 v = {0u, 0u, 0u, 0u};
+    R4Pair() = default;
+    __device__ R4Pair(double a, double b)
+        : v{(uint32_t)__double2loint(a), (uint32_t)__double2hiint(a), (uint32_t)__double2loint(b),
+            (uint32_t)__double2hiint(b)} {}
+    template <typename R>
+    __device__ void load(R r, uint32_t off) { v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0); }
+    template <typename R>
+    __device__ void store(R r, uint32_t off) const { __builtin_amdgcn_raw_buffer_store_b128(v, r, off, 0, 0); }
+    __device__ double first() const { return __hiloint2double((int)v[1], (int)v[0]); }
+    __device__ double second() const { return __hiloint2double((int)v[3], (int)v[2]); }
+};
+
+template <typename T, bool RESTRICT, bool PROLONG, bool XZERO, bool BETA>
+__global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
+    constexpr int NT = r4_threads<T>(), RG = NT / 32;  // row groups of the region
     constexpr bool kWide = RESTRICT && !XZERO;
     constexpr int HXY = kWide ? 6 : 4, HZ = kWide ? 5 : 4;
-    constexpr int TW = kR4Region - 2 * HXY;  // tile
+    constexpr int TW = kR4Region - 2 * HXY, TH = 2 * RG - 2 * HXY;  // tile
     constexpr int NR = RESTRICT ? 8 : 6;     // planes in flight
-    constexpr int ES = 34 * 32;              // row groups -1 .. 32 of one row parity
+    constexpr int ES = (RG + 2) * 32;        // row groups -1 .. RG of one row parity
     // exchanged rows: state t of plane k - t, stored in step j, goes to slot
     // xslot(t, j); states 0 .. 3 are read one step later (two buffers), the
     // residual also reads state 4 one step and state 3 two steps later (four)
@@ -735,74 +789,74 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
     auto xslot = [](int t, int j) {
         return t < 3 ? 2 * t + (j & 1) : t == 3 ? 6 + (j & (RESTRICT ? 3 : 1)) : 10 + (j & 1);
     };
-    constexpr int CW = 34;  // coarse window of the prolongation
-    __shared__ float ex[NE][2][ES];
-    __shared__ float cw[PROLONG ? 3 : 1][PROLONG ? CW * CW : 1];
+    constexpr int CW = 34, CN = CW * (RG + 2);  // coarse window of the prolongation
+    __shared__ T ex[NE][2][ES];
+    __shared__ T cw[PROLONG ? 3 : 1][PROLONG ? CN : 1];
     const int nx = a.nx, ny = a.ny, nz = a.nz;
     const uint32_t tile = xcd_block(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z),
                                     gridDim.x * gridDim.y * gridDim.z);
     const int bx = (int)(tile % gridDim.x), by = (int)((tile / gridDim.x) % gridDim.y);
     const int bz = (int)(tile / (gridDim.x * gridDim.y));
-    const int gx0 = bx * TW - HXY, gy0 = by * TW - HXY;
+    const int gx0 = bx * TW - HXY, gy0 = by * TH - HXY;
     const int nzc = (nz + a.zc - 1) / a.zc;
     const int comp = bz / nzc, zi = bz - comp * nzc;
     const int z0 = zi * a.zc, z1 = min(z0 + a.zc, nz);
-    const float* xsrc = XZERO ? nullptr : a.xin + (size_t)comp * a.G;
-    float* xdst = a.x + (size_t)comp * a.G;
-    const float* bcp = a.b + (size_t)comp * a.G;
-    const float* xcoarse = PROLONG ? a.xc + (size_t)comp * a.Gc : nullptr;
-    float* bnext = RESTRICT ? a.bn + (size_t)comp * a.Gc : nullptr;
+    const T* xsrc = XZERO ? nullptr : a.xin + (size_t)comp * a.G;
+    T* xdst = a.x + (size_t)comp * a.G;
+    const T* bcp = a.b + (size_t)comp * a.G;
+    const T* xcoarse = PROLONG ? a.xc + (size_t)comp * a.Gc : nullptr;
+    T* bnext = RESTRICT ? a.bn + (size_t)comp * a.Gc : nullptr;
     const int klo = max(z0 - HZ, 0), khi = min(z1 + HZ, nz);
     const int kend = z1 + 4 + (RESTRICT ? 1 : 0);
     const int kbeg = klo & ~1;  // ring slots and plane parities by the step count
     const size_t plane = (size_t)nx * ny;
-    const float omega = a.omega, beta = a.beta, bscale = a.bscale;
+    const T omega = a.omega, beta = a.beta, bscale = a.bscale;
     const int tid = threadIdx.x, m = tid & 31, rg = tid >> 5;
     const int i0 = gx0 + 2 * m;
     const bool xin = i0 >= 0 && i0 < nx;
-    for (int q = tid; q < NE * 2 * ES; q += 1024) (&ex[0][0][0])[q] = 0.f;
+    for (int q = tid; q < NE * 2 * ES; q += NT) (&ex[0][0][0])[q] = (T)0;
 
     // Planes are read and written as buffers of plane bytes (0 bytes: none),
     // so that loads off the grid give zero and stores outside the tile are
     // dropped without a branch: a step is straight-line code, and its loads
     // are waited for a whole step later.
     constexpr uint32_t kOff = 0x80000000u;  // beyond any plane
-    const uint32_t pbytes = (uint32_t)(plane * sizeof(float));
+    const uint32_t pbytes = (uint32_t)(plane * sizeof(T));
     uint32_t lofs[2], sofs[2];
     bool gin[2];
-    float wr[2];
+    T wr[2];
     // cells outside the grid next to a cell in the plane, and the diagonal's
     // reciprocal off and on the first and last plane
-    float nxy[2][2], d0[2][2], d1[2][2];
+    T nxy[2][2], d0[2][2], d1[2][2];
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         const int j = gy0 + 2 * rg + r, ly = 2 * rg + r;
         gin[r] = xin && j >= 0 && j < ny;
-        lofs[r] = gin[r] ? 4u * (uint32_t)(j * nx + i0) : kOff;
-        wr[r] = gin[r] ? omega : 0.f;
-        sofs[r] = ly >= HXY && ly < HXY + TW && 2 * m >= HXY && 2 * m < HXY + TW ? lofs[r] : kOff;
+        lofs[r] = gin[r] ? (uint32_t)sizeof(T) * (uint32_t)(j * nx + i0) : kOff;
+        wr[r] = gin[r] ? omega : (T)0;
+        sofs[r] = ly >= HXY && ly < HXY + TH && 2 * m >= HXY && 2 * m < HXY + TW ? lofs[r] : kOff;
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int i = i0 + e;
-            nxy[r][e] = (float)((i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1));
-            d0[r][e] = 1.0f / (6.0f - beta * nxy[r][e]);
-            d1[r][e] = 1.0f / (6.0f - beta * (nxy[r][e] + (nz == 1 ? 2.f : 1.f)));
+            nxy[r][e] = (T)((i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1));
+            d0[r][e] = (T)1.0 / ((T)6.0 - beta * nxy[r][e]);
+            d1[r][e] = (T)1.0 / ((T)6.0 - beta * (nxy[r][e] + (nz == 1 ? (T)2 : (T)1)));
         }
     }
     const int gI = i0 >> 1, gJ = (gy0 >> 1) + rg;
-    const uint32_t cofs = RESTRICT && sofs[0] != kOff && gI < a.cx && gJ < a.cy ? 4u * (uint32_t)(gJ * a.cx + gI) : kOff;
+    const uint32_t cofs = RESTRICT && sofs[0] != kOff && gI < a.cx && gJ < a.cy ? (uint32_t)sizeof(T) * (uint32_t)(gJ * a.cx + gI) : kOff;
     auto buffer = [](const void* p, uint32_t bytes) {
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
     };
 
     // [slot][row][pair cell]
-    float X[NR][2][2], B[NR][2][2];
-    uint2 px[2], pb[2];
-    float pc[2], pf = 0.f, rsum[2] = {0.f, 0.f};
+    T X[NR][2][2], B[NR][2][2];
+    R4Pair<T> px[2], pb[2];
+    T pc[2], pf = (T)0, rsum[2] = {(T)0, (T)0};
 #pragma unroll
     for (int q = 0; q < NR; q++)
 #pragma unroll
-        for (int r = 0; r < 2; r++) X[q][r][0] = X[q][r][1] = B[q][r][0] = B[q][r][1] = 0.f;
+        for (int r = 0; r < 2; r++) X[q][r][0] = X[q][r][1] = B[q][r][0] = B[q][r][1] = (T)0;
     auto fetch = [&](int k) {
         k = __builtin_amdgcn_readfirstlane(k);
         const bool real = k >= klo && k < khi;
@@ -810,40 +864,38 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
         const auto rb = buffer(bcp + ko, real ? pbytes : 0u);
 #pragma unroll
         for (int r = 0; r < 2; r++) {
-            px[r] = make_uint2(0u, 0u);
+            px[r] = R4Pair<T>{};
             if (!XZERO) {
                 const auto rx = buffer(xsrc + ko, real ? pbytes : 0u);
-                const auto v = __builtin_amdgcn_raw_buffer_load_b64(rx, lofs[r], 0, 0);
-                px[r] = make_uint2(v[0], v[1]);
+                px[r].load(rx, lofs[r]);
             }
-            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rb, lofs[r], 0, 0);
-            pb[r] = make_uint2(v[0], v[1]);
+            pb[r].load(rb, lofs[r]);
         }
     };
     // the coarse window, ghost-extended as k_rbc's; plane c in slot (c + 3) % 3.
     // A thread's two cells (the last of them beyond the window: not stored)
     const int cx0 = (gx0 >> 1) - 1, cy0 = (gy0 >> 1) - 1;
     uint32_t cq[2];  // byte offsets
-    float cf[2];
+    T cf[2];
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-        const int q = min(tid + 1024 * u, CW * CW - 1);
+        const int q = min(tid + NT * u, CN - 1);
         const int ci = cx0 + q % CW, cj = cy0 + q / CW;
         const int cic = PROLONG ? min(max(ci, 0), a.cx - 1) : 0, cjc = PROLONG ? min(max(cj, 0), a.cy - 1) : 0;
-        cq[u] = 4u * (uint32_t)(cjc * a.cx + cic);
-        cf[u] = (cic != ci ? a.betac : 1.f) * (cjc != cj ? a.betac : 1.f);
+        cq[u] = (uint32_t)sizeof(T) * (uint32_t)(cjc * a.cx + cic);
+        cf[u] = (cic != ci ? a.betac : (T)1) * (cjc != cj ? a.betac : (T)1);
     }
     auto fetch_coarse = [&](int c) {
         const int cc = min(max(c, 0), a.cz - 1);
-        pf = cc != c ? a.betac : 1.f;
+        pf = cc != c ? a.betac : (T)1;
         const char* p = reinterpret_cast<const char*>(xcoarse + (size_t)__builtin_amdgcn_readfirstlane(cc) * a.cy * a.cx);
-        pc[0] = *reinterpret_cast<const float*>(p + cq[0]);
-        pc[1] = *reinterpret_cast<const float*>(p + cq[1]);
+        pc[0] = *reinterpret_cast<const T*>(p + cq[0]);
+        pc[1] = *reinterpret_cast<const T*>(p + cq[1]);
     };
     auto store_coarse = [&](int c) {
-        float* w = cw[(c + 3) % 3];
+        T* w = cw[(c + 3) % 3];
         w[tid] = pc[0] * (cf[0] * pf);
-        if (tid + 1024 < CW * CW) w[tid + 1024] = pc[1] * (cf[1] * pf);
+        if (tid + NT < CN) w[tid + NT] = pc[1] * (cf[1] * pf);
     };
     if (PROLONG) {
         // (klo is even: the first step stores plane klo / 2 + 1)
@@ -858,12 +910,8 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
 
     // the neighbouring pair's cell: lane - 1's (m > 0) or lane + 1's; the
     // region's edge lanes read a row that is not theirs, inside the halo
-    auto from_left = [](float v) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, false));
-    };
-    auto from_right = [](float v) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, false));
-    };
+    auto from_left = [](T v) { return lane_shift<0x138>(v); };
+    auto from_right = [](T v) { return lane_shift<0x130>(v); };
     const int lo = rg * 32 + m;  // row group rg - 1 in an exchanged row; rg + 1 at lo + 64
 
     for (int k0 = kbeg;; k0 += NR) {
@@ -873,7 +921,7 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
             if (k >= kend) return;
             // ---- the exchanged rows of this step (with the coarse window's
             // cells in registers too, spills: the prolongation goes first)
-            float y[4][2];
+            T y[4][2];
             auto exchanged = [&]() {
 #pragma unroll
                 for (int t = XZERO ? 2 : 1; t <= 4; t++) {
@@ -883,7 +931,7 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
             };
             // of the residual: [row][colour]; colour 1 was last written by
             // half-sweep 3, colour 0 by 4
-            float yr[2][2];
+            T yr[2][2];
             if (RESTRICT) {
                 yr[0][0] = ex[xslot(3, j + 2)][1][lo];
                 yr[1][0] = ex[xslot(3, j + 2)][0][lo + 64];
@@ -893,33 +941,32 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
             if (!PROLONG) exchanged();
             // ---- state 0 of plane k (zero from khi on)
             {
-                float v[2][2] = {{__uint_as_float(px[0].x), __uint_as_float(px[0].y)},
-                                 {__uint_as_float(px[1].x), __uint_as_float(px[1].y)}};
+                T v[2][2] = {{px[0].first(), px[0].second()}, {px[1].first(), px[1].second()}};
                 if (PROLONG) {
                     // trilinear: parent column m + 1 of the window, neighbour m
                     // (first cell) or m + 2; parent row rg + 1, neighbour rg
                     // (first row) or rg + 2; parent plane k >> 1, neighbour one
                     // up (k odd) or down
                     const int pk = k >> 1, nk = pk + ((j & 1) ? 1 : -1);
-                    float w[2][2][2];
+                    T w[2][2][2];
                     // opaque: the slots repeat with the unrolled steps, and their
                     // addresses would all be kept in registers (spills)
                     int c00 = rg * CW + m;
                     __asm__ volatile("" : "+v"(c00));
 #pragma unroll
                     for (int z = 0; z < 2; z++) {
-                        const float* c0 = &cw[((z ? nk : pk) + 3) % 3][c00];
-                        float xe[3], xo[3];
+                        const T* c0 = &cw[((z ? nk : pk) + 3) % 3][c00];
+                        T xe[3], xo[3];
 #pragma unroll
                         for (int q = 0; q < 3; q++) {
-                            const float* c = c0 + q * CW;
-                            xe[q] = 0.75f * c[1] + 0.25f * c[0];
-                            xo[q] = 0.75f * c[1] + 0.25f * c[2];
+                            const T* c = c0 + q * CW;
+                            xe[q] = (T)0.75 * c[1] + (T)0.25 * c[0];
+                            xo[q] = (T)0.75 * c[1] + (T)0.25 * c[2];
                         }
 #pragma unroll
                         for (int r = 0; r < 2; r++) {
-                            w[z][r][0] = 0.75f * xe[1] + 0.25f * xe[2 * r];
-                            w[z][r][1] = 0.75f * xo[1] + 0.25f * xo[2 * r];
+                            w[z][r][0] = (T)0.75 * xe[1] + (T)0.25 * xe[2 * r];
+                            w[z][r][1] = (T)0.75 * xo[1] + (T)0.25 * xo[2 * r];
                         }
                     }
                     const bool real = k < khi;
@@ -927,7 +974,7 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
                     for (int r = 0; r < 2; r++)
 #pragma unroll
                         for (int e = 0; e < 2; e++) {
-                            const float f = v[r][e] + (0.75f * w[0][r][e] + 0.25f * w[1][r][e]);
+                            const T f = v[r][e] + ((T)0.75 * w[0][r][e] + (T)0.25 * w[1][r][e]);
                             v[r][e] = gin[r] && real ? f : v[r][e];
                         }
                 }
@@ -935,8 +982,8 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
                 for (int r = 0; r < 2; r++) {
                     X[j][r][0] = v[r][0];
                     X[j][r][1] = v[r][1];
-                    B[j][r][0] = __uint_as_float(pb[r].x);
-                    B[j][r][1] = __uint_as_float(pb[r].y);
+                    B[j][r][0] = pb[r].first();
+                    B[j][r][1] = pb[r].second();
                     // half-sweep 1 updates colour 1 and reads colour 0
                     if (!XZERO) ex[xslot(0, j)][r][lo + 32] = X[j][r][(r ^ j) & 1];
                 }
@@ -959,16 +1006,16 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
 #pragma unroll
                 for (int r = 0; r < 2; r++) {
                     const int e = (c ^ r ^ jp) & 1;
-                    float s = 0.f;
+                    T s = (T)0;
                     if (!(XZERO && t == 1)) {
-                        const float other = X[jp][r][1 - e];
+                        const T other = X[jp][r][1 - e];
                         s = e ? other + from_right(X[jp][r][0]) : from_left(X[jp][r][1]) + other;
                         s += r ? X[jp][0][e] + y[t - 1][1] : y[t - 1][0] + X[jp][1][e];
                         s += X[jm][r][e] + X[jq][r][e];
                     }
-                    s = fmaf(-bscale, B[jp][r][e], s);
-                    const float d = BETA ? (zb ? d1[r][e] : d0[r][e]) : 1.0f / 6.0f, xo = X[jp][r][e];
-                    const float xn = xo + (in ? wr[r] : 0.f) * (s * d - xo);
+                    s = r4_fma(-bscale, B[jp][r][e], s);
+                    const T d = BETA ? (zb ? d1[r][e] : d0[r][e]) : (T)1.0 / (T)6.0, xo = X[jp][r][e];
+                    const T xn = xo + (in ? wr[r] : (T)0) * (s * d - xo);
                     X[jp][r][e] = xn;
                     if (t < 4 || RESTRICT) ex[xslot(t, j)][r][lo + 32] = xn;
                 }
@@ -978,32 +1025,28 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
                 const int jw = (j + NR - 4) % NR, pw = __builtin_amdgcn_readfirstlane(k - 4);
                 const bool mine = pw >= z0 && pw < z1;
                 const auto rd = buffer(xdst + (mine ? (size_t)pw * plane : 0), mine ? pbytes : 0u);
-                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    const u32x2 v = {__float_as_uint(X[jw][r][0]), __float_as_uint(X[jw][r][1])};
-                    __builtin_amdgcn_raw_buffer_store_b64(v, rd, sofs[r], 0, 0);
-                }
+                for (int r = 0; r < 2; r++) R4Pair<T>(X[jw][r][0], X[jw][r][1]).store(rd, sofs[r]);
             }
             // ---- residual of plane k - 5 and its restriction: this thread's
             // 2 x 2 cells of a plane pair are one coarse cell
             if (RESTRICT) {
                 const int jr = (j + NR - 5) % NR, jm = (jr + NR - 1) % NR, jq = (jr + 1) % NR, pr = k - 5;
-                const float zb = (float)((pr == 0) + (pr == nz - 1));
-                float part[2];
+                const T zb = (T)((pr == 0) + (pr == nz - 1));
+                T part[2];
 #pragma unroll
                 for (int r = 0; r < 2; r++) {
-                    part[r] = 0.f;
+                    part[r] = (T)0;
 #pragma unroll
                     for (int c = 0; c < 2; c++) {
                         const int e = (c ^ r ^ jr) & 1;
-                        const float xo = X[jr][r][e], other = X[jr][r][1 - e];
-                        float s = e ? other + from_right(X[jr][r][0]) : from_left(X[jr][r][1]) + other;
+                        const T xo = X[jr][r][e], other = X[jr][r][1 - e];
+                        T s = e ? other + from_right(X[jr][r][0]) : from_left(X[jr][r][1]) + other;
                         s += r ? X[jr][0][e] + yr[1][c] : yr[0][c] + X[jr][1][e];
                         s += X[jm][r][e] + X[jq][r][e];
-                        s -= 6.0f * xo;
+                        s -= (T)6.0 * xo;
                         if (BETA) s += beta * (nxy[r][e] + zb) * xo;
-                        part[r] += fmaf(bscale, B[jr][r][e], -s);
+                        part[r] += r4_fma(bscale, B[jr][r][e], -s);
                     }
                 }
                 if ((jr & 1) == 0) {
@@ -1013,9 +1056,10 @@ __global__ void __launch_bounds__(1024) k_rb4(TbArgs a) {
                     const int gK = __builtin_amdgcn_readfirstlane(pr >> 1);
                     const bool mine = pr >= z0 && pr < z1 && gK < a.cz;
                     const auto rn = buffer(bnext + (mine ? (size_t)gK * a.cy * a.cx : 0),
-                                           mine ? 4u * (uint32_t)(a.cy * a.cx) : 0u);
-                    __builtin_amdgcn_raw_buffer_store_b32(
-                        __float_as_uint(((rsum[0] + part[0]) + (rsum[1] + part[1])) * 0.5f), rn, cofs, 0, 0);
+                                           mine ? (uint32_t)sizeof(T) * (uint32_t)(a.cy * a.cx) : 0u);
+                    const T c = ((rsum[0] + part[0]) + (rsum[1] + part[1])) * (T)0.5;
+                    static_assert(!RESTRICT || sizeof(T) == 4, "the restriction stores floats");
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)c), rn, cofs, 0, 0);
                 }
             }
             __syncthreads();
@@ -2112,10 +2156,10 @@ static void launch_rbc(TbArgs a, int ncomp, hipStream_t st) {
 // k_rb4 over all components, one workgroup a CU at a time: the number of z
 // chunks that needs the fewest steps, rounds of workgroups times a chunk's
 // planes with its halo.
-template <bool R, bool P, bool Z, bool B>
-static void launch_rb4(TbArgs a, int ncomp, hipStream_t st) {
-    constexpr int tw = kR4Region - (R && !Z ? 12 : 8), halo = (R && !Z ? 10 : 8) + 4;
-    const int tx = (a.nx + tw - 1) / tw, ty = (a.ny + tw - 1) / tw;
+template <typename T, bool R, bool P, bool Z, bool B>
+static void launch_rb4(TbArgsT<T> a, int ncomp, hipStream_t st) {
+    constexpr int rim = R && !Z ? 12 : 8, tw = kR4Region - rim, th = r4_threads<T>() / 16 - rim, halo = (R && !Z ? 10 : 8) + 4;
+    const int tx = (a.nx + tw - 1) / tw, ty = (a.ny + th - 1) / th;
     const int64_t tiles = (int64_t)tx * ty * ncomp, cus = cu_count();
     int64_t best = INT64_MAX;
     for (int c = 1; c <= 64; c++) {
@@ -2128,7 +2172,7 @@ static void launch_rb4(TbArgs a, int ncomp, hipStream_t st) {
         }
     }
     dim3 grid(tx, ty, (a.nz + a.zc - 1) / a.zc * ncomp);
-    hipLaunchKernelGGL((k_rb4<R, P, Z, B>), grid, dim3(1024), 0, st, a);
+    hipLaunchKernelGGL((k_rb4<T, R, P, Z, B>), grid, dim3(r4_threads<T>()), 0, st, a);
 }
 
 // One blocked pass over all components: kind 1 = k_rb2, 2 = k_rbc with a
@@ -2144,8 +2188,8 @@ static pppm_status launch_rb2(const TbArgs& a, int ncomp, int kind, hipStream_t 
     const bool beta = a.beta != 0.f;
     if (two_iter && (kind < 4 || (a.nx & 1) != 0)) return PPPM_ERR_INVALID;
     if (two_iter) {
-        if (beta) launch_rb4<R, P, Z, true>(a, ncomp, st);
-        else launch_rb4<R, P, Z, false>(a, ncomp, st);
+        if (beta) launch_rb4<float, R, P, Z, true>(a, ncomp, st);
+        else launch_rb4<float, R, P, Z, false>(a, ncomp, st);
     } else if (kind >= 2 && (a.nx & 1) == 0) {
         if (R || kind == 3) {
             if (beta) launch_rbc<R, P, Z, true, 6>(a, ncomp, st);
@@ -2220,13 +2264,32 @@ pppm_status MGHier<T>::smooth(int l, T* x, const T* b, T bscale, int iters, T om
         if (q & 1) return copy(x, tmp, cells(l) * ncomp_, st);
         return PPPM_OK;
     }
-    dim3 blk(64, 4), grid(div_up(div_up(nx, 2), 64), div_up(ny, 4), nz * ncomp_);
-    for (int it = 0; it < iters; it++)
-        for (int color = 1; color >= 0; color--) {
-            hipLaunchKernelGGL(k_rbgs<T>, grid, blk, 0, st, x, b, bscale, nx, ny, nz, cells(l), color, omega, beta);
-            PPPM_LAUNCH_CHECK();
-        }
-    return PPPM_OK;
+    T* cur = x;
+    if constexpr (std::is_same<T, double>::value) {
+        // large levels: two iterations a pass while two remain, x -> t -> x
+        if (tb_ && cells(l) >= kTileCells && t_[l] && !(nx & 1))
+            for (; iters >= 2; iters -= 2) {
+                T* dst = cur == x ? t_[l] : x;
+                TbArgsT<T> a{};
+                a.xin = cur;
+                a.x = dst;
+                a.b = b;
+                a.bscale = bscale;
+                a.nx = nx;
+                a.ny = ny;
+                a.nz = nz;
+                a.G = cells(l);
+                a.omega = omega;
+                a.beta = beta;
+                if (beta != 0) launch_rb4<T, false, false, false, true>(a, ncomp_, st);
+                else launch_rb4<T, false, false, false, false>(a, ncomp_, st);
+                PPPM_LAUNCH_CHECK();
+                cur = dst;
+            }
+    }
+    pppm_status s = smooth_colour(l, cur, b, bscale, iters, omega, beta, st);
+    if (s != PPPM_OK || cur == x) return s;
+    return copy(x, cur, cells(l) * ncomp_, st);
 }
 
 template <typename T>

@@ -53,3 +53,20 @@ def test_vcycles_equal_halfsweeps(native, dims, ncomp, nu):
         out.append(bx.to_array(np.float32, n))
     assert np.all(np.isfinite(out[1]))
     assert rel_l2(out[1], out[0]) < 1e-5
+
+
+@pytest.mark.parametrize("dims,nu", [((96, 80, 72), (4, 4)), ((114, 73, 66), (3, 2)), ((112, 96, 49), (2, 5))])
+def test_full_multigrid_fp64_large_level(native, oracle, dims, nu):
+    """One full-multigrid pass in FP64 whose finest level takes the pass of
+    two iterations (56 x 24 tiles): the oracle's iterate to 1e-10."""
+    n = int(np.prod(dims))
+    b = np.random.default_rng(sum(dims)).standard_normal(n)
+    omega = float(np.float32(1.43))
+    mg = native.MG(dims, native.F64)
+    bx, bb = native.DeviceBuffer(8 * n), native.DeviceBuffer.from_array(b)
+    bx.fill_zero()
+    print(f"[mg two] FMG dims={dims} nu={nu}", flush=True)
+    mg.solve(bx.ptr, bb.ptr, native.MG_REF_FMG, nu[0], nu[1], omega, 0.0, 1)
+    x = bx.to_array(np.float64, n)
+    xo, _, _ = oracle.mg_solve(b, dims, schedule=oracle.MG_REF_FMG, nu1=nu[0], nu2=nu[1], omega=omega)
+    assert rel_l2(x, xo) < 1e-10
