@@ -2267,7 +2267,7 @@ pppm_status MGHier<T>::smooth(int l, T* x, const T* b, T bscale, int iters, T om
     T* cur = x;
     if constexpr (std::is_same<T, double>::value) {
         // large levels: two iterations a pass while two remain, x -> t -> x
-        if (tb_ && cells(l) >= kTileCells && t_[l] && !(nx & 1))
+        if (wide_level(l))
             for (; iters >= 2; iters -= 2) {
                 T* dst = cur == x ? t_[l] : x;
                 TbArgsT<T> a{};
@@ -2364,7 +2364,7 @@ pppm_status MGHier<T>::tail(const T* xin, T* x, const T* b, T* b1, T bscale, int
 template <typename T>
 bool MGHier<T>::tile_level(int l, bool consistent) const {
     if (!tb_ || l >= L_ - 1 || !has_temp(cells(l)) || cells(l) >= kTileCells) return false;
-    if (cells(l) >= tb_min_cells_ && !(d_[l][0] & 1)) return false;  // k_rb4, k_rbc
+    if (sizeof(T) == 8 ? wide_level(l) : cells(l) >= tb_min_cells_ && !(d_[l][0] & 1)) return false;  // k_rb4, k_rbc
     for (int c = 0; c < 3; c++)
         // without the one launch of the smallest levels the one above the
         // coarsest runs a launch per half-sweep, with bitwise its results

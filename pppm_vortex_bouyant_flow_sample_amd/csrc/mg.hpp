@@ -110,6 +110,11 @@ class MGHier {
     // its right-hand side b (times bscale) and the coarsest one's b1 (written)
     pppm_status tail(const T* xin, T* x, const T* b, T* b1, T bscale, int nu1, int nu2, T omega, bool consistent,
                      hipStream_t st);
+    // whether level l takes passes of two iterations over the whole level in
+    // FP64 (k_rb4)
+    bool wide_level(int l) const {
+        return sizeof(T) == 8 && tb_ && cells(l) * (size_t)ncomp_ >= kRb4Doubles && t_[l] && !(d_[l][0] & 1);
+    }
     // whether level l of a V-cycle takes the tile passes (k_tile)
     bool tile_level(int l, bool consistent) const;
     // one tile pass, xin (null: zero) -> x: the prolongation of xc added
@@ -134,11 +139,16 @@ class MGHier {
     // kTile16Cells cells over all components.
     static constexpr size_t kTileCells = (size_t)1 << 19;
     static constexpr size_t kTile16Cells = (size_t)1 << 19;
-    // Blocked passes from here (us down and up, tile against blocked, FP32:
-    // 64^3 10.4 against 13.8 and for three components 16 + 18 against 16 + 19;
-    // 72^3 17 against 14, three 26 against 16; 80^3 23 against 14, three 28 +
-    // 34 against 17 + 19).  Doubles have no blocked passes.
-    size_t tb_min_cells_ = std::is_same<T, float>::value ? (size_t)5 << 16 : kTileCells;
+    // FP32 blocked passes from here (us down and up, tile against blocked: 64^3
+    // 10.4 against 13.8 and for three components 16 + 18 against 16 + 19; 72^3
+    // 17 against 14, three 26 against 16; 80^3 23 against 14, three 28 + 34
+    // against 17 + 19).
+    size_t tb_min_cells_ = (size_t)5 << 16;
+    // FP64 levels of at least this many cells over all components take k_rb4
+    // (us of a full multigrid V(4,4), tiles against k_rb4: 32^3 x 3 183 against
+    // 205, 48^3 289 against 302, 40^3 x 3 336 against 301, 56^3 355 against 325,
+    // 64^3 374 against 338, 64^3 x 3 598 against 388).
+    static constexpr size_t kRb4Doubles = (size_t)1 << 17;
     bool tail_ = true;
 };
 
