@@ -1936,20 +1936,39 @@ std::vector<double> coarse_tables(int nx, int ny, int nz, double beta) {
     return t;
 }
 
-template <typename T>
-size_t MGHier<T>::bytes_for(int nx, int ny, int nz, int ncomp) {
-    size_t b = 0, cells = (size_t)nx * ny * nz;
-    int x = nx, y = ny, z = nz, L = 1;
-    if (has_temp(cells)) b += cells * ncomp * sizeof(T);
-    while ((long)x * y * z > 512 && L < 16) {
+// Halvings of MultiGrid.h:115-127 (m_ComputeLevels): the levels' dimensions,
+// their number returned.
+static int level_dims(int x, int y, int z, int (*d)[3]) {
+    int L = 0;
+    for (;; L++) {
+        d[L][0] = x;
+        d[L][1] = y;
+        d[L][2] = z;
+        if ((long)x * y * z <= 512 || L + 1 >= 16) return L + 1;
         x = x / 2 > 0 ? x / 2 : 1;
         y = y / 2 > 0 ? y / 2 : 1;
         z = z / 2 > 0 ? z / 2 : 1;
-        L++;
-        cells = (size_t)x * y * z;
-        b += 2 * cells * ncomp * sizeof(T);
-        if (has_temp(cells)) b += cells * ncomp * sizeof(T);
     }
+}
+
+template <typename T>
+bool MGHier<T>::has_temp(const int (*d)[3], int L, int l) {
+    if (sizeof(T) == 4) return true;
+    const size_t n = (size_t)d[l][0] * d[l][1] * d[l][2];
+    const bool tail = l == L - 2 && L >= 3 && n <= (size_t)kTailMax && tail_fits(d[l]);
+    return n <= (size_t)1 << 24 && l < L - 1 && !tail;
+}
+
+template <typename T>
+size_t MGHier<T>::bytes_for(int nx, int ny, int nz, int ncomp) {
+    int d[16][3];
+    const int L = level_dims(nx, ny, nz, d);
+    size_t b = 0;
+    for (int l = 0; l < L; l++) {
+        const size_t n = (size_t)d[l][0] * d[l][1] * d[l][2] * ncomp * sizeof(T);
+        b += (l > 0 ? 2 : 0) * n + (has_temp(d, L, l) ? n : 0);
+    }
+    const int x = d[L - 1][0], y = d[L - 1][1], z = d[L - 1][2];
     // coarse tables (two bases, <= 3 * 512^2 doubles each at most) and norm partials
     b += 2 * (size_t)(x * x + y * y + z * z + x + y + z) * sizeof(double);
     b += (size_t)kNormBlocks * ncomp * 2 * sizeof(double) + 2 * (size_t)ncomp * sizeof(double);
@@ -1965,22 +1984,8 @@ pppm_status MGHier<T>::init(int nx, int ny, int nz, int ncomp) {
     if (nx < 1 || ny < 1 || nz < 1 || ncomp < 1 || ncomp > kMaxComp) return PPPM_ERR_INVALID;
     ncomp_ = ncomp;
     cap_ = ncomp;
-    // MultiGrid.h:115-127 (m_ComputeLevels), 93-98
-    L_ = 0;
-    int x = nx, y = ny, z = nz;
-    d_[0][0] = x;
-    d_[0][1] = y;
-    d_[0][2] = z;
-    while ((long)x * y * z > 512 && L_ + 1 < 16) {
-        x = x / 2 > 0 ? x / 2 : 1;
-        y = y / 2 > 0 ? y / 2 : 1;
-        z = z / 2 > 0 ? z / 2 : 1;
-        L_++;
-        d_[L_][0] = x;
-        d_[L_][1] = y;
-        d_[L_][2] = z;
-    }
-    L_ += 1;
+    // MultiGrid.h:93-98
+    L_ = level_dims(nx, ny, nz, d_);
     x_.assign(L_, nullptr);
     b_.assign(L_, nullptr);
     t_.assign(L_, nullptr);
@@ -1989,7 +1994,7 @@ pppm_status MGHier<T>::init(int nx, int ny, int nz, int ncomp) {
         if (std::is_same<T, float>::value) rbc_prime();
         // out-of-place targets of the blocked passes
         for (int l = 0; l < L_; l++) {
-            if (!has_temp(cells(l))) continue;
+            if (!has_temp(d_, L_, l)) continue;
             size_t n = cells(l) * ncomp_;
             if (hipMalloc(&t_[l], n * sizeof(T)) != hipSuccess) {
                 release_locked();
@@ -2363,7 +2368,7 @@ pppm_status MGHier<T>::tail(const T* xin, T* x, const T* b, T* b1, T bscale, int
 
 template <typename T>
 bool MGHier<T>::tile_level(int l, bool consistent) const {
-    if (!tb_ || l >= L_ - 1 || !has_temp(cells(l)) || cells(l) >= kTileCells) return false;
+    if (!tb_ || l >= L_ - 1 || !t_[l] || cells(l) >= kTileCells) return false;
     if (sizeof(T) == 8 ? wide_level(l) : cells(l) >= tb_min_cells_ && !(d_[l][0] & 1)) return false;  // k_rb4, k_rbc
     for (int c = 0; c < 3; c++)
         // without the one launch of the smallest levels the one above the

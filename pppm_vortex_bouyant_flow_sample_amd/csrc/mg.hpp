@@ -76,9 +76,10 @@ class MGHier {
     // out-of-place target of the blocked passes at level l (null where
     // has_temp is false)
     T* temp(int l) { return t_[l]; }
-    // levels with an out-of-place target: every float level (blocked
-    // smoother, tile passes), the double ones up to 256^3 (tile passes, k_rb4)
-    static bool has_temp(size_t cells) { return sizeof(T) == 4 || cells <= (size_t)1 << 24; }
+    // whether level l of L has an out-of-place target: every float level
+    // (blocked smoother, tile passes), the double ones up to 256^3 (tile
+    // passes, k_rb4) but those of the small levels' one launch
+    static bool has_temp(const int (*d)[3], int L, int l);
     double* partials() { return part_; }
     // the reduced norms, 2 per component (||r||^2, ||b||^2), after the partials
     double* norm_out() { return part_ + (size_t)kNormBlocks * ncomp_ * 2; }
