@@ -108,10 +108,10 @@ pppm_status pppm_set_graphs(pppm_ctx *ctx, int32_t on);
  * PPPM_NEAR_ORDER_AUTO (default): the sort's order (the potential-flow near
  * fields: renumbered in super-blocks of 8x4x4 cells when there are at least
  * 4,096 points and a quarter as many as x segments, and the near field's
- * sources and cell tables, 32 B a source and 8 B a cell, exceed 64 MiB).  _SORT: always the sort's
- * order.  _SUPER_BLOCKS: always renumbered.  On grids of more than 2^29
- * cells (sort keys without the octant) the order is the sort's in every
- * mode.  The orders differ in FP32 summation order only. */
+ * sources and cell tables, 32 B a source and 8 B a cell, exceed 64 MiB).
+ * _SORT: always the sort's order.  _SUPER_BLOCKS: always renumbered.  On grids
+ * of more than 2^29 cells (sort keys without the octant) the order is the
+ * sort's in every mode.  The orders differ in FP32 summation order only. */
 #define PPPM_NEAR_ORDER_AUTO 0
 #define PPPM_NEAR_ORDER_SORT 1
 #define PPPM_NEAR_ORDER_SUPER_BLOCKS 2

@@ -1976,6 +1976,7 @@ size_t MGHier<T>::bytes_for(int nx, int ny, int nz, int ncomp) {
 }
 
 static void rbc_prime();
+static int cu_count();
 
 template <typename T>
 pppm_status MGHier<T>::init(int nx, int ny, int nz, int ncomp) {
@@ -1992,6 +1993,7 @@ pppm_status MGHier<T>::init(int nx, int ny, int nz, int ncomp) {
     bytes_ = 0;
     {
         if (std::is_same<T, float>::value) rbc_prime();
+        else (void)cu_count();
         // out-of-place targets of the blocked passes
         for (int l = 0; l < L_; l++) {
             if (!has_temp(d_, L_, l)) continue;
@@ -2213,6 +2215,10 @@ static pppm_status launch_rb2(const TbArgs& a, int ncomp, int kind, hipStream_t 
     return PPPM_OK;
 }
 
+// k_rb4 addresses a plane of floats by 31-bit byte offsets (of doubles: levels
+// of at most 2^24 cells).
+static bool r4_plane(int nx, int ny) { return (size_t)nx * ny * sizeof(float) <= (size_t)1 << 31; }
+
 template <typename T>
 static pppm_status smooth_tb(const T*, T*, const T*, T, int, int, int, int, size_t, T, T, int, bool, hipStream_t) {
     return PPPM_ERR_INVALID;
@@ -2255,7 +2261,7 @@ pppm_status MGHier<T>::smooth(int l, T* x, const T* b, T bscale, int iters, T om
         // out-of-place passes of one iteration (two under kind 4 while two
         // remain), x -> t -> x ...; an odd pass count ends in t, copied back
         T* tmp = t_[l];
-        const bool pairs = tb_ == 4 && !(nx & 1);
+        const bool pairs = tb_ == 4 && !(nx & 1) && r4_plane(nx, ny);
         int q = 0;
         for (int done = 0; done < iters; q++) {
             const bool two = pairs && iters - done >= 2;
@@ -2579,7 +2585,7 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
         float* src = X[l];
         float* dst = m.temp(l);
         // kind 4 runs nu = 2 as one pass of two iterations
-        const bool two1 = kind == 4 && nu1 == 2;
+        const bool two1 = kind == 4 && nu1 == 2 && r4_plane(m.dims(l)[0], m.dims(l)[1]);
         for (int q = 0; q < (two1 ? 1 : nu1); q++) {
             TbArgs a = level_args(l);
             a.xin = src;
@@ -2621,7 +2627,7 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
         }
         float* src = cur[l];
         float* dst = src == X[l] ? m.temp(l) : X[l];
-        const bool two2 = kind == 4 && nu2 == 2;
+        const bool two2 = kind == 4 && nu2 == 2 && r4_plane(m.dims(l)[0], m.dims(l)[1]);
         for (int q = 0; q < (two2 ? 1 : nu2); q++) {
             TbArgs a = level_args(l);
             a.xin = src;
