@@ -320,7 +320,9 @@ extern "C" pppm_status pppm_mg_smooth(pppm_mg* m, void* x, const void* b, int32_
         return s;
     }
     if (blocked) FAIL(PPPM_ERR_INVALID, "the blocked smoother is float only");
-    return m->d.smooth(0, (double*)x, (const double*)b, 1.0, iters, omega, 0.0, st);
+    // in place, on the caller's arrays alone: calls that share a handle may
+    // overlap on several streams, so no pass through the handle's buffers
+    return m->d.smooth_colour(0, (double*)x, (const double*)b, 1.0, iters, omega, 0.0, st);
 }
 
 extern "C" pppm_status pppm_mg_set_blocked_min_cells(pppm_mg* m, uint64_t cells) {
