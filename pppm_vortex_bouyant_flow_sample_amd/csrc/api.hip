@@ -126,18 +126,19 @@ PathGeom make_geom(const pppm_params& p) {
 
 // dir table of the far-field correction (GPU_kernel.cu:2646-2677), FP64 on the
 // host, stored as float3 rows in ((dz+M)(2M+1)+(dy+M))(2M+1)+(dx+M) order, M =
-// max(K, 1).  The curl of the diagonal term c h^2 w (1976-2001), central
-// differences over the face neighbours, is part of the table: +- c / (2 h^2)
-// in component a at +- e_a (the kernel scales by h^3).
+// max(K, 1) (zero for K < 1), then for dz = 1 .. M the sum of component 2 over
+// the plane at dz.
+constexpr size_t kDirFloats = 3 * 9 * 9 * 9 + 4;  // the largest K, 4
 std::vector<float> far_dir_table(int K, double h) {
     const int M = K < 1 ? 1 : K;
     const int W = 2 * M + 1;
-    std::vector<float> out((size_t)W * W * W * 3, 0.f);
+    std::vector<float> out((size_t)W * W * W * 3 + M, 0.f);
+    if (K < 1) return out;
     auto R = [](double ax, double ay, double az, double bx, double by, double bz) {
         double r2 = (ax - bx) * (ax - bx) + (ay - by) * (ay - by) + (az - bz) * (az - bz);
         return r2 > 1e-12 ? kRefFourPi * std::sqrt(r2) : 1e24;
     };
-    const double diag = 0.5 * kRefDiagPsi / (h * h);
+    std::vector<double> plane(M + 1, 0.0);
     for (int kk = -M; kk <= M; kk++)
         for (int jj = -M; jj <= M; jj++)
             for (int ii = -M; ii <= M; ii++) {
@@ -146,17 +147,13 @@ std::vector<float> far_dir_table(int K, double h) {
                 double dx = 0.5 * ((1.0 / R(X + h, X, X, px, py, pz)) - (1.0 / R(X - h, X, X, px, py, pz))) / h;
                 double dy = 0.5 * ((1.0 / R(X, X + h, X, px, py, pz)) - (1.0 / R(X, X - h, X, px, py, pz))) / h;
                 double dz = 0.5 * ((1.0 / R(X, X, X + h, px, py, pz)) - (1.0 / R(X, X, X - h, px, py, pz))) / h;
-                if (K < 1) dx = dy = dz = 0;  // the diagonal term alone
-                if (std::abs(ii) + std::abs(jj) + std::abs(kk) == 1) {
-                    dx += ii * diag;
-                    dy += jj * diag;
-                    dz += kk * diag;
-                }
                 size_t o = 3 * (size_t)(((kk + M) * W + (jj + M)) * W + (ii + M));
                 out[o] = (float)dx;
                 out[o + 1] = (float)dy;
                 out[o + 2] = (float)dz;
+                if (kk > 0) plane[kk] += (double)out[o + 2];
             }
+    for (int kk = 1; kk <= M; kk++) out[(size_t)W * W * W * 3 + kk - 1] = (float)plane[kk];
     return out;
 }
 
@@ -186,7 +183,7 @@ static size_t ctx_bytes(const pppm_params& p, uint32_t capN, uint32_t capM) {
         b += 3 * G * 4;  // psi32
     if (p.precision == PPPM_PREC_MIXED && p.mg_schedule == PPPM_MG_REF_FMG)
         b += MGHier<double>::bytes_for((int)p.g, (int)p.g, (int)p.g, 3);  // the FP64 hierarchy
-    b += 4 * 3 * 9 * 9 * 9;  // direction table
+    b += 4 * kDirFloats;  // direction table
     b += MGHier<float>::bytes_for((int)p.g, (int)p.g, (int)p.g, 3);
     if (capN) b += (size_t)capN * (4 * 4 + 16 + 16) + sort_scratch_bytes(capN);
     if (capM) b += (size_t)capM * (4 * 4 + 16 + 16) + sort_scratch_bytes(capM);
@@ -365,7 +362,7 @@ struct pppm_ctx {
         } else {
             TRY(dev_alloc(&psi32, 3 * G));
         }
-        TRY(dev_alloc(&dir, 3 * 9 * 9 * 9));
+        TRY(dev_alloc(&dir, kDirFloats));
         TRY(upload_dir());
         TRY(mg.init((int)g, (int)g, (int)g, 3));
         return PPPM_OK;

@@ -20,24 +20,31 @@ namespace pppm {
 // next.  dir[D] has component a odd in D_a and even in the other two (a central
 // difference along a of 1/(4 pi |r|)), so the (2K+1)^2 neighbours of a plane are
 // folded to sums and differences over +-y and +-x first and the planes at +-dz
-// share their products: 191 vector instructions a cell at K = 2 where the sum
-// over neighbour pairs took 650, and 45 8-byte LDS reads for two cells where it
-// took 372 4-byte ones a cell.  The curl of the diagonal term, differences over
-// the six face neighbours, is part of the same sum: dir[+-e_a]_a carries
-// +- diag / h^3, and the clamp to the edge (the sum reads zero outside) adds the
-// cell's own w back on the faces of the grid.
-// A thread owns two cells along x.  The curl of psi reads global memory at the
-// end of a plane.  Bound by vector issue and the loads of psi; us a launch, sum
-// over pairs with a ring of 2K+1 planes -> here: 32^3
-// (FP64 psi) 80 -> 17, 64^3 85 -> 20, 96^3 88 -> 44, 128^3 101 -> 68, 256^3 504
-// -> 331 (FP32 psi 483 -> 295).  Held to 3 or 4 waves per SIMD the compiler
-// spills: 1.0 ms at 256^3.
+// share their products.
+// No sum may hold more than differences of w: dir is odd, so a mean of w over
+// the neighbourhood cancels, and would do so in FP32 after rounding.  Along x
+// and y the differences are formed first.  Along z the planes meet only in the
+// output's sum, so dir_2 takes w less a base value of the plane (the mean of
+// the pair's four cells at +-1 in y, rounding nothing where w is smooth), and what the
+// bases would have added, dir_2's plane sums C_dz times their differences
+// over +-dz, joins at the end (C follows dir in the table).  RMS error against 64
+// bits, K = 2, relative to that of one FP32 sum over the pairs w[c+D] - w[c-D]:
+// 0.63 for white noise, 0.14 for 1 + 2% ripple, 0.3 for a sine over the box;
+// with sums in place of the differences 0.7, 9.9 and 1.6.
+// The curl of the diagonal term (face neighbours, clamped to the edge) has its
+// own sums, joined in FP64.  A thread owns two cells along x.  The curl of psi
+// reads global memory at the end of a plane.  Bound by vector issue and the
+// loads of psi; us a launch, sum over pairs with a ring of 2K+1 planes -> here,
+// K = 2: 32^3 (FP64 psi) 80 -> 18, 64^3 85 -> 21, 96^3 89 -> 45, 128^3 101 -> 69,
+// 256^3 503 -> 336 (FP32 psi 467 -> 302); at 128^3 K = 1 51 -> 48, K = 0 83 -> 32.
+// Held to 3 or 4 waves per SIMD the compiler spills.
 constexpr int kCfThreads = 256;
 
 template <typename TP, typename TC, int K, int TX, bool EVEN>
 __global__ void __launch_bounds__(kCfThreads) k_curl_far(const TP* __restrict__ psi, const float* __restrict__ wg,
                                                          float* __restrict__ far, const float* __restrict__ dir,
-                                                         uint32_t g, float h3, TC half_invh, float diag_h3, int zc) {
+                                                         uint32_t g, float h3, TC half_invh, float cdiag_half_invh,
+                                                         int zc) {
     constexpr bool kSum = K >= 0;           // else the grid velocity alone
     constexpr int KC = K < 1 ? 1 : K;       // reach of the sum with the diagonal term
     constexpr int KE = KC + (KC & 1);       // x halo, even
@@ -56,11 +63,17 @@ __global__ void __launch_bounds__(kCfThreads) k_curl_far(const TP* __restrict__ 
     const int gx0 = bx * TX - KE, gy0 = by * TY - KC;
     auto at = [&](int a, int b, int c) { return ((size_t)c * g + (size_t)b) * g + (size_t)a; };
 
-    float acc[W][3][2];
+    // by slot: the sums of the output planes in flight, their diagonal terms
+    // (over 0.5 c h), and of the planes of w the bases and the own x and y
+    // components
+    float acc[W][3][2], dg[W][3][2], bs[W][2], own[W][2][2];
 #pragma unroll
-    for (int s = 0; s < W; s++)
+    for (int s = 0; s < W; s++) {
+        bs[s][0] = bs[s][1] = 0.f;
 #pragma unroll
-        for (int c = 0; c < 3; c++) acc[s][c][0] = acc[s][c][1] = 0.f;
+        for (int c = 0; c < 3; c++) acc[s][c][0] = acc[s][c][1] = dg[s][c][0] = dg[s][c][1] = 0.f;
+        own[s][0][0] = own[s][0][1] = own[s][1][0] = own[s][1][1] = 0.f;
+    }
 
     // plane p of w into registers (zero outside the grid), then LDS
     float ld[NL];
@@ -78,10 +91,10 @@ __global__ void __launch_bounds__(kCfThreads) k_curl_far(const TP* __restrict__ 
         for (int u = 0; u < NL; u++)
             if (tid + kCfThreads * u < 3 * PL) reinterpret_cast<float*>(pl[buf])[tid + kCfThreads * u] = ld[u];
     };
-    // component a of dir at (dx, dy, dz) >= 0, the diagonal term included
+    // component a of dir at (dx, dy, dz) >= 0
     auto coef = [&](int a, int dx, int dy, int dz) { return dir[3 * (((dz + KC) * W + dy + KC) * W + dx + KC) + a]; };
     // outputs z0 .. z1 - 1; plane p = z0 - KC + s, output p - KC complete
-    // after it.  Slot of output k: (k - z0 + KC) mod W.
+    // after it.  Slot of output or plane k: (k - z0 + KC) mod W.
     const int steps = (kSum ? z1 - z0 + 2 * KC : z1 - z0);
     if (kSum) {
         fetch(z0 - KC);
@@ -97,105 +110,157 @@ __global__ void __launch_bounds__(kCfThreads) k_curl_far(const TP* __restrict__ 
             const int k = kSum ? p - KC : p;  // the output that ends here
             if (kSum) {
                 if (s + 1 < steps) fetch(p + 1);
+                bs[sj][0] = bs[sj][1] = 0.f;
                 if (p >= 0 && p < gi) {
-                    float ctr[3][2];  // the cells' own w
 #pragma unroll
                     for (int c = 0; c < 3; c++) {
-                        // rows of component c, folded over +-y
-                        float E[KC + 1][NV], O[KC + 1][NV];
+                        // the pair's row and those r above and below
+                        float r0[NV], up[KC][NV], dn[KC][NV];
 #pragma unroll
                         for (int r = 0; r <= KC; r++) {
-                            const float2* up = &pl[s & 1][(c * PL + (ty + KC + r) * LX) / 2 + tx];
-                            const float2* dn = &pl[s & 1][(c * PL + (ty + KC - r) * LX) / 2 + tx];
+                            const float2* a = &pl[s & 1][(c * PL + (ty + KC + r) * LX) / 2 + tx];
+                            const float2* b = &pl[s & 1][(c * PL + (ty + KC - r) * LX) / 2 + tx];
 #pragma unroll
                             for (int q = 0; q < NV / 2; q++) {
-                                const float2 a = up[q];
+                                const float2 va = a[q];
                                 if (r == 0) {
-                                    E[0][2 * q] = a.x;
-                                    E[0][2 * q + 1] = a.y;
+                                    r0[2 * q] = va.x;
+                                    r0[2 * q + 1] = va.y;
                                 } else {
-                                    const float2 b = dn[q];
-                                    E[r][2 * q] = a.x + b.x;
-                                    E[r][2 * q + 1] = a.y + b.y;
-                                    O[r][2 * q] = a.x - b.x;
-                                    O[r][2 * q + 1] = a.y - b.y;
+                                    const float2 vb = b[q];
+                                    up[r ? r - 1 : 0][2 * q] = va.x;
+                                    up[r ? r - 1 : 0][2 * q + 1] = va.y;
+                                    dn[r ? r - 1 : 0][2 * q] = vb.x;
+                                    dn[r ? r - 1 : 0][2 * q + 1] = vb.y;
                                 }
                             }
                         }
+                        // the diagonal term's differences in the plane, clamped
 #pragma unroll
                         for (int e = 0; e < 2; e++) {
                             const int m = KE + e;
-                            ctr[c][e] = E[0][m];
-                            // sums over the plane for |dz| = 0 .. KC: with
-                            // dir_2 (even in x and y; odd in z, so none at
-                            // dz = 0), dir_0 (odd in x), dir_1 (odd in y)
-                            float s2[KC + 1], s0_[KC + 1], s1[KC + 1];
+                            const float o = r0[m];
+                            const float xm = e == 0 && i == 0 ? o : r0[m - 1], xp = i + e == gi - 1 ? o : r0[m + 1];
+                            const float ym = j == 0 ? o : dn[0][m], yp = j == gi - 1 ? o : up[0][m];
+                            if (c < 2) own[sj][c][e] = o;
+                            if (c == 0) dg[sj][2][e] = ym - yp;
+                            if (c == 1) dg[sj][2][e] += xp - xm;
+                            if (c == 2) {
+                                dg[sj][0][e] = yp - ym;
+                                dg[sj][1][e] = xm - xp;
+                            }
+                        }
+                        if constexpr (K >= 1) {
+                            // folded over +-y: less the base, and differences
+                            float bb = 0.f;
+                            if (c < 2) {
+                                bb = 0.25f * ((up[0][KE] + dn[0][KE]) + (up[0][KE + 1] + dn[0][KE + 1]));
+                                bs[sj][c] = bb;
+                            }
+                            float E[KC + 1][NV], O[KC + 1][NV];
 #pragma unroll
-                            for (int dz = 0; dz <= KC; dz++) s2[dz] = s0_[dz] = s1[dz] = 0.f;
+                            for (int q = 0; q < NV; q++) {
+                                E[0][q] = r0[q] - bb;
 #pragma unroll
-                            for (int dy = 0; dy <= KC; dy++)
-#pragma unroll
-                                for (int dx = 0; dx <= KC; dx++) {
-                                    const float ee = dx == 0 ? E[dy][m] : E[dy][m + dx] + E[dy][m - dx];
-                                    const float oe = dx == 0 ? 0.f : E[dy][m + dx] - E[dy][m - dx];
-                                    const float eo = dy == 0   ? 0.f
-                                                     : dx == 0 ? O[dy][m]
-                                                               : O[dy][m + dx] + O[dy][m - dx];
-#pragma unroll
-                                    for (int dz = 0; dz <= KC; dz++) {
-                                        if (K < 1 && dx + dy + dz != 1) continue;  // no local correction
-                                        if (c != 2 && dz > 0) s2[dz] = fmaf(coef(2, dx, dy, dz), ee, s2[dz]);
-                                        if (c != 0 && dx > 0) s0_[dz] = fmaf(coef(0, dx, dy, dz), oe, s0_[dz]);
-                                        if (c != 1 && dy > 0) s1[dz] = fmaf(coef(1, dx, dy, dz), eo, s1[dz]);
-                                    }
+                                for (int r = 1; r <= KC; r++) {
+                                    E[r][q] = (up[r - 1][q] - bb) + (dn[r - 1][q] - bb);
+                                    O[r][q] = up[r - 1][q] - dn[r - 1][q];
                                 }
-                            // dir x w: x = d1 wz - d2 wy, y = d2 wx - d0 wz,
-                            // z = d0 wy - d1 wx, of outputs p - dz (D_z = dz)
-                            // and p + dz (dir_2 turned round)
+                            }
 #pragma unroll
-                            for (int dz = 0; dz <= KC; dz++) {
-                                const int sl = (sj - dz + W) % W, sh = (sj + dz) % W;
-                                if (c == 0) {
-                                    acc[sl][1][e] += s2[dz];
-                                    acc[sl][2][e] -= s1[dz];
-                                    if (dz > 0) {
-                                        acc[sh][1][e] -= s2[dz];
-                                        acc[sh][2][e] -= s1[dz];
+                            for (int e = 0; e < 2; e++) {
+                                const int m = KE + e;
+                                // sums over the plane for |dz| = 0 .. KC: with
+                                // dir_2 (even in x and y; odd in z, so none at
+                                // dz = 0), dir_0 (odd in x), dir_1 (odd in y)
+                                float s2[KC + 1], s0_[KC + 1], s1[KC + 1];
+#pragma unroll
+                                for (int dz = 0; dz <= KC; dz++) s2[dz] = s0_[dz] = s1[dz] = 0.f;
+#pragma unroll
+                                for (int dy = 0; dy <= KC; dy++)
+#pragma unroll
+                                    for (int dx = 0; dx <= KC; dx++) {
+                                        const int y = dy ? dy - 1 : 0;
+                                        const float ee = dx == 0 ? E[dy][m] : E[dy][m + dx] + E[dy][m - dx];
+                                        // (z has no base: its differences first)
+                                        const float oe = dx == 0  ? 0.f
+                                                         : c < 2  ? E[dy][m + dx] - E[dy][m - dx]
+                                                         : dy == 0 ? r0[m + dx] - r0[m - dx]
+                                                                   : (up[y][m + dx] - up[y][m - dx]) +
+                                                                         (dn[y][m + dx] - dn[y][m - dx]);
+                                        const float eo = dy == 0   ? 0.f
+                                                         : dx == 0 ? O[dy][m]
+                                                                   : O[dy][m + dx] + O[dy][m - dx];
+#pragma unroll
+                                        for (int dz = 0; dz <= KC; dz++) {
+                                            if (c != 2 && dz > 0) s2[dz] = fmaf(coef(2, dx, dy, dz), ee, s2[dz]);
+                                            if (c != 0 && dx > 0) s0_[dz] = fmaf(coef(0, dx, dy, dz), oe, s0_[dz]);
+                                            if (c != 1 && dy > 0) s1[dz] = fmaf(coef(1, dx, dy, dz), eo, s1[dz]);
+                                        }
                                     }
-                                } else if (c == 1) {
-                                    acc[sl][0][e] -= s2[dz];
-                                    acc[sl][2][e] += s0_[dz];
-                                    if (dz > 0) {
-                                        acc[sh][0][e] += s2[dz];
-                                        acc[sh][2][e] += s0_[dz];
-                                    }
-                                } else {
-                                    acc[sl][0][e] += s1[dz];
-                                    acc[sl][1][e] -= s0_[dz];
-                                    if (dz > 0) {
-                                        acc[sh][0][e] += s1[dz];
-                                        acc[sh][1][e] -= s0_[dz];
+                                // dir x w: x = d1 wz - d2 wy, y = d2 wx - d0 wz,
+                                // z = d0 wy - d1 wx, of outputs p - dz (D_z = dz)
+                                // and p + dz (dir_2 turned round)
+#pragma unroll
+                                for (int dz = 0; dz <= KC; dz++) {
+                                    const int sl = (sj - dz + W) % W, sh = (sj + dz) % W;
+                                    if (c == 0) {
+                                        if (dz > 0) {
+                                            acc[sl][1][e] += s2[dz];
+                                            acc[sh][1][e] -= s2[dz];
+                                            acc[sh][2][e] -= s1[dz];
+                                        }
+                                        acc[sl][2][e] -= s1[dz];
+                                    } else if (c == 1) {
+                                        if (dz > 0) {
+                                            acc[sl][0][e] -= s2[dz];
+                                            acc[sh][0][e] += s2[dz];
+                                            acc[sh][2][e] += s0_[dz];
+                                        }
+                                        acc[sl][2][e] += s0_[dz];
+                                    } else {
+                                        acc[sl][0][e] += s1[dz];
+                                        acc[sl][1][e] -= s0_[dz];
+                                        if (dz > 0) {
+                                            acc[sh][0][e] += s1[dz];
+                                            acc[sh][1][e] -= s0_[dz];
+                                        }
                                     }
                                 }
                             }
                         }
                     }
-                    // the diagonal term's differences clamp to the edge
-                    if (p == 0 || p == gi - 1 || j == 0 || j == gi - 1 || i == 0 || i + 2 >= gi) {
+                }
+                // the diagonal term of output p - 1: differences along z, clamped
+                {
+                    const int q = p - 1, sq = (sj - 1 + W) % W, sm = (sj - 2 + W) % W;
 #pragma unroll
-                        for (int e = 0; e < 2; e++) {
-                            const float fx = diag_h3 * ((i + e == gi - 1 ? 1.f : 0.f) - (i + e == 0 ? 1.f : 0.f));
-                            const float fy = diag_h3 * ((j == gi - 1 ? 1.f : 0.f) - (j == 0 ? 1.f : 0.f));
-                            const float fz = diag_h3 * ((p == gi - 1 ? 1.f : 0.f) - (p == 0 ? 1.f : 0.f));
-                            acc[sj][0][e] += fy * ctr[2][e] - fz * ctr[1][e];
-                            acc[sj][1][e] += fz * ctr[0][e] - fx * ctr[2][e];
-                            acc[sj][2][e] += fx * ctr[1][e] - fy * ctr[0][e];
-                        }
+                    for (int e = 0; e < 2; e++) {
+                        const float xm = q == 0 ? own[sq][0][e] : own[sm][0][e];
+                        const float ym = q == 0 ? own[sq][1][e] : own[sm][1][e];
+                        const float xp = q == gi - 1 ? own[sq][0][e] : own[sj][0][e];
+                        const float yp = q == gi - 1 ? own[sq][1][e] : own[sj][1][e];
+                        dg[sq][0][e] += ym - yp;
+                        dg[sq][1][e] += xp - xm;
                     }
                 }
             }
             constexpr int KO = kSum ? KC : 0;
             const int so = (sj - KO + W) % W;
+            if constexpr (K >= 1) {
+                // what the bases of the planes at +-dz stand for
+                const float* c2 = dir + 3 * W * W * W;
+#pragma unroll
+                for (int dz = 1; dz <= KC; dz++) {
+                    const int sl = (so - dz + W) % W, sh = (so + dz) % W;
+                    const float tx_ = c2[dz - 1] * (bs[sh][0] - bs[sl][0]), ty_ = c2[dz - 1] * (bs[sh][1] - bs[sl][1]);
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        acc[so][1][e] += tx_;
+                        acc[so][0][e] -= ty_;
+                    }
+                }
+            }
             if (k >= z0 && k < z1 && i < gi && j < gi) {
                 const int jm = j > 0 ? j - 1 : 0, jp = j < gi - 1 ? j + 1 : gi - 1;
                 const int km = k > 0 ? k - 1 : 0, kp = k < gi - 1 ? k + 1 : gi - 1;
@@ -240,9 +305,12 @@ __global__ void __launch_bounds__(kCfThreads) k_curl_far(const TP* __restrict__ 
                     const TC uy = half_invh * (xzp[e] - xzm[e] + zx[e] - zx[e + 2]);
                     const TC uz = half_invh * (yx[e + 2] - yx[e] + xm_[e] - xp_[e]);
                     const size_t c = at(i + e, j, k);
-                    far[c] = (float)((double)ux - (double)(acc[so][0][e] * h3));
-                    far[G + c] = (float)((double)uy - (double)(acc[so][1][e] * h3));
-                    far[2 * G + c] = (float)((double)uz - (double)(acc[so][2][e] * h3));
+                    const double u[3] = {(double)ux, (double)uy, (double)uz};
+#pragma unroll
+                    for (int q = 0; q < 3; q++) {
+                        const float v = acc[so][q][e] * h3, d = cdiag_half_invh * dg[so][q][e];
+                        far[q * G + c] = (float)(kSum ? u[q] - (double)v - (double)d : u[q]);
+                    }
                 }
             }
 #pragma unroll
@@ -255,8 +323,10 @@ __global__ void __launch_bounds__(kCfThreads) k_curl_far(const TP* __restrict__ 
     }
 }
 
-// K = 4: the sums of nine planes do not fit the registers of k_curl_far (1.0 to
-// 1.7 ms at 128^3 against 0.64 here), so the sum runs over pairs of neighbours.
+// K = 3 and 4: the sums of seven or nine planes do not fit the registers of
+// k_curl_far (us, k_curl_far against here: 32^3 50 / 28, 128^3 228 / 177, 256^3
+// 1020 / 1232 at K = 3; K = 4 at 128^3 1.0 to 1.7 ms / 645), so the sum runs over
+// pairs of neighbours.
 // A workgroup owns a 32 x 8 tile of cells and a run of z planes.  The grid
 // vorticity streams through an LDS ring of 2K+1 planes with a K-cell halo
 // (zero outside the grid, which is the reference's in-grid-only sum), so the
@@ -267,8 +337,7 @@ constexpr int kCfTX = 32, kCfTY = 8;
 template <typename TP, typename TC, int K>
 __global__ void __launch_bounds__(256) k_curl_far_pairs(const TP* __restrict__ psi, const float* __restrict__ wg,
                                                   float* __restrict__ far, const float* __restrict__ dir, uint32_t g,
-                                                  float h3, TC half_invh, float diag_h3,
-                                                  int zc) {
+                                                  float h3, TC half_invh, float cdiag_half_invh, int zc) {
     constexpr int W = 2 * K + 1, LXW = kCfTX + 2 * K, LYW = kCfTY + 2 * K, PLW = LXW * LYW;
     __shared__ float ring[W][3][PLW];
     const uint32_t G = g * g * g;
@@ -318,21 +387,20 @@ __global__ void __launch_bounds__(256) k_curl_far_pairs(const TP* __restrict__ p
                                  (TC)Pz[at(ip, j, k)]);
             TC uz = half_invh * ((TC)Py[at(ip, j, k)] - (TC)Py[at(im, j, k)] + (TC)Px[at(i, jm, k)] -
                                  (TC)Px[at(i, jp, k)]);
+            // diagonal term: curl of 0.2505806 h^2 w with the same clamped
+            // stencil; the ring holds the neighbours (the clamp reads the edge
+            // cell itself, which the ring holds too)
+            auto wr = [&](int comp, int ii, int jj, int kk) {
+                return ring[((kk % W) + W) % W][comp][(jj - gy0) * LXW + (ii - gx0)];
+            };
+            const float dx = cdiag_half_invh * (wr(2, i, jp, k) - wr(2, i, jm, k) + (wr(1, i, j, km) - wr(1, i, j, kp)));
+            const float dy = cdiag_half_invh * (wr(0, i, j, kp) - wr(0, i, j, km) + (wr(2, im, j, k) - wr(2, ip, j, k)));
+            const float dz = cdiag_half_invh * (wr(1, ip, j, k) - wr(1, im, j, k) + (wr(0, i, jm, k) - wr(0, i, jp, k)));
             // local correction over the (2K+1)^3 block.  dir is odd,
             // dir[-D] = -dir[D] (a central difference of the even 1/(4 pi |r|),
             // computed so in FP64 and rounded), so D and -D are taken
             // together: dir[D] x (w[c+D] - w[c-D]); h^3 is applied once.
             float vx = 0.f, vy = 0.f, vz = 0.f;
-            if (k == 0 || k == gi - 1 || j == 0 || j == gi - 1 || i == 0 || i == gi - 1) {
-                // the diagonal term's differences clamp to the edge
-                const float* c = &ring[((k % W) + W) % W][0][(ly + K) * LXW + lx + K];
-                const float fx = diag_h3 * ((i == gi - 1 ? 1.f : 0.f) - (i == 0 ? 1.f : 0.f));
-                const float fy = diag_h3 * ((j == gi - 1 ? 1.f : 0.f) - (j == 0 ? 1.f : 0.f));
-                const float fz = diag_h3 * ((k == gi - 1 ? 1.f : 0.f) - (k == 0 ? 1.f : 0.f));
-                vx = fy * c[2 * PLW] - fz * c[PLW];
-                vy = fz * c[0] - fx * c[2 * PLW];
-                vz = fx * c[PLW] - fy * c[0];
-            }
 #pragma unroll
             for (int a = 0; a <= K; a++) {
                 const float* rp = &ring[(((k + a) % W) + W) % W][0][0];
@@ -359,9 +427,9 @@ __global__ void __launch_bounds__(256) k_curl_far_pairs(const TP* __restrict__ p
             vy *= h3;
             vz *= h3;
             const size_t c = at(i, j, k);
-            far[c] = (float)((double)ux - (double)vx);
-            far[(size_t)G + c] = (float)((double)uy - (double)vy);
-            far[2 * (size_t)G + c] = (float)((double)uz - (double)vz);
+            far[c] = (float)((double)ux - (double)vx - (double)dx);
+            far[(size_t)G + c] = (float)((double)uy - (double)vy - (double)dy);
+            far[2 * (size_t)G + c] = (float)((double)uz - (double)vz - (double)dz);
         }
         __syncthreads();  // the next plane load reuses the slot of plane k - K
     }
@@ -381,12 +449,15 @@ static void launch_curl_far_k(const TP* psi, const float* wgrid, float* far, con
         case 0: hipLaunchKernelGGL((k_curl_far<TP, TC, 0, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
         case 1: hipLaunchKernelGGL((k_curl_far<TP, TC, 1, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
         case 2: hipLaunchKernelGGL((k_curl_far<TP, TC, 2, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
-        case 3: hipLaunchKernelGGL((k_curl_far<TP, TC, 3, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
+        case 3:
         case 4: {
-            // two workgroups (69 KB of LDS each) a CU
-            const uint32_t t4 = div_up(g, kCfTX) * div_up(g, kCfTY);
-            const int zc4 = std::max(2, std::min(16, (int)div_up(g * t4, 512)));
-            hipLaunchKernelGGL((k_curl_far_pairs<TP, TC, 4>), dim3(t4, div_up(g, zc4)), blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc4);
+            // as many workgroups as fit the chip's LDS at once: three of 45 KB
+            // a CU (K = 3), two of 69 KB (K = 4)
+            const uint32_t tp = div_up(g, kCfTX) * div_up(g, kCfTY);
+            const int zp = std::max(2, std::min(16, (int)div_up(g * tp, K == 3 ? 768 : 512)));
+            const dim3 gp(tp, div_up(g, zp));
+            if (K == 3) hipLaunchKernelGGL((k_curl_far_pairs<TP, TC, 3>), gp, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zp);
+            else hipLaunchKernelGGL((k_curl_far_pairs<TP, TC, 4>), gp, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zp);
             break;
         }
         default: hipLaunchKernelGGL((k_curl_far<TP, TC, -1, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
@@ -397,9 +468,8 @@ pppm_status launch_curl_far_impl(const void* psi, int psi_dtype, const float* wg
                                  uint32_t g, int K, double h, hipStream_t st) {
     const float h3 = (float)(h * h * h);
     const double half_invh = 0.5 * (1.0 / h);
-    // the diagonal term's difference factor over h^3 (the sum is scaled by
-    // h^3); vortex-in-cell (K < 0): the buffer is the grid velocity itself
-    const float cd = K < 0 ? 0.0f : (float)(kRefDiagPsi * h * h * half_invh / (h * h * h));
+    // vortex-in-cell (K < 0): the far-field buffer is the grid velocity itself
+    const float cd = K < 0 ? 0.0f : (float)(kRefDiagPsi * h * h * half_invh);
     // 64-cell tiles along x, or 32 where they would leave a third of the
     // threads or more without cells
     const bool t64 = g % 64 == 0 || g > 128;
