@@ -35,35 +35,67 @@ __device__ inline T nb_sum(const T* __restrict__ x, size_t t, int i, int j, int 
     return r;
 }
 
-// Relaxation factor over the diagonal 6 - beta nout of a cell with nout
-// neighbours outside and a ghost factor beta; 0 stands for omega / 6.
+// What k_rbgs, k_tile, k_vtail and (FP64) k_rb4 do to a cell, to a residual and
+// to a coarse value is written here once, with its fused multiply-adds spelt
+// out and no others, so that a level's values are bitwise the same whichever of
+// them runs it: the choice may go by the work of all components together, and a
+// component solved with others is bitwise the one solved alone.
+__device__ inline float fma_(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ inline double fma_(double a, double b, double c) { return fma(a, b, c); }
+// relaxation factor over the diagonal 6 - beta nout of a cell with nout
+// neighbours outside and a ghost factor beta; w6 = omega / 6 (the host's: a
+// division a thread made k_rbgs<double> 2% slower)
 template <typename T>
-__device__ inline T rbgs_weight(int nout, T omega, T beta) {
-    return beta == (T)0 || nout == 0 ? (T)0 : omega / ((T)6 - beta * (T)nout);
+__device__ inline T relax_weight(int nout, T omega, T beta, T w6) {
+    return beta == (T)0 || nout == 0 ? w6 : omega / fma_(-beta, (T)nout, (T)6);
 }
-// SOR update of a cell: x from the sum r of its neighbours, bscale times its
-// right-hand side bv and its rbgs_weight w (k_rbgs; k_vtail on a level held in
-// LDS, which forms w once for all its half-sweeps).
+// SOR update of a cell: x from the sum s of its neighbours, bscale times its
+// right-hand side b, its relax_weight w and om1 = 1 - omega
 template <typename T>
-__device__ inline T rbgs_value(T x, T r, T bv, T bscale, T w, T omega) {
-    r -= bscale * bv;
-    const T s = w != (T)0 ? w * r : omega * r * (T)(1.0 / 6.0);
-    return ((T)1 - omega) * x + s;
+__device__ inline T relax(T x, T s, T b, T bscale, T w, T om1) {
+#pragma clang fp contract(off)
+    return fma_(w, fma_(-bscale, b, s), om1 * x);
 }
+// residual of a cell, s the sum of its neighbours
+template <typename T>
+__device__ inline T residual_of(T x, T s, T b, T bscale, int nout, T beta) {
+#pragma clang fp contract(off)
+    s = fma_((T)-6, x, s);
+    if (beta != (T)0) s = fma_(beta * (T)nout, x, s);
+    return fma_(bscale, b, -s);
+}
+// 1 - w and w of a parent and its neighbour
+template <typename T>
+__device__ inline T lerp_(T w, T parent, T neighbour) {
+#pragma clang fp contract(off)
+    return fma_(w, neighbour, ((T)1 - w) * parent);
+}
+// coarse value c outside the coarse grid: ghost factors of the three axes
+template <typename T>
+__device__ inline T ghost(T fi, T fj, T fk, T c) {
+#pragma clang fp contract(off)
+    return ((fi * fj) * fk) * c;
+}
+// the 8 children's residuals of a coarse cell: pairs along x, then y, then z
+template <typename T>
+__device__ inline T restrict_sum(T p00, T p10, T p01, T p11) {
+    return ((p00 + p10) + (p01 + p11)) * (T)0.5;
+}
+
 template <typename T>
 __device__ inline void rbgs_point(T* xc, T bv, T bscale, int i, int j, int k, int nx, int ny, int nz, T omega,
-                                  T beta) {
+                                  T beta, T w6) {
     const size_t t = ((size_t)k * ny + j) * nx + i;
     int nout;
-    const T r = nb_sum(xc, t, i, j, k, nx, ny, nz, nout);
-    xc[t] = rbgs_value(xc[t], r, bv, bscale, rbgs_weight(nout, omega, beta), omega);
+    const T s = nb_sum(xc, t, i, j, k, nx, ny, nz, nout);
+    xc[t] = relax(xc[t], s, bv, bscale, relax_weight(nout, omega, beta, w6), (T)1 - omega);
 }
 
 // One colour of red-black SOR.  color 1 = (i+j+k) odd (swept first, as the
 // reference's "red" kernel), 0 = even.
 template <typename T>
 __global__ void __launch_bounds__(256) k_rbgs(T* __restrict__ x, const T* __restrict__ b, T bscale, int nx, int ny,
-                                              int nz, size_t G, int color, T omega, T beta) {
+                                              int nz, size_t G, int color, T omega, T beta, T w6) {
     const int i2 = blockIdx.x * 64 + threadIdx.x;
     const int j = blockIdx.y * 4 + threadIdx.y;
     const int comp = blockIdx.z / nz, k = blockIdx.z - comp * nz;
@@ -71,7 +103,7 @@ __global__ void __launch_bounds__(256) k_rbgs(T* __restrict__ x, const T* __rest
     const int i = 2 * i2 + ((j + k + color) & 1);
     if (i >= nx) return;
     const size_t t = ((size_t)k * ny + j) * nx + i;
-    rbgs_point(x + (size_t)comp * G, b[(size_t)comp * G + t], bscale, i, j, k, nx, ny, nz, omega, beta);
+    rbgs_point(x + (size_t)comp * G, b[(size_t)comp * G + t], bscale, i, j, k, nx, ny, nz, omega, beta, w6);
 }
 
 // Tile of the blocked smoother k_rb2 (below): 64 x 16 cells per workgroup.
@@ -87,6 +119,7 @@ struct TbArgsT {
     int nx, ny, nz;
     size_t G;            // cells per component
     T omega, beta;   // SOR factor, ghost factor of this level
+    T w6;            // omega / 6 (FP64)
     int zc;              // z planes per workgroup chunk (even)
     // RESTRICT: residual restricted into bn (coarse dims cx, cy, cz = n / 2)
     T* bn;
@@ -717,7 +750,9 @@ k_rbc(TbArgs a) {
 // exact beyond the region, which saves one.  Planes outside the grid are
 // zero and stay so, as cells outside it in x and y.  Needs nx even.
 //
-// Sums are formed in k_rbc's order.  One workgroup of 16 waves a CU, bound
+// Sums are formed in k_rbc's order; FP32 updates are k_rbc's, FP64 ones relax
+// (x + w (s d - x) rounds at the size of the x that it replaces; full multigrid
+// at 64^3 from its 80-bit evaluation: 8.5e-16, with relax 5.3e-16).  One workgroup of 16 waves a CU, bound
 // by its planes' loads and by vector issue at once.  256^3 x 3, V(2,2) (us):
 // down from zero 107 + 179 (two k_rbc passes) -> 128, up 203 + 151 -> 205;
 // 96^3 x 3: 39 -> 18, 41 -> 22.
@@ -727,9 +762,6 @@ constexpr int kR4Region = 64;
 // 64 x 32, whose planes in flight need the registers of two waves per SIMD.
 template <typename T>
 constexpr int r4_threads() { return sizeof(T) == 4 ? 1024 : 512; }
-
-__device__ inline float r4_fma(float a, float b, float c) { return fmaf(a, b, c); }
-__device__ inline double r4_fma(double a, double b, double c) { return fma(a, b, c); }
 
 // value of the lane that DPP control C selects (0x130: lane + 1, 0x138: lane - 1)
 template <int C>
@@ -777,6 +809,7 @@ struct R4Pair<double> {
 template <typename T, bool RESTRICT, bool PROLONG, bool XZERO, bool BETA>
 __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
     constexpr int NT = r4_threads<T>(), RG = NT / 32;  // row groups of the region
+    constexpr bool kRelax = sizeof(T) == 8;  // relax, as the kernels of smaller levels; FP32: k_rbc's form
     constexpr bool kWide = RESTRICT && !XZERO;
     constexpr int HXY = kWide ? 6 : 4, HZ = kWide ? 5 : 4;
     constexpr int TW = kR4Region - 2 * HXY, TH = 2 * RG - 2 * HXY;  // tile
@@ -826,8 +859,10 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
     bool gin[2];
     T wr[2];
     // cells outside the grid next to a cell in the plane, and the diagonal's
-    // reciprocal off and on the first and last plane
+    // reciprocal (kRelax: the relaxation factor) off and on the first and last
+    // plane
     T nxy[2][2], d0[2][2], d1[2][2];
+    const T om1 = (T)1 - omega;
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         const int j = gy0 + 2 * rg + r, ly = 2 * rg + r;
@@ -838,9 +873,15 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int i = i0 + e;
-            nxy[r][e] = (T)((i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1));
-            d0[r][e] = (T)1.0 / ((T)6.0 - beta * nxy[r][e]);
-            d1[r][e] = (T)1.0 / ((T)6.0 - beta * (nxy[r][e] + (nz == 1 ? (T)2 : (T)1)));
+            const int no = (i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1), noz = no + (nz == 1 ? 2 : 1);
+            nxy[r][e] = (T)no;
+            if constexpr (kRelax) {  // a cell outside the grid is 0 and stays so
+                d0[r][e] = gin[r] ? relax_weight(no, omega, BETA ? beta : (T)0, a.w6) : (T)0;
+                d1[r][e] = gin[r] ? relax_weight(noz, omega, BETA ? beta : (T)0, a.w6) : (T)0;
+            } else {
+                d0[r][e] = (T)1.0 / ((T)6.0 - beta * (T)no);
+                d1[r][e] = (T)1.0 / ((T)6.0 - beta * (T)noz);
+            }
         }
     }
     const int gI = i0 >> 1, gJ = (gy0 >> 1) + rg;
@@ -1013,9 +1054,16 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
                         s += r ? X[jp][0][e] + y[t - 1][1] : y[t - 1][0] + X[jp][1][e];
                         s += X[jm][r][e] + X[jq][r][e];
                     }
-                    s = r4_fma(-bscale, B[jp][r][e], s);
-                    const T d = BETA ? (zb ? d1[r][e] : d0[r][e]) : (T)1.0 / (T)6.0, xo = X[jp][r][e];
-                    const T xn = xo + (in ? wr[r] : (T)0) * (s * d - xo);
+                    const T xo = X[jp][r][e];
+                    T xn;
+                    if constexpr (kRelax) {
+                        const T w = BETA && zb ? d1[r][e] : d0[r][e];
+                        xn = relax(xo, s, B[jp][r][e], bscale, in ? w : (T)0, om1);
+                    } else {
+                        s = fma_(-bscale, B[jp][r][e], s);
+                        const T d = BETA ? (zb ? d1[r][e] : d0[r][e]) : (T)1.0 / (T)6.0;
+                        xn = xo + (in ? wr[r] : (T)0) * (s * d - xo);
+                    }
                     X[jp][r][e] = xn;
                     if (t < 4 || RESTRICT) ex[xslot(t, j)][r][lo + 32] = xn;
                 }
@@ -1046,7 +1094,7 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
                         s += X[jm][r][e] + X[jq][r][e];
                         s -= (T)6.0 * xo;
                         if (BETA) s += beta * (nxy[r][e] + zb) * xo;
-                        part[r] += r4_fma(bscale, B[jr][r][e], -s);
+                        part[r] += fma_(bscale, B[jr][r][e], -s);
                     }
                 }
                 if ((jr & 1) == 0) {
@@ -1072,30 +1120,25 @@ __device__ inline T residual_at(const T* __restrict__ x, const T* __restrict__ b
                                 int nx, int ny, int nz, T beta) {
     const size_t t = ((size_t)k * ny + j) * nx + i;
     int nout;
-    T s = nb_sum(x, t, i, j, k, nx, ny, nz, nout);
-    s -= (T)6 * x[t];
-    if (beta != (T)0 && nout) s += beta * (T)nout * x[t];
-    return bscale * b[t] - s;
+    const T s = nb_sum(x, t, i, j, k, nx, ny, nz, nout);
+    return residual_of(x[t], s, b[t], bscale, nout, beta);
 }
 
 // r = b - A x at the 8 children of coarse cell (ci, cj, ck), summed and
-// halved (children order as MultiGrid_kernel.cu:897-904).
+// halved (the sum of MultiGrid_kernel.cu:897-904).
 template <typename T>
 __device__ inline T restrict_point(const T* xc, const T* bc, T bscale, int ci, int cj, int ck, int nx, int ny, int nz,
                                    T beta) {
     const int i = 2 * ci, j = 2 * cj, k = 2 * ck;
     // children beyond a fine dimension of 1 do not exist
     const bool hi = i + 1 < nx, hj = j + 1 < ny, hk = k + 1 < nz;
-    T r = 0;
-    r += residual_at(xc, bc, bscale, i, j, k, nx, ny, nz, beta);
-    if (hi) r += residual_at(xc, bc, bscale, i + 1, j, k, nx, ny, nz, beta);
-    if (hj) r += residual_at(xc, bc, bscale, i, j + 1, k, nx, ny, nz, beta);
-    if (hi && hj) r += residual_at(xc, bc, bscale, i + 1, j + 1, k, nx, ny, nz, beta);
-    if (hk) r += residual_at(xc, bc, bscale, i, j, k + 1, nx, ny, nz, beta);
-    if (hi && hk) r += residual_at(xc, bc, bscale, i + 1, j, k + 1, nx, ny, nz, beta);
-    if (hj && hk) r += residual_at(xc, bc, bscale, i, j + 1, k + 1, nx, ny, nz, beta);
-    if (hi && hj && hk) r += residual_at(xc, bc, bscale, i + 1, j + 1, k + 1, nx, ny, nz, beta);
-    return r * (T)0.5;
+    auto pair = [&](int jj, int kk) {
+        const T r = residual_at(xc, bc, bscale, i, jj, kk, nx, ny, nz, beta);
+        return hi ? r + residual_at(xc, bc, bscale, i + 1, jj, kk, nx, ny, nz, beta) : r;
+    };
+    const T p00 = pair(j, k), p10 = hj ? pair(j + 1, k) : (T)0;
+    const T p01 = hk ? pair(j, k + 1) : (T)0, p11 = hj && hk ? pair(j + 1, k + 1) : (T)0;
+    return restrict_sum(p00, p10, p01, p11);
 }
 
 // b_c = restrict_point at every coarse cell.
@@ -1128,14 +1171,14 @@ __device__ inline T prolong_point(const T* c, int i, int j, int k, int nx, int n
         if (ni < 0 || ni > cx - 1) { ni = pi; fi = betac; }
         if (nj < 0 || nj > cy - 1) { nj = pj; fj = betac; }
         if (nk < 0 || nk > cz - 1) { nk = pk; fk = betac; }
-        auto C = [&](int a, int bb, int cc) { return c[((size_t)cc * cy + bb) * cx + a]; };
-        T p0 = ((T)1 - wi) * C(pi, pj, pk) + wi * fi * C(ni, pj, pk);
-        T p1 = ((T)1 - wi) * C(pi, nj, pk) + wi * fi * C(ni, nj, pk);
-        T p2 = ((T)1 - wi) * C(pi, pj, nk) + wi * fi * C(ni, pj, nk);
-        T p3 = ((T)1 - wi) * C(pi, nj, nk) + wi * fi * C(ni, nj, nk);
-        T q0 = ((T)1 - wj) * p0 + wj * fj * p1;
-        T q1 = ((T)1 - wj) * p2 + wj * fj * p3;
-        v = ((T)1 - wk) * q0 + wk * fk * q1;
+        // the parent's or the neighbour's value on each axis
+        auto C = [&](bool x, bool y, bool z) {
+            return ghost(x ? fi : (T)1, y ? fj : (T)1, z ? fk : (T)1,
+                         c[((size_t)(z ? nk : pk) * cy + (y ? nj : pj)) * cx + (x ? ni : pi)]);
+        };
+        const T p0 = lerp_(wi, C(0, 0, 0), C(1, 0, 0)), p1 = lerp_(wi, C(0, 1, 0), C(1, 1, 0));
+        const T p2 = lerp_(wi, C(0, 0, 1), C(1, 0, 1)), p3 = lerp_(wi, C(0, 1, 1), C(1, 1, 1));
+        v = lerp_(wk, lerp_(wj, p0, p1), lerp_(wj, p2, p3));
     }
     return v;
 }
@@ -1186,7 +1229,7 @@ struct TileArgs {
     T bscale;
     int nx, ny, nz;
     size_t G;
-    T omega, beta;
+    T omega, beta, w6;  // w6 = omega / 6
     int iters;  // 1 or 2
     int tx, ty, tz;
     // residual restricted into bn (null: none), coarse dims n / 2
@@ -1276,8 +1319,8 @@ __global__ void __launch_bounds__(tile_threads(TI)) k_tile(TileArgs<T> a) {
             const int q = min(tid + NT * u, CW * CW * CW - 1);
             const int cx_ = c0x + q % CW, cy_ = c0y + (q / CW) % CW, cz_ = c0z + q / (CW * CW);
             const int ix = min(max(cx_, 0), a.cx - 1), iy = min(max(cy_, 0), a.cy - 1), iz = min(max(cz_, 0), a.cz - 1);
-            const T f = (ix != cx_ ? gb : (T)1) * (iy != cy_ ? gb : (T)1) * (iz != cz_ ? gb : (T)1);
-            cv[u] = f * xc[((size_t)iz * a.cy + iy) * a.cx + ix];
+            cv[u] = ghost(ix != cx_ ? gb : (T)1, iy != cy_ ? gb : (T)1, iz != cz_ ? gb : (T)1,
+                          xc[((size_t)iz * a.cy + iy) * a.cx + ix]);
         }
 #pragma unroll
         for (int u = 0; u < NC; u++) aux[min(tid + NT * u, CW * CW * CW - 1)] = cv[u];
@@ -1298,23 +1341,22 @@ __global__ void __launch_bounds__(tile_threads(TI)) k_tile(TileArgs<T> a) {
             } else {
                 // 3/4 the parent, 1/4 its neighbour on the cell's side
                 const int qy = py + ((gj & 1) ? 1 : -1), qz = pz + ((gk & 1) ? 1 : -1);
+                const T w4 = (T)0.25;
                 T ye[2], yo[2];
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const T* r0 = aux + ((h ? qz : pz) * CW + py) * CW + px;
                     const T* r1 = aux + ((h ? qz : pz) * CW + qy) * CW + px;
-                    ye[h] = (T)0.75 * ((T)0.75 * r0[0] + (T)0.25 * r0[-1]) +
-                            (T)0.25 * ((T)0.75 * r1[0] + (T)0.25 * r1[-1]);
-                    yo[h] = (T)0.75 * ((T)0.75 * r0[0] + (T)0.25 * r0[1]) +
-                            (T)0.25 * ((T)0.75 * r1[0] + (T)0.25 * r1[1]);
+                    ye[h] = lerp_(w4, lerp_(w4, r0[0], r0[-1]), lerp_(w4, r1[0], r1[-1]));
+                    yo[h] = lerp_(w4, lerp_(w4, r0[0], r0[1]), lerp_(w4, r1[0], r1[1]));
                 }
-                xr[0][q] += (T)0.75 * ye[0] + (T)0.25 * ye[1];
-                xr[1][q] += (T)0.75 * yo[0] + (T)0.25 * yo[1];
+                xr[0][q] += lerp_(w4, ye[0], ye[1]);
+                xr[1][q] += lerp_(w4, yo[0], yo[1]);
             }
         }
         // first, second cell -> colour 0, 1; a second cell that does not
         // exist stays 0 (its relaxation factor is 0)
-        const T u0 = xr[0][q], u1 = two ? xr[1][q] : (T)0, d0 = a.bscale * bc[0][q], d1 = a.bscale * bc[1][q];
+        const T u0 = xr[0][q], u1 = two ? xr[1][q] : (T)0, d0 = bc[0][q], d1 = bc[1][q];
         const bool sw = (p ^ (q & 1)) != 0;
         xr[0][q] = sw ? u1 : u0;
         xr[1][q] = sw ? u0 : u1;
@@ -1328,18 +1370,17 @@ __global__ void __launch_bounds__(tile_threads(TI)) k_tile(TileArgs<T> a) {
     // x neighbour outside the pair is the other colour's at index e ? + 1 : - 1.
     // Xn[v]: that index for e = p ^ v.
     const T* const Xn[2] = {X + (p ? 1 : -1), X + (p ? -1 : 1)};
-    // relaxation factor over the diagonal of cell e = p ^ v: w / 6, and with a
-    // ghost factor beta (nout neighbours outside) w / (6 - beta nout), wz in
-    // the first and last grid plane
+    // relax_weight of cell e = p ^ v, wz in the first and last grid plane (0
+    // for a second cell that does not exist)
     const int nout_y = (gj == 0) + (gj == ny - 1);
     T w[2], wz[2];
 #pragma unroll
     for (int v = 0; v < 2; v++) {
         const int e = p ^ v, i = gi + e;
         const int no = nout_y + (i == 0) + (i == nx - 1);
-        const T om = e == 0 || two ? a.omega : (T)0;
-        w[v] = BETA ? om / ((T)6 - a.beta * (T)no) : om * (T)(1.0 / 6.0);
-        wz[v] = BETA ? om / ((T)6 - a.beta * (T)(no + 1)) : w[v];
+        const bool cell = e == 0 || two;
+        w[v] = cell ? relax_weight(no, a.omega, BETA ? a.beta : (T)0, a.w6) : (T)0;
+        wz[v] = BETA && cell ? relax_weight(no + 1, a.omega, a.beta, a.w6) : w[v];
     }
     const int qlo = -gk0, qhi = nz - 1 - gk0;  // plane indices of the z boundaries
     const T om1 = (T)1 - a.omega;
@@ -1362,9 +1403,8 @@ __global__ void __launch_bounds__(tile_threads(TI)) k_tile(TileArgs<T> a) {
                 T r = xr[1 - c][q] + Xn[v][(1 - c) * PC + q * PZ];
                 r += O[q * PZ + PX] + O[q * PZ - PX];
                 r += zm + zp;
-                r -= bc[c][q];
                 const T wq = BETA && (q == qlo || q == qhi) ? wz[v] : w[v];
-                xr[c][q] = om1 * xr[c][q] + wq * r;
+                xr[c][q] = relax(xr[c][q], r, bc[c][q], a.bscale, wq, om1);
                 X[c * PC + q * PZ] = xr[c][q];
             }
             __syncthreads();
@@ -1391,13 +1431,10 @@ __global__ void __launch_bounds__(tile_threads(TI)) k_tile(TileArgs<T> a) {
             T r = xr[1 - c][q] + Xn[v][(1 - c) * PC + q * PZ];
             r += O[q * PZ + PX] + O[q * PZ - PX];
             r += O[q * PZ - PZ] + O[q * PZ + PZ];
-            r -= (T)6 * xr[c][q];
-            if (BETA) {
-                const int i = gi + (p ^ v);
-                const int no = nout_y + (i == 0) + (i == nx - 1) + (gk == 0) + (gk == nz - 1);
-                r += a.beta * (T)no * xr[c][q];
-            }
-            part += bc[c][q] - r;
+            const int i = gi + (p ^ v);
+            const int no = nout_y + (i == 0) + (i == nx - 1) + (gk == 0) + (gk == nz - 1);
+            r = residual_of(xr[c][q], r, bc[c][q], a.bscale, no, BETA ? a.beta : (T)0);
+            part = c == 0 ? r : part + r;
         }
         aux[((gk - t0z) * TI + (gj - t0y)) * RW + ((gi - t0x) >> 1)] = part;
     }
@@ -1410,7 +1447,7 @@ __global__ void __launch_bounds__(tile_threads(TI)) k_tile(TileArgs<T> a) {
             if (ci >= a.cx || cj >= a.cy || ck >= a.cz) continue;
             const T* r = aux + ((2 * K) * TI + 2 * J) * RW + I;
             bn[((size_t)ck * a.cy + cj) * a.cx + ci] =
-                ((r[0] + r[RW]) + (r[TI * RW] + r[TI * RW + RW])) * (T)0.5;
+                restrict_sum(r[0], r[RW], r[TI * RW], r[TI * RW + RW]);
         }
     }
 }
@@ -1522,7 +1559,7 @@ struct TailArgs {
     T beta0, beta1;       // ghost factors of the two levels
     int mode;             // prolongation
     int nu1, nu2;
-    T omega;
+    T omega, w6;          // w6 = omega / 6
     const double* tab;    // coarsest eigenbasis
 };
 
@@ -1603,9 +1640,10 @@ __global__ void __launch_bounds__(kTailThreads) k_vtail(TailArgs<T> a) {
     T we[kTailPairs], wo[kTailPairs];
 #pragma unroll
     for (int q = 0; q < kTailPairs; q++) {
-        we[q] = rbgs_weight(outside(0, k0 + q), a.omega, a.beta0);
-        wo[q] = rbgs_weight(outside(1, k0 + q), a.omega, a.beta0);
+        we[q] = relax_weight(outside(0, k0 + q), a.omega, a.beta0, a.w6);
+        wo[q] = relax_weight(outside(1, k0 + q), a.omega, a.beta0, a.w6);
     }
+    const T om1 = (T)1 - a.omega;
     auto smooth = [&](int iters) {
         for (int h = 0; h < iters; h++)
 #pragma unroll
@@ -1614,8 +1652,8 @@ __global__ void __launch_bounds__(kTailThreads) k_vtail(TailArgs<T> a) {
                 for (int q = 0; q < kTailPairs; q++) {
                     const int e = p ^ c ^ (q & 1), o = o0 + q * PZ;
                     if (q < nq && (e == 0 || two))
-                        xa[c][o] = rbgs_value(xa[c][o], nbr(c, o, e), e ? bo[q] : be[q], a.bscale,
-                                              e ? wo[q] : we[q], a.omega);
+                        xa[c][o] = relax(xa[c][o], nbr(c, o, e), e ? bo[q] : be[q], a.bscale, e ? wo[q] : we[q],
+                                         om1);
                 }
                 __syncthreads();
             }
@@ -1632,11 +1670,7 @@ __global__ void __launch_bounds__(kTailThreads) k_vtail(TailArgs<T> a) {
                 const int c = p ^ e ^ (q & 1);
                 if (e == 1 && !two) continue;
                 const T xv = xa[c][o];
-                T r = nbr(c, o, e);
-                r -= (T)6 * xv;
-                const int no = outside(e, k0 + q);
-                if (a.beta0 != (T)0 && no) r += a.beta0 * (T)no * xv;
-                rs[t + e] = a.bscale * (e ? bo[q] : be[q]) - r;
+                rs[t + e] = residual_of(xv, nbr(c, o, e), e ? bo[q] : be[q], a.bscale, outside(e, k0 + q), a.beta0);
             }
         }
     __syncthreads();
@@ -1644,16 +1678,9 @@ __global__ void __launch_bounds__(kTailThreads) k_vtail(TailArgs<T> a) {
         const int ci = q % cx, cj = (q / cx) % cy, ck = q / (cx * cy);
         const bool hi = 2 * ci + 1 < nx, hj = 2 * cj + 1 < ny, hk = 2 * ck + 1 < nz;
         const T* f = rs + ((2 * ck) * ny + 2 * cj) * nx + 2 * ci;
-        T r = 0;
-        r += f[0];
-        if (hi) r += f[1];
-        if (hj) r += f[nx];
-        if (hi && hj) r += f[nx + 1];
-        if (hk) r += f[nx * ny];
-        if (hi && hk) r += f[nx * ny + 1];
-        if (hj && hk) r += f[nx * ny + nx];
-        if (hi && hj && hk) r += f[nx * ny + nx + 1];
-        r *= (T)0.5;
+        auto pair = [&](int o) { return hi ? f[o] + f[o + 1] : f[o]; };
+        const T r = restrict_sum(pair(0), hj ? pair(nx) : (T)0, hk ? pair(nx * ny) : (T)0,
+                                 hj && hk ? pair(nx * ny + nx) : (T)0);
         b1[q] = r;
         cv[q] = (double)1.0f * (double)r;
     }
@@ -2248,7 +2275,8 @@ pppm_status MGHier<T>::smooth_colour(int l, T* x, const T* b, T bscale, int iter
     dim3 blk(64, 4), grid(div_up(div_up(nx, 2), 64), div_up(ny, 4), nz * ncomp_);
     for (int it = 0; it < iters; it++)
         for (int color = 1; color >= 0; color--) {
-            hipLaunchKernelGGL(k_rbgs<T>, grid, blk, 0, st, x, b, bscale, nx, ny, nz, cells(l), color, omega, beta);
+            hipLaunchKernelGGL(k_rbgs<T>, grid, blk, 0, st, x, b, bscale, nx, ny, nz, cells(l), color, omega, beta,
+                               omega / (T)6);
             PPPM_LAUNCH_CHECK();
         }
     return PPPM_OK;
@@ -2292,6 +2320,7 @@ pppm_status MGHier<T>::smooth(int l, T* x, const T* b, T bscale, int iters, T om
                 a.G = cells(l);
                 a.omega = omega;
                 a.beta = beta;
+                a.w6 = omega / (T)6;
                 if (beta != 0) launch_rb4<T, false, false, false, true>(a, ncomp_, st);
                 else launch_rb4<T, false, false, false, false>(a, ncomp_, st);
                 PPPM_LAUNCH_CHECK();
@@ -2366,6 +2395,7 @@ pppm_status MGHier<T>::tail(const T* xin, T* x, const T* b, T* b1, T bscale, int
     a.nu1 = nu1;
     a.nu2 = nu2;
     a.omega = omega;
+    a.w6 = omega / (T)6;
     a.tab = consistent ? tab_cons_ : tab_ref_;
     hipLaunchKernelGGL(k_vtail<T>, dim3(ncomp_), dim3(kTailThreads), 0, st, a);
     PPPM_LAUNCH_CHECK();
@@ -2400,6 +2430,7 @@ pppm_status MGHier<T>::tile(int l, const T* xin, T* x, const T* b, T bscale, int
     a.G = cells(l);
     a.omega = omega;
     a.beta = beta;
+    a.w6 = omega / (T)6;
     a.iters = iters;
     a.bn = bnext;
     a.cx = c[0];
@@ -2798,7 +2829,8 @@ pppm_status ref_rbgs(T* x, const T* b, int iters, int nx, int ny, int nz, T omeg
     const size_t G = (size_t)nx * ny * nz;
     for (int it = 0; it < iters; it++)
         for (int color = 1; color >= 0; color--) {
-            hipLaunchKernelGGL(k_rbgs<T>, grid, blk, 0, st, x, b, (T)1, nx, ny, nz, G, color, omega, (T)0);
+            hipLaunchKernelGGL(k_rbgs<T>, grid, blk, 0, st, x, b, (T)1, nx, ny, nz, G, color, omega, (T)0,
+                               omega / (T)6);
             PPPM_LAUNCH_CHECK();
         }
     return PPPM_OK;
