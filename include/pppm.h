@@ -321,11 +321,14 @@ pppm_status pppm_mg_smooth(pppm_mg *mg, void *x, const void *b, int32_t iters, d
  * passes, 0 one launch per half-sweep, residual, restriction and
  * prolongation. */
 pppm_status pppm_mg_set_blocked(pppm_mg *mg, int32_t blocked);
-/* Levels with at least this many cells per component take the blocked
- * passes in PPPM_F32 V-cycles (default 327680: 69^3 and larger); smaller ones
- * of even dimensions take tile passes (two red-black iterations with the
- * residual or the prolongation in one launch), others one launch per
- * half-sweep. */
+/* Levels of even dimensions with at least this many cells per component take
+ * the blocked passes in PPPM_F32 V-cycles (default 327680: 70^3 and larger),
+ * and those with four fifths of it (64^3) where all components together have
+ * 851968 cells or more.  Smaller levels of even dimensions with fewer than
+ * 524288 cells take tile passes (two red-black iterations with the residual or
+ * the prolongation in one launch), all others one launch per half-sweep.  The
+ * results are the same, bit for bit, whichever it is (kind 1 of
+ * pppm_mg_set_blocked apart). */
 pppm_status pppm_mg_set_blocked_min_cells(pppm_mg *mg, uint64_t cells);
 /* PPPM_F32 V-cycles: one_launch = 1 (the default) runs the level above the
  * coarsest (when it is below that threshold and has at most 4096 cells, as

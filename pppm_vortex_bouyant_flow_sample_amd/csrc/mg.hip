@@ -35,9 +35,9 @@ __device__ inline T nb_sum(const T* __restrict__ x, size_t t, int i, int j, int 
     return r;
 }
 
-// What k_rbgs, k_tile, k_vtail and (FP64) k_rb4 do to a cell, to a residual and
-// to a coarse value is written here once, with its fused multiply-adds spelt
-// out and no others, so that a level's values are bitwise the same whichever of
+// What k_rbgs, k_tile, k_vtail, k_rbc and k_rb4 do to a cell, to a residual and to
+// a coarse value is written here once, with its fused multiply-adds spelt out
+// and no others, so that a level's values are bitwise the same whichever of
 // them runs it: the choice may go by the work of all components together, and a
 // component solved with others is bitwise the one solved alone.
 __device__ inline float fma_(float a, float b, float c) { return fmaf(a, b, c); }
@@ -55,6 +55,16 @@ template <typename T>
 __device__ inline T relax(T x, T s, T b, T bscale, T w, T om1) {
 #pragma clang fp contract(off)
     return fma_(w, fma_(-bscale, b, s), om1 * x);
+}
+// the same with om1 x formed in x's register once the sum is there: the blocked
+// passes, which have few registers to spare, spill where it is formed early
+__device__ inline double relax_late(double x, double s, double b, double bscale, double w, double om1) {
+    return relax(x, s, b, bscale, w, om1);
+}
+__device__ inline float relax_late(float x, float s, float b, float bscale, float w, float om1) {
+    const float r = fmaf(-bscale, b, s);
+    __asm__("v_mul_f32 %0, %1, %0" : "+v"(x) : "s"(om1), "v"(r));
+    return fmaf(w, r, x);
 }
 // residual of a cell, s the sum of its neighbours
 template <typename T>
@@ -76,10 +86,11 @@ __device__ inline T ghost(T fi, T fj, T fk, T c) {
 #pragma clang fp contract(off)
     return ((fi * fj) * fk) * c;
 }
-// the 8 children's residuals of a coarse cell: pairs along x, then y, then z
+// the 8 children's residuals of a coarse cell, p[y][z] the sums of the pairs
+// along x: over z, then y
 template <typename T>
 __device__ inline T restrict_sum(T p00, T p10, T p01, T p11) {
-    return ((p00 + p10) + (p01 + p11)) * (T)0.5;
+    return ((p00 + p01) + (p10 + p11)) * (T)0.5;
 }
 
 template <typename T>
@@ -119,7 +130,7 @@ struct TbArgsT {
     int nx, ny, nz;
     size_t G;            // cells per component
     T omega, beta;   // SOR factor, ghost factor of this level
-    T w6;            // omega / 6 (FP64)
+    T w6, om1;       // omega / 6, 1 - omega (not k_rb2)
     int zc;              // z planes per workgroup chunk (even)
     // RESTRICT: residual restricted into bn (coarse dims cx, cy, cz = n / 2)
     T* bn;
@@ -465,7 +476,7 @@ k_rbc(TbArgs a) {
     const int klo = max(z0 - HY, 0), khi = min(z1 + HY, nz);
     const int kend = khi + S + (RESTRICT ? 1 : 0);
     const size_t plane = (size_t)nx * ny;
-    const float omega = a.omega, beta = a.beta, bscale = a.bscale;
+    const float omega = a.omega, beta = a.beta, bscale = a.bscale, w6 = a.w6;
     const int tid = threadIdx.x;
 
     for (int q = tid; q < NR * PS; q += 256) xs[q] = 0.f;
@@ -495,7 +506,7 @@ k_rbc(TbArgs a) {
         exn[u][0] = e[u] + sp - 1;
         exn[u][1] = e[u] - sp;
         gob[u] = in ? 4u * (uint32_t)(j * nx + i0) : 0u;
-        wu[u] = in ? omega : 0.f;
+        wu[u] = in ? (BETA ? omega : w6) : 0.f;
         sv[u] = valid;
         gin[u] = in;
         swp[u] = sp != 0;
@@ -603,13 +614,11 @@ k_rbc(TbArgs a) {
                             const float* cz_ = z ? cn0 : cp0;
                             const float* a0 = cz_ + rp * CLX + m;
                             const float* a1 = cz_ + rn * CLX + m;
-                            const float xe0 = 0.75f * a0[1] + 0.25f * a0[0], xo0 = 0.75f * a0[1] + 0.25f * a0[2];
-                            const float xe1 = 0.75f * a1[1] + 0.25f * a1[0], xo1 = 0.75f * a1[1] + 0.25f * a1[2];
-                            ye[z] = 0.75f * xe0 + 0.25f * xe1;
-                            yo[z] = 0.75f * xo0 + 0.25f * xo1;
+                            ye[z] = lerp_(0.25f, lerp_(0.25f, a0[1], a0[0]), lerp_(0.25f, a1[1], a1[0]));
+                            yo[z] = lerp_(0.25f, lerp_(0.25f, a0[1], a0[2]), lerp_(0.25f, a1[1], a1[2]));
                         }
-                        xv.x += 0.75f * ye[0] + 0.25f * ye[1];
-                        xv.y += 0.75f * yo[0] + 0.25f * yo[1];
+                        xv.x += lerp_(0.25f, ye[0], ye[1]);
+                        xv.y += lerp_(0.25f, yo[0], yo[1]);
                     }
                     P[ea[u][j & 1]] = xv.x;
                     P[ea[u][(j & 1) ^ 1]] = xv.y;
@@ -655,16 +664,15 @@ k_rbc(TbArgs a) {
                         if (u == NP - 1 && !sv[u]) continue;
                         const int o = e[u];
                         const float xo = xos[u];
-                        float r = fmaf(-bscale, c ? bq[jp][u].y : bq[jp][u].x, rr[u]);
-                        float d = 1.0f / 6.0f;
+                        float wq = wu[u];
                         if (BETA) {
                             const int m = o % HXP, ly = o / HXP - 1;
                             const int i = gx0 + 2 * m + ((swp[u] ? 1 : 0) ^ w), jj = gy0 + ly;
                             const int nout = (i == 0) + (i == nx - 1) + (jj == 0) + (jj == ny - 1) + (p == 0) +
                                              (p == nz - 1);
-                            d = 1.0f / (6.0f - beta * (float)nout);
+                            wq = nout == 0 ? (gin[u] ? w6 : 0.f) : wu[u] / fmaf(-beta, (float)nout, 6.f);
                         }
-                        PC[o] = xo + wu[u] * (r * d - xo);
+                        PC[o] = relax_late(xo, rr[u], c ? bq[jp][u].y : bq[jp][u].x, bscale, wq, a.om1);
                     }
                 }
                 if (t < S || kBarAfter) __syncthreads();
@@ -706,15 +714,16 @@ k_rbc(TbArgs a) {
                             float sres = PB[ox] + PB[ox + 1];
                             sres += PB[o - HXP] + PB[o + HXP];
                             sres += PM[o] + PQ[o];
-                            sres -= 6.0f * xo;
+                            int nout = 0;
                             if (BETA) {
                                 const int m = o % HXP, ly = o / HXP - 1;
                                 const int i = gx0 + 2 * m + ((swp[u] ? 1 : 0) ^ w), jj = gy0 + ly;
-                                const int nout = (i == 0) + (i == nx - 1) + (jj == 0) + (jj == ny - 1) + (pr == 0) +
-                                                 (pr == nz - 1);
-                                sres += beta * (float)nout * xo;
+                                nout = (i == 0) + (i == nx - 1) + (jj == 0) + (jj == ny - 1) + (pr == 0) +
+                                       (pr == nz - 1);
                             }
-                            part += fmaf(bscale, c ? bq[jr][u].y : bq[jr][u].x, -sres);
+                            const float r = residual_of(xo, sres, c ? bq[jr][u].y : bq[jr][u].x, bscale, nout,
+                                                        BETA ? beta : 0.f);
+                            part = c == 0 ? r : part + r;
                         }
                         if ((jr & 1) == 0) rsum[u] = part;
                         else rs[rsi[u]] = rsum[u] + part;
@@ -750,9 +759,7 @@ k_rbc(TbArgs a) {
 // exact beyond the region, which saves one.  Planes outside the grid are
 // zero and stay so, as cells outside it in x and y.  Needs nx even.
 //
-// Sums are formed in k_rbc's order; FP32 updates are k_rbc's, FP64 ones relax
-// (x + w (s d - x) rounds at the size of the x that it replaces; full multigrid
-// at 64^3 from its 80-bit evaluation: 8.5e-16, with relax 5.3e-16).  One workgroup of 16 waves a CU, bound
+// One workgroup of 16 waves a CU, bound
 // by its planes' loads and by vector issue at once.  256^3 x 3, V(2,2) (us):
 // down from zero 107 + 179 (two k_rbc passes) -> 128, up 203 + 151 -> 205;
 // 96^3 x 3: 39 -> 18, 41 -> 22.
@@ -809,7 +816,6 @@ struct R4Pair<double> {
 template <typename T, bool RESTRICT, bool PROLONG, bool XZERO, bool BETA>
 __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
     constexpr int NT = r4_threads<T>(), RG = NT / 32;  // row groups of the region
-    constexpr bool kRelax = sizeof(T) == 8;  // relax, as the kernels of smaller levels; FP32: k_rbc's form
     constexpr bool kWide = RESTRICT && !XZERO;
     constexpr int HXY = kWide ? 6 : 4, HZ = kWide ? 5 : 4;
     constexpr int TW = kR4Region - 2 * HXY, TH = 2 * RG - 2 * HXY;  // tile
@@ -857,31 +863,25 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
     const uint32_t pbytes = (uint32_t)(plane * sizeof(T));
     uint32_t lofs[2], sofs[2];
     bool gin[2];
-    T wr[2];
-    // cells outside the grid next to a cell in the plane, and the diagonal's
-    // reciprocal (kRelax: the relaxation factor) off and on the first and last
-    // plane
-    T nxy[2][2], d0[2][2], d1[2][2];
-    const T om1 = (T)1 - omega;
+    // cells outside the grid next to a cell in the plane, and its relaxation
+    // factor off and on the first and last plane (0: a cell outside the grid,
+    // which is 0 and stays so)
+    int nxy[2][2];
+    T wr[2], d0[2][2], d1[2][2];  // BETA: d0, d1
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         const int j = gy0 + 2 * rg + r, ly = 2 * rg + r;
         gin[r] = xin && j >= 0 && j < ny;
+        wr[r] = gin[r] ? a.w6 : (T)0;
         lofs[r] = gin[r] ? (uint32_t)sizeof(T) * (uint32_t)(j * nx + i0) : kOff;
-        wr[r] = gin[r] ? omega : (T)0;
         sofs[r] = ly >= HXY && ly < HXY + TH && 2 * m >= HXY && 2 * m < HXY + TW ? lofs[r] : kOff;
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int i = i0 + e;
             const int no = (i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1), noz = no + (nz == 1 ? 2 : 1);
-            nxy[r][e] = (T)no;
-            if constexpr (kRelax) {  // a cell outside the grid is 0 and stays so
-                d0[r][e] = gin[r] ? relax_weight(no, omega, BETA ? beta : (T)0, a.w6) : (T)0;
-                d1[r][e] = gin[r] ? relax_weight(noz, omega, BETA ? beta : (T)0, a.w6) : (T)0;
-            } else {
-                d0[r][e] = (T)1.0 / ((T)6.0 - beta * (T)no);
-                d1[r][e] = (T)1.0 / ((T)6.0 - beta * (T)noz);
-            }
+            nxy[r][e] = no;
+            d0[r][e] = gin[r] ? relax_weight(no, omega, beta, a.w6) : (T)0;
+            d1[r][e] = gin[r] ? relax_weight(noz, omega, beta, a.w6) : (T)0;
         }
     }
     const int gI = i0 >> 1, gJ = (gy0 >> 1) + rg;
@@ -1001,13 +1001,13 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
 #pragma unroll
                         for (int q = 0; q < 3; q++) {
                             const T* c = c0 + q * CW;
-                            xe[q] = (T)0.75 * c[1] + (T)0.25 * c[0];
-                            xo[q] = (T)0.75 * c[1] + (T)0.25 * c[2];
+                            xe[q] = lerp_((T)0.25, c[1], c[0]);
+                            xo[q] = lerp_((T)0.25, c[1], c[2]);
                         }
 #pragma unroll
                         for (int r = 0; r < 2; r++) {
-                            w[z][r][0] = (T)0.75 * xe[1] + (T)0.25 * xe[2 * r];
-                            w[z][r][1] = (T)0.75 * xo[1] + (T)0.25 * xo[2 * r];
+                            w[z][r][0] = lerp_((T)0.25, xe[1], xe[2 * r]);
+                            w[z][r][1] = lerp_((T)0.25, xo[1], xo[2 * r]);
                         }
                     }
                     const bool real = k < khi;
@@ -1015,7 +1015,7 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
                     for (int r = 0; r < 2; r++)
 #pragma unroll
                         for (int e = 0; e < 2; e++) {
-                            const T f = v[r][e] + ((T)0.75 * w[0][r][e] + (T)0.25 * w[1][r][e]);
+                            const T f = v[r][e] + lerp_((T)0.25, w[0][r][e], w[1][r][e]);
                             v[r][e] = gin[r] && real ? f : v[r][e];
                         }
                 }
@@ -1055,15 +1055,8 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
                         s += X[jm][r][e] + X[jq][r][e];
                     }
                     const T xo = X[jp][r][e];
-                    T xn;
-                    if constexpr (kRelax) {
-                        const T w = BETA && zb ? d1[r][e] : d0[r][e];
-                        xn = relax(xo, s, B[jp][r][e], bscale, in ? w : (T)0, om1);
-                    } else {
-                        s = fma_(-bscale, B[jp][r][e], s);
-                        const T d = BETA ? (zb ? d1[r][e] : d0[r][e]) : (T)1.0 / (T)6.0;
-                        xn = xo + (in ? wr[r] : (T)0) * (s * d - xo);
-                    }
+                    const T w = BETA ? (zb ? d1[r][e] : d0[r][e]) : wr[r];
+                    const T xn = relax_late(xo, s, B[jp][r][e], bscale, in ? w : (T)0, a.om1);
                     X[jp][r][e] = xn;
                     if (t < 4 || RESTRICT) ex[xslot(t, j)][r][lo + 32] = xn;
                 }
@@ -1080,7 +1073,7 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
             // 2 x 2 cells of a plane pair are one coarse cell
             if (RESTRICT) {
                 const int jr = (j + NR - 5) % NR, jm = (jr + NR - 1) % NR, jq = (jr + 1) % NR, pr = k - 5;
-                const T zb = (T)((pr == 0) + (pr == nz - 1));
+                const int zb = (pr == 0) + (pr == nz - 1);
                 T part[2];
 #pragma unroll
                 for (int r = 0; r < 2; r++) {
@@ -1092,9 +1085,8 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
                         T s = e ? other + from_right(X[jr][r][0]) : from_left(X[jr][r][1]) + other;
                         s += r ? X[jr][0][e] + yr[1][c] : yr[0][c] + X[jr][1][e];
                         s += X[jm][r][e] + X[jq][r][e];
-                        s -= (T)6.0 * xo;
-                        if (BETA) s += beta * (nxy[r][e] + zb) * xo;
-                        part[r] += fma_(bscale, B[jr][r][e], -s);
+                        const T v = residual_of(xo, s, B[jr][r][e], bscale, nxy[r][e] + zb, BETA ? beta : (T)0);
+                        part[r] = c == 0 ? v : part[r] + v;
                     }
                 }
                 if ((jr & 1) == 0) {
@@ -1105,7 +1097,7 @@ __global__ void __launch_bounds__(r4_threads<T>()) k_rb4(TbArgsT<T> a) {
                     const bool mine = pr >= z0 && pr < z1 && gK < a.cz;
                     const auto rn = buffer(bnext + (mine ? (size_t)gK * a.cy * a.cx : 0),
                                            mine ? (uint32_t)sizeof(T) * (uint32_t)(a.cy * a.cx) : 0u);
-                    const T c = ((rsum[0] + part[0]) + (rsum[1] + part[1])) * (T)0.5;
+                    const T c = restrict_sum(rsum[0], rsum[1], part[0], part[1]);
                     static_assert(!RESTRICT || sizeof(T) == 4, "the restriction stores floats");
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)c), rn, cofs, 0, 0);
                 }
@@ -2265,6 +2257,8 @@ pppm_status smooth_tb<float>(const float* xin, float* x, const float* b, float b
     a.G = G;
     a.omega = omega;
     a.beta = beta;
+    a.w6 = omega / 6.0f;
+    a.om1 = 1.0f - omega;
     a.zc = tb_zchunk(nx, ny, nz, ncomp);
     return launch_rb2<false, false, false>(a, ncomp, kind, st, two_iter);
 }
@@ -2321,6 +2315,7 @@ pppm_status MGHier<T>::smooth(int l, T* x, const T* b, T bscale, int iters, T om
                 a.omega = omega;
                 a.beta = beta;
                 a.w6 = omega / (T)6;
+                a.om1 = (T)1 - omega;
                 if (beta != 0) launch_rb4<T, false, false, false, true>(a, ncomp_, st);
                 else launch_rb4<T, false, false, false, false>(a, ncomp_, st);
                 PPPM_LAUNCH_CHECK();
@@ -2405,7 +2400,7 @@ pppm_status MGHier<T>::tail(const T* xin, T* x, const T* b, T* b1, T bscale, int
 template <typename T>
 bool MGHier<T>::tile_level(int l, bool consistent) const {
     if (!tb_ || l >= L_ - 1 || !t_[l] || cells(l) >= kTileCells) return false;
-    if (sizeof(T) == 8 ? wide_level(l) : cells(l) >= tb_min_cells_ && !(d_[l][0] & 1)) return false;  // k_rb4, k_rbc
+    if (sizeof(T) == 8 ? wide_level(l) : blocked_level(l) && !(d_[l][0] & 1)) return false;  // k_rb4, k_rbc
     for (int c = 0; c < 3; c++)
         // without the one launch of the smallest levels the one above the
         // coarsest runs a launch per half-sweep, with bitwise its results
@@ -2577,6 +2572,8 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
         a.G = m.cells(l);
         a.omega = omega;
         a.beta = (float)mg_beta(l);
+        a.w6 = omega / 6.0f;
+        a.om1 = 1.0f - omega;
         a.zc = tb_zchunk(d[0], d[1], d[2], nc);
         a.cx = c[0];
         a.cy = c[1];
@@ -2588,7 +2585,7 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
     // amortise: levels below the hierarchy's threshold run the tile passes
     // (k_tile), or with odd dimensions the one-launch-per-colour kernels in
     // place.
-    auto blocked = [&](int l) { return m.cells(l) >= m.blocked_min_cells() && m.even(l); };
+    auto blocked = [&](int l) { return m.blocked_level(l) && m.even(l); };
     // the small levels in one launch where they fit (l0 >= 1: X and B of
     // those levels are the hierarchy's own)
     const int l0 = m.tail_level();

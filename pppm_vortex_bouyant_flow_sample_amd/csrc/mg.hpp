@@ -98,7 +98,7 @@ class MGHier {
     void set_blocked_smoother(int kind) { tb_ = kind; }
     int blocked_smoother() const { return tb_; }
     // V-cycles run the blocked passes on levels with at least this many cells
-    // per component, the tile passes below
+    // per component (blocked_level), the tile passes below
     void set_blocked_min_cells(size_t n) { tb_min_cells_ = n; }
     size_t blocked_min_cells() const { return tb_min_cells_; }
     // V-cycles: the level above the coarsest and the coarsest solve in one
@@ -115,6 +115,12 @@ class MGHier {
     // FP64 (k_rb4)
     bool wide_level(int l) const {
         return sizeof(T) == 8 && tb_ && cells(l) * (size_t)ncomp_ >= kRb4Doubles && t_[l] && !(d_[l][0] & 1);
+    }
+    // whether level l of a V-cycle takes the FP32 blocked passes (if its
+    // dimensions let it)
+    bool blocked_level(int l) const {
+        const size_t n = cells(l);
+        return n >= tb_min_cells_ || (n >= tb_min_cells_ / 5 * 4 && n * (size_t)ncomp_ >= kBlockedCells);
     }
     // whether level l of a V-cycle takes the tile passes (k_tile)
     bool tile_level(int l, bool consistent) const;
@@ -141,9 +147,12 @@ class MGHier {
     static constexpr size_t kTileCells = (size_t)1 << 19;
     static constexpr size_t kTile16Cells = (size_t)1 << 19;
     // FP32 blocked passes from here (us down and up, tile against blocked: 64^3
-    // 10.4 against 13.8 and for three components 16 + 18 against 16 + 19; 72^3
-    // 17 against 14, three 26 against 16; 80^3 23 against 14, three 28 + 34
-    // against 17 + 19).
+    // 10.4 against 13.8; 72^3 17 against 14, three components 26 against 16; 80^3
+    // 23 against 14, three 28 + 34 against 17 + 19), and from four fifths of it
+    // where all components together hold kBlockedCells or more (us of four V(2,2)
+    // cycles: 64^3 x 3 265 / 274, x 6 404 / 333, x 12 597 / 431, x 48 1769 / 875;
+    // 66^3 x 1 302 / 307, x 3 396 / 341; 68^3 x 3 436 / 368).
+    static constexpr size_t kBlockedCells = (size_t)13 << 16;
     size_t tb_min_cells_ = (size_t)5 << 16;
     // FP64 levels of at least this many cells over all components take k_rb4
     // (us of a full multigrid V(4,4), tiles against k_rb4: 32^3 x 3 183 against

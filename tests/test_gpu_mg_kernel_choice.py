@@ -1,8 +1,7 @@
 """Results do not depend on which kernel a level takes.  Levels are given to
 tile passes, passes of two iterations, the small levels' one launch or launches
 per half-sweep by their size, the number of components and a switch; all of them
-but the FP32 blocked passes (whose line goes by a component's cells) do the same
-arithmetic, so the results are compared bitwise."""
+do the same arithmetic, so the results are compared bitwise."""
 import numpy as np
 import pytest
 
@@ -30,6 +29,8 @@ def _cycles(native, dims, dtype, b, x0, nu, sched, omega, small=True):
                           ((33, 35, 31), 7, 2, (2, 2), "vcycle"),   # odd levels
                           ((64, 64, 64), 3, 1, (2, 2), "vcycle"),   # tiles of 8^3 alone, of 16^3 together
                           ((50, 68, 62), 4, 1, (2, 1), "vcycle"),   # ... that the grid does not fill
+                          ((64, 64, 64), 4, 1, (2, 1), "vcycle"),   # together in blocked passes
+                          ((66, 64, 68), 3, 1, (1, 2), "vcycle"),
                           ((32, 32, 32), 48, 1, (2, 2), "vcycle")])
 def test_component_equals_alone(native, dims, ncomp, dtype, nu, sched):
     t = np.float64 if dtype == native.F64 else np.float32
@@ -42,6 +43,29 @@ def test_component_equals_alone(native, dims, ncomp, dtype, nu, sched):
     for c in {0, ncomp // 2, ncomp - 1}:
         alone = _cycles(native, dims, dtype, b[c:c + 1], x0[c:c + 1], nu, sched, 1.15)
         np.testing.assert_array_equal(both[c], alone[0])
+
+
+@pytest.mark.parametrize("dims,nu", [((64, 64, 64), (2, 2)), ((64, 64, 64), (1, 1)), ((96, 72, 80), (2, 1)),
+                                     ((80, 112, 72), (1, 2)), ((128, 64, 64), (2, 2))])
+def test_blocked_kinds_equal_half_sweeps(native, dims, nu):
+    """FP32 V-cycles of one launch per half-sweep and in blocked passes (kinds 2
+    to 4) and tiles, three components."""
+    rng = np.random.default_rng(sum(dims))
+    shape = (3, int(np.prod(dims)))
+    b, x0 = rng.standard_normal(shape).astype(np.float32), rng.standard_normal(shape).astype(np.float32)
+    out = []
+    for kind in (0, 2, 3, 4):
+        print(f"[mg choice] dims={dims} nu={nu} kind={kind}", flush=True)
+        mg = native.MG(dims, native.F32, ncomp=3)
+        mg.set_blocked(kind)
+        if kind == 3:
+            mg.set_blocked_min_cells(1)  # every level above the coarsest two
+        bx, bb = native.DeviceBuffer.from_array(x0), native.DeviceBuffer.from_array(b)
+        mg.vcycles(bx.ptr, bb.ptr, 2, nu[0], nu[1], 1.15)
+        native.synchronize()
+        out.append(bx.to_array(np.float32, b.size))
+    for o in out[1:]:
+        np.testing.assert_array_equal(o, out[0])
 
 
 @pytest.mark.parametrize("dims", [(16, 16, 16), (12, 20, 14), (2, 1024, 2), (22, 22, 22), (32, 32, 32)])
