@@ -2401,6 +2401,7 @@ template <typename T>
 bool MGHier<T>::tile_level(int l, bool consistent) const {
     if (!tb_ || l >= L_ - 1 || !t_[l] || cells(l) >= kTileCells) return false;
     if (sizeof(T) == 8 ? wide_level(l) : blocked_level(l) && !(d_[l][0] & 1)) return false;  // k_rb4, k_rbc
+    if (sizeof(T) == 8 && (d_[l][0] & 1) && cells(l) * (size_t)ncomp_ >= kOddTileDoubles) return false;
     for (int c = 0; c < 3; c++)
         // without the one launch of the smallest levels the one above the
         // coarsest runs a launch per half-sweep, with bitwise its results

@@ -159,6 +159,13 @@ class MGHier {
     // 205, 48^3 289 against 302, 40^3 x 3 336 against 301, 56^3 355 against 325,
     // 64^3 374 against 338, 64^3 x 3 598 against 388).
     static constexpr size_t kRb4Doubles = (size_t)1 << 17;
+    // FP64 levels with odd nx, which k_rb4 does not take, run a launch per
+    // half-sweep from this many cells over all components, as their tiles
+    // recompute more of the halo than the launches cost (us of two full
+    // multigrid solves V(4,4), tiles / launches: 71^3 468 / 560, x 2 629 / 697,
+    // x 3 842 / 834; 63^3 x 2 474 / 480, x 6 980 / 729; 45^3 x 12 828 / 700; 65^3
+    // x 12 2050 / 1365).
+    static constexpr size_t kOddTileDoubles = (size_t)3 << 18;
     bool tail_ = true;
 };
 
