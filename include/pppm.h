@@ -322,13 +322,14 @@ pppm_status pppm_mg_smooth(pppm_mg *mg, void *x, const void *b, int32_t iters, d
  * prolongation. */
 pppm_status pppm_mg_set_blocked(pppm_mg *mg, int32_t blocked);
 /* Levels of even dimensions with at least this many cells per component take
- * the blocked passes in PPPM_F32 V-cycles (default 327680: 70^3 and larger),
- * and those with four fifths of it (64^3) where all components together have
- * 851968 cells or more.  Smaller levels of even dimensions with fewer than
- * 524288 cells take tile passes (two red-black iterations with the residual or
- * the prolongation in one launch), all others one launch per half-sweep.  The
- * results are the same, bit for bit, whichever it is (kind 1 of
- * pppm_mg_set_blocked apart). */
+ * the blocked passes in PPPM_F32 V-cycles (default 327680: 70^3 and larger);
+ * at that default also smaller ones where the components together keep the
+ * chip busy (from 851968 cells, or 294912 where tiles would be filled badly).
+ * Other levels of even dimensions with fewer than 524288 cells take tile
+ * passes (two red-black iterations with the residual or the prolongation in
+ * one launch) unless a dimension is below 8 and the components hold 98304
+ * cells or more; all others one launch per half-sweep.  The results are the
+ * same, bit for bit, whichever it is (kind 1 of pppm_mg_set_blocked apart). */
 pppm_status pppm_mg_set_blocked_min_cells(pppm_mg *mg, uint64_t cells);
 /* PPPM_F32 V-cycles: one_launch = 1 (the default) runs the level above the
  * coarsest (when it is below that threshold and has at most 4096 cells, as

@@ -43,8 +43,8 @@ __device__ inline T nb_sum(const T* __restrict__ x, size_t t, int i, int j, int 
 __device__ inline float fma_(float a, float b, float c) { return fmaf(a, b, c); }
 __device__ inline double fma_(double a, double b, double c) { return fma(a, b, c); }
 // relaxation factor over the diagonal 6 - beta nout of a cell with nout
-// neighbours outside and a ghost factor beta; w6 = omega / 6 (the host's: a
-// division a thread made k_rbgs<double> 2% slower)
+// neighbours outside and a ghost factor beta; w6 = omega / 6 (from the
+// host: a division a thread made k_rbgs<double> 2% slower)
 template <typename T>
 __device__ inline T relax_weight(int nout, T omega, T beta, T w6) {
     return beta == (T)0 || nout == 0 ? w6 : omega / fma_(-beta, (T)nout, (T)6);
@@ -93,20 +93,11 @@ __device__ inline T restrict_sum(T p00, T p10, T p01, T p11) {
     return ((p00 + p01) + (p10 + p11)) * (T)0.5;
 }
 
-template <typename T>
-__device__ inline void rbgs_point(T* xc, T bv, T bscale, int i, int j, int k, int nx, int ny, int nz, T omega,
-                                  T beta, T w6) {
-    const size_t t = ((size_t)k * ny + j) * nx + i;
-    int nout;
-    const T s = nb_sum(xc, t, i, j, k, nx, ny, nz, nout);
-    xc[t] = relax(xc[t], s, bv, bscale, relax_weight(nout, omega, beta, w6), (T)1 - omega);
-}
-
 // One colour of red-black SOR.  color 1 = (i+j+k) odd (swept first, as the
-// reference's "red" kernel), 0 = even.
-template <typename T>
-__global__ void __launch_bounds__(256) k_rbgs(T* __restrict__ x, const T* __restrict__ b, T bscale, int nx, int ny,
-                                              int nz, size_t G, int color, T omega, T beta, T w6) {
+// reference's "red" kernel), 0 = even.  BETA: a ghost factor that is not zero.
+template <typename T, bool BETA>
+__global__ void __launch_bounds__(256) k_rbgs(T* __restrict__ x, const T* __restrict__ b, size_t G, int nx, int ny,
+                                              int nz, int color, T bscale, T w6, T om1, T omega, T beta) {
     const int i2 = blockIdx.x * 64 + threadIdx.x;
     const int j = blockIdx.y * 4 + threadIdx.y;
     const int comp = blockIdx.z / nz, k = blockIdx.z - comp * nz;
@@ -114,7 +105,23 @@ __global__ void __launch_bounds__(256) k_rbgs(T* __restrict__ x, const T* __rest
     const int i = 2 * i2 + ((j + k + color) & 1);
     if (i >= nx) return;
     const size_t t = ((size_t)k * ny + j) * nx + i;
-    rbgs_point(x + (size_t)comp * G, b[(size_t)comp * G + t], bscale, i, j, k, nx, ny, nz, omega, beta, w6);
+    T* xc = x + (size_t)comp * G;
+    int nout;
+    const T s = nb_sum(xc, t, i, j, k, nx, ny, nz, nout);
+    xc[t] = relax(xc[t], s, b[(size_t)comp * G + t], bscale, BETA ? relax_weight(nout, omega, beta, w6) : w6, om1);
+}
+
+// one colour of ncomp components
+template <typename T>
+static void launch_rbgs(T* x, const T* b, T bscale, int nx, int ny, int nz, int ncomp, int color, T omega, T beta,
+                        hipStream_t st) {
+    dim3 blk(64, 4), grid(div_up(div_up(nx, 2), 64), div_up(ny, 4), nz * ncomp);
+    const size_t G = (size_t)nx * ny * nz;
+    const T w6 = omega / (T)6, om1 = (T)1 - omega;
+    if (beta != (T)0)
+        hipLaunchKernelGGL((k_rbgs<T, true>), grid, blk, 0, st, x, b, G, nx, ny, nz, color, bscale, w6, om1, omega, beta);
+    else
+        hipLaunchKernelGGL((k_rbgs<T, false>), grid, blk, 0, st, x, b, G, nx, ny, nz, color, bscale, w6, om1, omega, beta);
 }
 
 // Tile of the blocked smoother k_rb2 (below): 64 x 16 cells per workgroup.
@@ -1558,20 +1565,25 @@ struct TailArgs {
 // Level l0 in LDS by colours, as a tile of k_tile with the whole level as its
 // region: pair (m, y) of plane z at index ((z + 1) (ny + 2) + y + 1) (hx + 1) +
 // m + 1 of each colour, hx = ceil(nx / 2), zeros around.
-constexpr int kTailLds = 4096;
+// Values of a colour that LDS holds: in FP32 those of whatever shape stands two
+// levels above nothing but the coarsest ((1, 1024, 4): 2 x 1026 x 6), in FP64 of
+// the usual ones.
+template <typename T>
+constexpr int tail_lds() { return sizeof(T) == 4 ? 12320 : 4096; }
 inline int tail_pairs(const int* d) { return ((d[0] + 1) / 2 + 1) * (d[1] + 2) * (d[2] + 2) + 1; }
 // the fit test of level l0 (host side): thread t owns column (m, y) = t mod P
 // (P = hx ny columns) at kq = ceil(nz / (threads / P)) planes
+template <typename T>
 inline bool tail_fits(const int* d) {
     const int P = ((d[0] + 1) / 2) * d[1];
-    if (P > kTailThreads || tail_pairs(d) > kTailLds) return false;
+    if (P > kTailThreads || tail_pairs(d) > tail_lds<T>()) return false;
     const int R = kTailThreads / P;
     return (d[2] + R - 1) / R <= kTailPairs;
 }
 
 template <typename T>
 __global__ void __launch_bounds__(kTailThreads) k_vtail(TailArgs<T> a) {
-    __shared__ T xa[2][kTailLds];
+    __shared__ T xa[2][tail_lds<T>()];
     __shared__ T rs[kTailMax];  // residuals of level l0, in grid order
     __shared__ T xc[512];
     __shared__ double cv[512], cw[512], ltab[kCoarseTab];
@@ -1974,7 +1986,7 @@ template <typename T>
 bool MGHier<T>::has_temp(const int (*d)[3], int L, int l) {
     if (sizeof(T) == 4) return true;
     const size_t n = (size_t)d[l][0] * d[l][1] * d[l][2];
-    const bool tail = l == L - 2 && L >= 3 && n <= (size_t)kTailMax && tail_fits(d[l]);
+    const bool tail = l == L - 2 && L >= 3 && n <= (size_t)kTailMax && tail_fits<T>(d[l]);
     return n <= (size_t)1 << 24 && l < L - 1 && !tail;
 }
 
@@ -2265,12 +2277,9 @@ pppm_status smooth_tb<float>(const float* xin, float* x, const float* b, float b
 
 template <typename T>
 pppm_status MGHier<T>::smooth_colour(int l, T* x, const T* b, T bscale, int iters, T omega, T beta, hipStream_t st) {
-    const int nx = d_[l][0], ny = d_[l][1], nz = d_[l][2];
-    dim3 blk(64, 4), grid(div_up(div_up(nx, 2), 64), div_up(ny, 4), nz * ncomp_);
     for (int it = 0; it < iters; it++)
         for (int color = 1; color >= 0; color--) {
-            hipLaunchKernelGGL(k_rbgs<T>, grid, blk, 0, st, x, b, bscale, nx, ny, nz, cells(l), color, omega, beta,
-                               omega / (T)6);
+            launch_rbgs(x, b, bscale, d_[l][0], d_[l][1], d_[l][2], ncomp_, color, omega, beta, st);
             PPPM_LAUNCH_CHECK();
         }
     return PPPM_OK;
@@ -2363,7 +2372,7 @@ int MGHier<T>::tail_level() const {
     if (!tb_ || !tail_ || L_ < 3) return -1;
     // the level above the coarsest, below the blocked levels
     const int l0 = L_ - 2;
-    if (cells(l0) >= tb_min_cells_ || cells(l0) > (size_t)kTailMax || cells(L_ - 1) > 512 || !tail_fits(d_[l0]))
+    if (cells(l0) >= tb_min_cells_ || cells(l0) > (size_t)kTailMax || cells(L_ - 1) > 512 || !tail_fits<T>(d_[l0]))
         return -1;
     return l0;
 }
@@ -2398,10 +2407,28 @@ pppm_status MGHier<T>::tail(const T* xin, T* x, const T* b, T* b1, T bscale, int
 }
 
 template <typename T>
+bool MGHier<T>::blocked_level(int l) const {
+    const size_t n = cells(l), all = n * (size_t)ncomp_;
+    if (n >= tb_min_cells_) return true;
+    if (tb_ < 2 || tb_min_cells_ > kBlockedMin) return false;
+    if (n >= tb_min_cells_ / 5 * 4 && (all >= kBlockedCells || thin(l))) return true;
+    if (thin(l) || d_[l][0] < 20) return false;  // regions of 64 cells along x
+    if (all >= kBlockedCells) return true;
+    // tiles that the level fills badly: by a quarter more cells than it has,
+    // three fifths for those of 16^3
+    const int TI = tile_size(l);
+    size_t in_tiles = 1;
+    for (int c = 0; c < 3; c++) in_tiles *= (size_t)((d_[l][c] + TI - 1) / TI * TI);
+    return all >= kBlockedPartial && (TI == 8 ? in_tiles * 4 >= n * 5 : in_tiles * 5 >= n * 8);
+}
+
+template <typename T>
 bool MGHier<T>::tile_level(int l, bool consistent) const {
     if (!tb_ || l >= L_ - 1 || !t_[l] || cells(l) >= kTileCells) return false;
     if (sizeof(T) == 8 ? wide_level(l) : blocked_level(l) && !(d_[l][0] & 1)) return false;  // k_rb4, k_rbc
     if (sizeof(T) == 8 && (d_[l][0] & 1) && cells(l) * (size_t)ncomp_ >= kOddTileDoubles) return false;
+    // thin levels leave most of a tile empty
+    if (sizeof(T) == 4 && thin(l) && cells(l) * (size_t)ncomp_ >= kThinCells) return false;
     for (int c = 0; c < 3; c++)
         // without the one launch of the smallest levels the one above the
         // coarsest runs a launch per half-sweep, with bitwise its results
@@ -2439,8 +2466,8 @@ pppm_status MGHier<T>::tile(int l, const T* xin, T* x, const T* b, T bscale, int
     // 16^3 tiles recompute less halo (26^3 cells against 18^3 for an eighth
     // of the tile) where they still fill the chip; doubles of them do not fit
     // LDS with a second workgroup
-    const bool big = std::is_same<T, float>::value && cells(l) * (size_t)ncomp_ >= kTile16Cells;
-    const int TI = big ? 16 : 8;
+    const int TI = tile_size(l);
+    const bool big = TI == 16;
     a.tx = (d[0] + TI - 1) / TI;
     a.ty = (d[1] + TI - 1) / TI;
     a.tz = (d[2] + TI - 1) / TI;
@@ -2587,6 +2614,12 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
     // (k_tile), or with odd dimensions the one-launch-per-colour kernels in
     // place.
     auto blocked = [&](int l) { return m.blocked_level(l) && m.even(l); };
+    // smoothing where odd dimensions keep the transfers apart: out of place where
+    // the level is large enough for blocked passes, which ask for an even nx only
+    auto sweeps = [&](int l, float bs, int nu, float beta) {
+        return m.blocked_level(l) && m.dims(l)[0] % 2 == 0 ? m.smooth(l, X[l], B[l], bs, nu, omega, beta, st)
+                                                            : m.smooth_colour(l, X[l], B[l], bs, nu, omega, beta, st);
+    };
     // the small levels in one launch where they fit (l0 >= 1: X and B of
     // those levels are the hierarchy's own)
     const int l0 = m.tail_level();
@@ -2606,7 +2639,7 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
         if (!blocked(l)) {
             const float bs = l == 0 ? bscale0 : 1.0f, beta = (float)mg_beta(l);
             if ((l > 0 || x0_zero) && (s = m.fill(X[l], m.cells(l) * nc, st)) != PPPM_OK) return s;
-            if ((s = m.smooth_colour(l, X[l], B[l], bs, nu1, omega, beta, st)) != PPPM_OK) return s;
+            if ((s = sweeps(l, bs, nu1, beta)) != PPPM_OK) return s;
             if ((s = m.residual_restrict(l, X[l], B[l], bs, beta, B[l + 1], st)) != PPPM_OK) return s;
             cur[l] = X[l];
             continue;
@@ -2651,7 +2684,7 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
             const float bs = l == 0 ? bscale0 : 1.0f, beta = (float)mg_beta(l);
             if ((s = m.prolong(l, X[l], X[l + 1], PROLONG_TRILINEAR, (float)mg_beta(l + 1), st)) != PPPM_OK)
                 return s;
-            if ((s = m.smooth_colour(l, X[l], B[l], bs, nu2, omega, beta, st)) != PPPM_OK) return s;
+            if ((s = sweeps(l, bs, nu2, beta)) != PPPM_OK) return s;
             continue;
         }
         float* src = cur[l];
@@ -2823,12 +2856,9 @@ __global__ void __launch_bounds__(256) k_restrict_full(T* __restrict__ bc, const
 
 template <typename T>
 pppm_status ref_rbgs(T* x, const T* b, int iters, int nx, int ny, int nz, T omega, hipStream_t st) {
-    dim3 blk(64, 4), grid(div_up(div_up(nx, 2), 64), div_up(ny, 4), nz);
-    const size_t G = (size_t)nx * ny * nz;
     for (int it = 0; it < iters; it++)
         for (int color = 1; color >= 0; color--) {
-            hipLaunchKernelGGL(k_rbgs<T>, grid, blk, 0, st, x, b, (T)1, nx, ny, nz, G, color, omega, (T)0,
-                               omega / (T)6);
+            launch_rbgs(x, b, (T)1, nx, ny, nz, 1, color, omega, (T)0, st);
             PPPM_LAUNCH_CHECK();
         }
     return PPPM_OK;

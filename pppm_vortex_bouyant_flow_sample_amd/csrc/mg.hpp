@@ -118,9 +118,12 @@ class MGHier {
     }
     // whether level l of a V-cycle takes the FP32 blocked passes (if its
     // dimensions let it)
-    bool blocked_level(int l) const {
-        const size_t n = cells(l);
-        return n >= tb_min_cells_ || (n >= tb_min_cells_ / 5 * 4 && n * (size_t)ncomp_ >= kBlockedCells);
+    bool blocked_level(int l) const;
+    // a dimension of fewer than 8 cells
+    bool thin(int l) const { return d_[l][0] < 8 || d_[l][1] < 8 || d_[l][2] < 8; }
+    // edge of level l's tiles
+    int tile_size(int l) const {
+        return sizeof(T) == 4 && cells(l) * (size_t)ncomp_ >= kTile16Cells ? 16 : 8;
     }
     // whether level l of a V-cycle takes the tile passes (k_tile)
     bool tile_level(int l, bool consistent) const;
@@ -146,14 +149,22 @@ class MGHier {
     // kTile16Cells cells over all components.
     static constexpr size_t kTileCells = (size_t)1 << 19;
     static constexpr size_t kTile16Cells = (size_t)1 << 19;
-    // FP32 blocked passes from here (us down and up, tile against blocked: 64^3
-    // 10.4 against 13.8; 72^3 17 against 14, three components 26 against 16; 80^3
-    // 23 against 14, three 28 + 34 against 17 + 19), and from four fifths of it
-    // where all components together hold kBlockedCells or more (us of four V(2,2)
-    // cycles: 64^3 x 3 265 / 274, x 6 404 / 333, x 12 597 / 431, x 48 1769 / 875;
-    // 66^3 x 1 302 / 307, x 3 396 / 341; 68^3 x 3 436 / 368).
-    static constexpr size_t kBlockedCells = (size_t)13 << 16;
-    size_t tb_min_cells_ = (size_t)5 << 16;
+    // FP32 blocked passes (blocked_level) from kBlockedMin cells (us down and up,
+    // tile against blocked: 64^3 10.4 against 13.8; 72^3 17 against 14, three
+    // components 26 against 16), and below where the components together keep
+    // the chip busy, as the tiles recompute more of their halo: from
+    // kBlockedCells over all of them, or kBlockedPartial where the level fills its
+    // tiles badly (us of four V(2,2) cycles, tile / blocked: 64^3 x 3 265 / 274,
+    // x 6 404 / 333, x 48 1769 / 875; 52^3 x 6 449 / 308, x 3 302 / 254; 40^3 x 3
+    // 196 / 231, x 12 325 / 246; 34^3 x 12 296 / 230).
+    static constexpr size_t kBlockedMin = (size_t)5 << 16;
+    static constexpr size_t kBlockedCells = (size_t)13 << 16, kBlockedPartial = (size_t)9 << 15;
+    size_t tb_min_cells_ = kBlockedMin;
+    // Levels with a dimension below 8 take no FP32 tiles from this many cells over
+    // all components (us, tiles / a launch per half-sweep: 86 x 4 x 52 x 48 394 /
+    // 315; 98 x 2 x 44 x 24 252 / 182; 64 x 64 x 2 x 12 127 / 116; below 98K tiles
+    // are the faster).
+    static constexpr size_t kThinCells = (size_t)3 << 15;
     // FP64 levels of at least this many cells over all components take k_rb4
     // (us of a full multigrid V(4,4), tiles against k_rb4: 32^3 x 3 183 against
     // 205, 48^3 289 against 302, 40^3 x 3 336 against 301, 56^3 355 against 325,

@@ -31,6 +31,8 @@ def _cycles(native, dims, dtype, b, x0, nu, sched, omega, small=True):
                           ((50, 68, 62), 4, 1, (2, 1), "vcycle"),   # ... that the grid does not fill
                           ((64, 64, 64), 4, 1, (2, 1), "vcycle"),   # together in blocked passes
                           ((66, 64, 68), 3, 1, (1, 2), "vcycle"),
+                          ((34, 34, 34), 12, 1, (1, 1), "vcycle"),  # ... as they fill their tiles badly
+                          ((64, 64, 2), 12, 1, (2, 2), "vcycle"),   # thin: half-sweeps together
                           ((32, 32, 32), 48, 1, (2, 2), "vcycle")])
 def test_component_equals_alone(native, dims, ncomp, dtype, nu, sched):
     t = np.float64 if dtype == native.F64 else np.float32
@@ -68,7 +70,8 @@ def test_blocked_kinds_equal_half_sweeps(native, dims, nu):
         np.testing.assert_array_equal(o, out[0])
 
 
-@pytest.mark.parametrize("dims", [(16, 16, 16), (12, 20, 14), (2, 1024, 2), (22, 22, 22), (32, 32, 32)])
+@pytest.mark.parametrize("dims", [(16, 16, 16), (12, 20, 14), (2, 1024, 2), (22, 22, 22), (32, 32, 32), (5, 139, 57),
+                                  (1, 2, 2048)])
 def test_small_levels_switch_without_the_one_launch(native, dims):
     """pppm_mg_set_small_levels changes no bit where the one launch does not
     apply either: two levels (16^3 above 8^3), or one it cannot hold."""
