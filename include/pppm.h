@@ -328,8 +328,9 @@ pppm_status pppm_mg_set_blocked(pppm_mg *mg, int32_t blocked);
  * Other levels of even dimensions with fewer than 524288 cells take tile
  * passes (two red-black iterations with the residual or the prolongation in
  * one launch) unless a dimension is below 8 and the components hold 98304
- * cells or more; all others one launch per half-sweep.  The results are the
- * same, bit for bit, whichever it is (kind 1 of pppm_mg_set_blocked apart). */
+ * cells or more; all others one launch per half-sweep or, with odd
+ * dimensions, the blocked smoothing alone.  The results are the same, bit for
+ * bit, whichever it is. */
 pppm_status pppm_mg_set_blocked_min_cells(pppm_mg *mg, uint64_t cells);
 /* PPPM_F32 V-cycles: one_launch = 1 (the default) runs the level above the
  * coarsest (when it is below that threshold and has at most 4096 cells, as

@@ -35,7 +35,7 @@ __device__ inline T nb_sum(const T* __restrict__ x, size_t t, int i, int j, int 
     return r;
 }
 
-// What k_rbgs, k_tile, k_vtail, k_rbc and k_rb4 do to a cell, to a residual and to
+// What k_rbgs, k_tile, k_vtail, k_rb2, k_rbc and k_rb4 do to a cell, to a residual and to
 // a coarse value is written here once, with its fused multiply-adds spelt out
 // and no others, so that a level's values are bitwise the same whichever of
 // them runs it: the choice may go by the work of all components together, and a
@@ -137,7 +137,7 @@ struct TbArgsT {
     int nx, ny, nz;
     size_t G;            // cells per component
     T omega, beta;   // SOR factor, ghost factor of this level
-    T w6, om1;       // omega / 6, 1 - omega (not k_rb2)
+    T w6, om1;       // omega / 6, 1 - omega
     int zc;              // z planes per workgroup chunk (even)
     // RESTRICT: residual restricted into bn (coarse dims cx, cy, cz = n / 2)
     T* bn;
@@ -165,13 +165,13 @@ __device__ inline float tb_prolong_lds(const float (*cw)[CLY][CLX], int i, int j
     if (nk < 0 || nk > cz - 1) { nk = pk; fk = betac; }
     const int sp = pk % 3, sn = nk % 3;
     const int ip = pi - cx0, in_ = ni - cx0, jp = pj - cy0, jn = nj - cy0;
-    const float p0 = 0.75f * cw[sp][jp][ip] + 0.25f * fi * cw[sp][jp][in_];
-    const float p1 = 0.75f * cw[sp][jn][ip] + 0.25f * fi * cw[sp][jn][in_];
-    const float p2 = 0.75f * cw[sn][jp][ip] + 0.25f * fi * cw[sn][jp][in_];
-    const float p3 = 0.75f * cw[sn][jn][ip] + 0.25f * fi * cw[sn][jn][in_];
-    const float q0 = 0.75f * p0 + 0.25f * fj * p1;
-    const float q1 = 0.75f * p2 + 0.25f * fj * p3;
-    return 0.75f * q0 + 0.25f * fk * q1;
+    // the parent's or the neighbour's value on each axis
+    auto C = [&](bool x, bool y, bool z) {
+        return ghost(x ? fi : 1.f, y ? fj : 1.f, z ? fk : 1.f, cw[z ? sn : sp][y ? jn : jp][x ? in_ : ip]);
+    };
+    const float p0 = lerp_(0.25f, C(0, 0, 0), C(1, 0, 0)), p1 = lerp_(0.25f, C(0, 1, 0), C(1, 1, 0));
+    const float p2 = lerp_(0.25f, C(0, 0, 1), C(1, 0, 1)), p3 = lerp_(0.25f, C(0, 1, 1), C(1, 1, 1));
+    return lerp_(0.25f, lerp_(0.25f, p0, p1), lerp_(0.25f, p2, p3));
 }
 
 // Blocked red-black smoother: one red-black iteration (two half-sweeps) per
@@ -292,7 +292,7 @@ __global__ void __launch_bounds__(256) k_rb2(TbArgs a) {
     }
     fetch(klo);
     __syncthreads();  // zeroed rings before the first stores
-    float rsum = 0.f;  // RESTRICT: this thread's coarse cell, partial over a plane pair
+    float rsum[2] = {0.f, 0.f};  // RESTRICT: this thread's coarse cell, its rows of the even plane
     for (int k = klo; k < khi + 2 + (RESTRICT ? 1 : 0); k++) {
         if (PROLONG) {
             if (k < khi && k > klo && (k & 1) == 0) store_coarse((k >> 1) + 1);  // fetched during plane k - 1
@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(256) k_rb2(TbArgs a) {
                             xv += tb_prolong_lds<CLX, CLY>(cw, i, j, k, cx0, cy0, a.cx, a.cy, a.cz, a.betac);
                     }
                     xr[ly * LXP + lx] = xv;
-                    br[ly * LXP + lx] = a.bscale * pb[u];
+                    br[ly * LXP + lx] = pb[u];
                 }
             }
         }
@@ -346,15 +346,13 @@ __global__ void __launch_bounds__(256) k_rb2(TbArgs a) {
                     float r = x0[o - 1] + x0[o + 1];
                     r += x0[o - LXP] + x0[o + LXP];
                     r += (zlo ? 0.f : xm[o]) + (zhi ? 0.f : xp[o]);
-                    r -= b0[o];
-                    const float xo = x0[o];
-                    float d = 1.0f / 6.0f;
+                    float w = a.w6;
                     if (BETA) {
                         const int i = gx0 + lx, j = gy0 + ly;
                         const int nout = (i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1) + zlo + zhi;
-                        d = 1.0f / (6.0f - beta * (float)nout);
+                        w = relax_weight(nout, omega, beta, a.w6);
                     }
-                    x0[o] = xo + omega * (r * d - xo);
+                    x0[o] = relax(x0[o], r, b0[o], a.bscale, w, a.om1);
                 }
             }
             __syncthreads();
@@ -380,7 +378,7 @@ __global__ void __launch_bounds__(256) k_rb2(TbArgs a) {
                 const float* xp = xs + ((pr + 1) % NR) * PL;
                 const float* b0 = bs + (pr % NB) * PL;
                 const bool zlo = pr == 0, zhi = pr == nz - 1;
-                float part = 0.f;
+                float part[2] = {0.f, 0.f};  // the two rows
 #pragma unroll
                 for (int dj = 0; dj < 2; dj++)
 #pragma unroll
@@ -389,23 +387,21 @@ __global__ void __launch_bounds__(256) k_rb2(TbArgs a) {
                         const int i = gx0 + lx, j = gy0 + ly;
                         if (i >= nx || j >= ny) continue;
                         const int o = ly * LXP + lx;
-                        const float xo = x0[o];
                         float sres = x0[o - 1] + x0[o + 1];
                         sres += x0[o - LXP] + x0[o + LXP];
                         sres += (zlo ? 0.f : xm[o]) + (zhi ? 0.f : xp[o]);
-                        sres -= 6.0f * xo;
-                        if (BETA) {
-                            const int nout = (i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1) + zlo + zhi;
-                            sres += beta * (float)nout * xo;
-                        }
-                        part += b0[o] - sres;
+                        const int nout = BETA ? (i == 0) + (i == nx - 1) + (j == 0) + (j == ny - 1) + zlo + zhi : 0;
+                        const float r = residual_of(x0[o], sres, b0[o], a.bscale, nout, BETA ? beta : 0.f);
+                        part[dj] = di == 0 ? r : part[dj] + r;
                     }
                 if ((pr & 1) == 0) {
-                    rsum = part;
+                    rsum[0] = part[0];
+                    rsum[1] = part[1];
                 } else {
                     const int gI = bx * (kTbTX / 2) + I, gJ = by * (kTbTY / 2) + J, gK = pr / 2;
                     if (gI < a.cx && gJ < a.cy && gK < a.cz)
-                        a.bn[(size_t)comp * a.Gc + ((size_t)gK * a.cy + gJ) * a.cx + gI] = (rsum + part) * 0.5f;
+                        a.bn[(size_t)comp * a.Gc + ((size_t)gK * a.cy + gJ) * a.cx + gI] =
+                            restrict_sum(rsum[0], rsum[1], part[0], part[1]);
                 }
             }
             // the next load reuses the ring slots of planes pr - 1 (x) and pr (b)
@@ -2614,11 +2610,17 @@ pppm_status vcycle_fused<float>(MGHier<float>& m, std::vector<float*>& X, std::v
     // (k_tile), or with odd dimensions the one-launch-per-colour kernels in
     // place.
     auto blocked = [&](int l) { return m.blocked_level(l) && m.even(l); };
-    // smoothing where odd dimensions keep the transfers apart: out of place where
-    // the level is large enough for blocked passes, which ask for an even nx only
+    // smoothing where odd dimensions keep the transfers apart: two iterations out
+    // of place on levels large enough for blocked passes; one (copied back), and
+    // any for odd nx (k_rb2), on a large level with many components only (us of
+    // four V(2,2) cycles, a launch per half-sweep / k_rb2: 145 x 13 x 191 x 12 1278 /
+    // 1027, 129 x 145 x 26 x 24 2539 / 1883; 65^3 x 12 842 / 887)
     auto sweeps = [&](int l, float bs, int nu, float beta) {
-        return m.blocked_level(l) && m.dims(l)[0] % 2 == 0 ? m.smooth(l, X[l], B[l], bs, nu, omega, beta, st)
-                                                            : m.smooth_colour(l, X[l], B[l], bs, nu, omega, beta, st);
+        const size_t n = m.cells(l);
+        const bool pass = (nu == 2 && m.dims(l)[0] % 2 == 0 && m.blocked_level(l)) ||
+                          (n >= m.blocked_min_cells() / 5 * 4 && n * nc >= (size_t)1 << 22);
+        return pass ? m.smooth(l, X[l], B[l], bs, nu, omega, beta, st)
+                    : m.smooth_colour(l, X[l], B[l], bs, nu, omega, beta, st);
     };
     // the small levels in one launch where they fit (l0 >= 1: X and B of
     // those levels are the hierarchy's own)

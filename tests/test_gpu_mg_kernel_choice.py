@@ -33,6 +33,8 @@ def _cycles(native, dims, dtype, b, x0, nu, sched, omega, small=True):
                           ((66, 64, 68), 3, 1, (1, 2), "vcycle"),
                           ((34, 34, 34), 12, 1, (1, 1), "vcycle"),  # ... as they fill their tiles badly
                           ((64, 64, 2), 12, 1, (2, 2), "vcycle"),   # thin: half-sweeps together
+                          ((38, 54, 141), 3, 1, (2, 2), "vcycle"),  # odd nz: smoothing alone out of place
+                          ((65, 66, 68), 16, 1, (2, 1), "vcycle"),  # odd nx
                           ((32, 32, 32), 48, 1, (2, 2), "vcycle")])
 def test_component_equals_alone(native, dims, ncomp, dtype, nu, sched):
     t = np.float64 if dtype == native.F64 else np.float32
@@ -50,13 +52,13 @@ def test_component_equals_alone(native, dims, ncomp, dtype, nu, sched):
 @pytest.mark.parametrize("dims,nu", [((64, 64, 64), (2, 2)), ((64, 64, 64), (1, 1)), ((96, 72, 80), (2, 1)),
                                      ((80, 112, 72), (1, 2)), ((128, 64, 64), (2, 2))])
 def test_blocked_kinds_equal_half_sweeps(native, dims, nu):
-    """FP32 V-cycles of one launch per half-sweep and in blocked passes (kinds 2
+    """FP32 V-cycles of one launch per half-sweep and in blocked passes (kinds 1
     to 4) and tiles, three components."""
     rng = np.random.default_rng(sum(dims))
     shape = (3, int(np.prod(dims)))
     b, x0 = rng.standard_normal(shape).astype(np.float32), rng.standard_normal(shape).astype(np.float32)
     out = []
-    for kind in (0, 2, 3, 4):
+    for kind in (0, 1, 2, 3, 4):
         print(f"[mg choice] dims={dims} nu={nu} kind={kind}", flush=True)
         mg = native.MG(dims, native.F32, ncomp=3)
         mg.set_blocked(kind)
