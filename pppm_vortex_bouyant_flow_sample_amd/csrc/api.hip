@@ -1087,9 +1087,10 @@ struct NearOverride {
 // strengths, 32 B a source, and the cell tables, 8 B a cell) than twice the
 // chip's L2 (8 XCDs x 4 MiB); at 1M sources on 128^3 the sort's order is 7%
 // faster.  The vortex near field, whose waves split a union box that wraps
-// around a row or plane, is faster in the sort's order at every size: 11.6
-// against 12.9 ms at the 8M plume on 256^3, 30.3 against 34.4 at 33.5M on
-// 512^3, 1.43 against 1.62 at 1M on 128^3.
+// around a row or plane, takes the sort's order: plumes of 8M on 256^3 11.6
+// against 12.9 ms, 33.5M on 512^3 30.3 against 34.4, 1M on 128^3 1.43 against
+// 1.62; scattered vortices (uniform, 256^3, 1 / 0.5 / 0.25 / 0.06 a cell) 7.7 / 4.1 /
+// 2.6 / 0.55 against 8.7 / 4.0 / 2.1 / 0.57.
 static pppm_status super_block_order(pppm_ctx* c, const uint32_t* keys, uint32_t m, uint32_t* spare, bool potential,
                                      uint32_t** perm) {
     *perm = nullptr;

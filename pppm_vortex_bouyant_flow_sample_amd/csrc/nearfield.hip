@@ -3,7 +3,8 @@
 // (GPU_kernel.cu:2886-2964 BiotSavartInterpolate_far_field_kernel2,
 //  2262-2436 BiotSavartPPCorrScaleMN_kernel, BiotSavartSolverImp.cpp:452-484).
 #include "pppm_internal.hpp"
-#include <cstdlib>
+#include <algorithm>
+#include <type_traits>
 
 namespace pppm {
 
@@ -456,12 +457,16 @@ __global__ void __launch_bounds__(256) k_pot_near(const float4* __restrict__ epo
 // min / max over the T points that every T consecutive lanes hold
 template <int T>
 __device__ inline float group_min(float v) {
+    if (T == 1) return v;
+    if (T == 2) return fminf(v, dpp_mov<0xB1>(v));
     v = quad_min(v);
     if (T == 8) v = fminf(v, dpp_mov<0x124>(v));
     return v;
 }
 template <int T>
 __device__ inline float group_max(float v) {
+    if (T == 1) return v;
+    if (T == 2) return fmaxf(v, dpp_mov<0xB1>(v));
     v = quad_max(v);
     if (T == 8) v = fmaxf(v, dpp_mov<0x124>(v));
     return v;
@@ -492,33 +497,47 @@ __device__ inline float transpose_reduce(float (&v)[T], int lane) {
     return v[0];
 }
 
+// When a group of points is given up for its halves: beyond vlim cells, and where
+// few vortices share a cell (SPARSE) only if that costs less.
+struct NearSplit {
+    int vlim, edge;           // edge: of a point's own box
+    float pass, row, vortex;  // instructions of a pass, of a grid row and a vortex in it
+    float mean;               // vortices a cell
+};
+
 // One wave takes T consecutive sorted evaluation points.  Their coordinates
 // sit in scalar registers and the sources in lanes: the hash rows covering the
-// union of the points' boxes are packed into one stream of sources (), those inside the union box are compacted into a ring of
-// 128, and every full window of 64 is read back one source a lane and tested
-// against the T points in turn.  A source is read from LDS once for T points
+// union of the points' boxes are packed into one stream of sources, those inside
+// the union box are compacted into a ring of 128, and every full window of 64 is
+// read back one source a lane and tested against the T points in turn.  A source is read from LDS once for T points
 // (one read per pair in k_pot_near's point-by-slice layout), and a point
 // whose box holds few of a window's sources costs little, since the sources of
 // a window follow the hash rows and the lanes that fail the box test come in
 // runs.  What bounds it is the vector issue rate: 6 instructions a source and
 // point, 20 more where some lane passes.
-// A union box of more than vlim cells (points around the end of a grid row or
-// plane, or far apart in a sparse scene) is given up for two halves of the
-// points, down to single ones: before, one wave at the end of a plane walked
-// all of its rows and ran on alone (0.79 -> 0.45 ms at 700,001 uniform
-// vortices on 96^3).
+// A union box of more than split.vlim cells (points around the end of a grid row
+// or plane, or far apart) is given up for two halves of the points, down to
+// single ones: before, one wave at the end of a plane walked all of its rows and
+// ran on alone (0.79 -> 0.45 ms at 700,001 uniform vortices on 96^3).  In sparse
+// scenes (SPARSE) eight points stretch over a large part of a grid row, whose
+// halves hold the same vortices in all: they stay together unless the halves or
+// the single points cost less (uniform on 256^3, ms, split beyond vlim / by cost:
+// 1/8 a cell 1.77 / 1.29, 1/16 1.14 / 0.55; 512^3 of 1/16 8.97 / 5.26).
 // Measured, ms a launch, k_pot_near -> here (same box, in the sort's order):
 // 8M plume 256^3 16.4 -> 11.6, 33.5M plume 512^3 45.9 -> 30.3, 2M ring 128^3
 // 28.8 -> 22.6, 1M plume 128^3 1.87 -> 1.43, 700k uniform 96^3 0.79 -> 0.37,
-// 65,536 uniform 32^3 0.153 -> 0.073.  T = 16 needs 96 VGPRs: 12.4 ms at the
-// 8M plume.
-template <int KERNEL, bool SEGMENT, typename TO, bool WIDE, int T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T == 8 ? 7 : 8)))
+// 65,536 uniform 32^3 0.153 -> 0.073; the Gaussian core's 1M plume 2.65 -> 2.61,
+// 700k uniform 0.92 -> 0.49.  T = 16 needs 96 VGPRs: 12.4 ms at the 8M plume.  At
+// eight points and seven waves a SIMD the compiler keeps 2 VGPRs in scratch (12
+// bytes a lane; 4 to 10 in the SPARSE and Gaussian forms); six waves without
+// scratch are slower: 4M plume 256^3 3.49 / 3.61, ring of 500k 96^3 3.07 / 3.11.
+template <int KERNEL, bool SEGMENT, typename TO, bool WIDE, int T, bool SPARSE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T == 8 || KERNEL == PPPM_KERNEL_GAUSSIAN ? 7 : 8)))
 k_m2p_near(const float4* __restrict__ epos, const float4* __restrict__ eoth, const uint32_t* __restrict__ eidx, uint32_t m,
        const uint32_t* __restrict__ off, const float4* __restrict__ spos, const float4* __restrict__ somg,
-       const float* __restrict__ far, uint32_t g, double invh, NearConst nc, int vlim, TO* __restrict__ ux,
+       const float* __restrict__ far, uint32_t g, double invh, NearConst nc, NearSplit split, TO* __restrict__ ux,
        TO* __restrict__ uy, TO* __restrict__ uz, uint32_t u_stride, const uint32_t* __restrict__ tperm) {
-    static_assert(T == 4 || T == 8, "group_min, group_max and transpose_reduce");
+    static_assert(T == 1 || T == 2 || T == 4 || T == 8, "group_min, group_max and transpose_reduce");
     __shared__ float4 ring[4][2][128];
     const int lane0 = threadIdx.x & 63, w = threadIdx.x >> 6;
     // groups of 256 consecutive workgroups per XCD, so each L2 serves one run
@@ -596,9 +615,38 @@ k_m2p_near(const float4* __restrict__ epos, const float4* __restrict__ eoth, con
             zhi = __builtin_amdgcn_readlane(cbnd, 5);
             ny_ = yhi - ylo + 1;
             nrows = (xlo <= xhi && ylo <= yhi && zlo <= zhi) ? (zhi - zlo + 1) * ny_ : 0;
-            if (sz > 1 && nrows * (xhi - xlo + 1) > vlim) {
-                sz >>= 1;
-                continue;
+            if (T > 1 && sz > 1 && nrows * (xhi - xlo + 1) > split.vlim) {
+                bool pays = true;
+                if constexpr (SPARSE) {
+                    // the boxes of the two halves, in lanes 0 .. 5 and 6 .. 11
+                    const int hj = lane < 12 ? lane % 6 : 0, p0 = s0 + (lane < 6 ? 0 : sz >> 1), p1 = p0 + (sz >> 1);
+                    float hv = hj < 3 ? 3.0e38f : -3.0e38f;
+                    for (int p = 0; p < T; p++) {
+                        const float v = hj % 3 == 0 ? lanef(a.x, p) : hj % 3 == 1 ? lanef(a.y, p) : lanef(a.z, p);
+                        if (p >= p0 && p < p1 && v == v) hv = hj < 3 ? fminf(hv, v) : fmaxf(hv, v);
+                    }
+                    const int hb = near_cell_bound(hv, rb, invh, gi, hj >= 3);
+                    // vortices a cell: the mean, or more in the first point's row
+                    const int cy = min(max(cell_of(lanef(a.y, s0), invh), 0), gi - 1),
+                              cz = min(max(cell_of(lanef(a.z, s0), invh), 0), gi - 1);
+                    const uint32_t row0 = __builtin_amdgcn_readfirstlane(((uint32_t)cz * g + (uint32_t)cy) * g);
+                    const float here = (float)(off[row0 + xhi + 1] - off[row0 + xlo]);
+                    const float cell = split.vortex * fmaxf(split.mean, here / (float)(xhi - xlo + 1));
+                    auto cost = [&](int nr, int nx_) { return split.row * (float)nr + cell * ((float)nr * (float)nx_); };
+                    auto half_cost = [&](int l) {
+                        const int nx_ = __builtin_amdgcn_readlane(hb, l + 3) - __builtin_amdgcn_readlane(hb, l) + 1,
+                                  ny = __builtin_amdgcn_readlane(hb, l + 4) - __builtin_amdgcn_readlane(hb, l + 1) + 1,
+                                  nz = __builtin_amdgcn_readlane(hb, l + 5) - __builtin_amdgcn_readlane(hb, l + 2) + 1;
+                        return nx_ > 0 && ny > 0 && nz > 0 ? cost(ny * nz, nx_) : 0.f;
+                    };
+                    const float halves = half_cost(0) + half_cost(6) + split.pass;
+                    const float singles = (float)sz * (cost(split.edge * split.edge, split.edge) + split.pass) - split.pass;
+                    pays = __builtin_amdgcn_readfirstlane(fminf(halves, singles) < cost(nrows, xhi - xlo + 1));
+                }
+                if (pays) {
+                    sz >>= 1;
+                    continue;
+                }
             }
             const float sbnd = near_stage_bound(bvv, rb * (1.0 + 0x1p-21), bup);
             lox = lanef(sbnd, 0);
@@ -777,7 +825,17 @@ k_m2p_near(const float4* __restrict__ epos, const float4* __restrict__ eoth, con
             }
         }
         // ---- the lanes of a point (a fixed order)
-        if (T == 4) {
+        if (T == 1) {
+            rx += dpp_mov<0xB1>(rx);
+            ry += dpp_mov<0xB1>(ry);
+            rz += dpp_mov<0xB1>(rz);
+        }
+        if (T <= 2) {
+            rx += dpp_mov<0x4E>(rx);
+            ry += dpp_mov<0x4E>(ry);
+            rz += dpp_mov<0x4E>(rz);
+        }
+        if (T <= 4) {
             rx += dpp_mov<0x124>(rx);
             ry += dpp_mov<0x124>(ry);
             rz += dpp_mov<0x124>(rz);
@@ -802,36 +860,57 @@ k_m2p_near(const float4* __restrict__ epos, const float4* __restrict__ eoth, con
     }
 }
 
+// two rounds of resident waves (256 CUs x 28) of eight points
+constexpr uint32_t kNearMany = 8u * 2u * 256u * 28u;
+
 template <int KERNEL, bool SEGMENT, bool WIDE, int T>
 static void launch_near_sized(const NearArgs& a, const NearConst& nc, hipStream_t st) {
-    // A group's union box: at most five times a single point's cells (a box
+    // A group's union box stays up to five times a single point's cells (a box
     // of 2K + 1 cells, one more where it straddles).  Limits of 2, 3, 5, 7 and
     // 12 boxes: 0.71, 0.55, 0.37, 0.36 and 0.37 ms at 700,001 uniform vortices
     // on 96^3; 16.3, 15.5 at the 8M plume (2, 3), then unchanged; 65,536
     // uniform on 32^3: 0.073 ms at 5, 0.083 at 7.
-    const int vlim = 5 * (2 * a.K + 2) * (2 * a.K + 2) * (2 * a.K + 2);
-    dim3 grid(div_up(div_up(a.m, T), 4)), blk(256);
-    if (a.u_dtype == PPPM_F64)
-        hipLaunchKernelGGL((k_m2p_near<KERNEL, SEGMENT, double, WIDE, T>), grid, blk, 0, st, a.epos, a.eoth, a.eidx, a.m,
-                           a.off, a.spos, a.somg, a.far, a.g, a.invh, nc, vlim, (double*)a.ux, (double*)a.uy,
-                           (double*)a.uz, a.u_stride, a.tperm);
-    else
-        hipLaunchKernelGGL((k_m2p_near<KERNEL, SEGMENT, float, WIDE, T>), grid, blk, 0, st, a.epos, a.eoth, a.eidx, a.m,
-                           a.off, a.spos, a.somg, a.far, a.g, a.invh, nc, vlim, (float*)a.ux, (float*)a.uy,
-                           (float*)a.uz, a.u_stride, a.tperm);
+    NearSplit split;
+    const int edge = 2 * a.K + 2;
+    split.vlim = 5 * edge * edge * edge;
+    split.pass = 200.f;
+    split.row = 8.f;
+    split.vortex = 2.5f;
+    split.mean = (float)(a.nsrc / ((double)a.g * a.g * a.g));
+    split.edge = edge;
+    auto run = [&](auto to, auto sparse) {
+        using TO = decltype(to);
+        hipLaunchKernelGGL((k_m2p_near<KERNEL, SEGMENT, TO, WIDE, T, decltype(sparse)::value>),
+                           dim3(div_up(div_up(a.m, T), 4)), dim3(256), 0, st, a.epos, a.eoth, a.eidx, a.m, a.off, a.spos,
+                           a.somg, a.far, a.g, a.invh, nc, split, (TO*)a.ux, (TO*)a.uy, (TO*)a.uz, a.u_stride, a.tperm);
+    };
+    // Sparse: groups stretch beyond vlim along a row, not only around its end.
+    // Weighing costs takes 3 to 5% of the dense scenes' time in registers (plume
+    // of 8M on 256^3 11.6 / 11.9 ms, of 1/4 vortex a cell 3.75 / 3.87).
+    const float line = edge < 6 ? 7.2f / (float)(edge * edge) : 0.2f;
+    const bool sparse = T > 1 && split.mean < line;
+    if (a.u_dtype == PPPM_F64) sparse ? run(double(), std::bool_constant<(T > 1)>()) : run(double(), std::false_type());
+    else sparse ? run(float(), std::bool_constant<(T > 1)>()) : run(float(), std::false_type());
 }
 template <int KERNEL, bool SEGMENT>
 static void launch_near(const NearArgs& a, const NearConst& nc, hipStream_t st) {
-    // Eight points a wave once that is two rounds of resident waves (256 CUs
-    // x 28); below, four points keep more waves in flight (10,007 points:
-    // 0.031 against 0.050 ms; 65,536: 0.073 against 0.079; 1M: 1.57 against
-    // 1.43).
-    const bool t8 = a.m > 8u * 2u * 256u * 28u;
+    // Eight points a wave once that is two rounds of resident waves; below, four
+    // keep more waves in flight (10,007 points: 0.031 against 0.050 ms; 65,536:
+    // 0.073 against 0.079; 1M: 1.57 against 1.43), and two or one where four
+    // leave SIMDs without a wave (us, four / two / one: 306 points 26 / 14 / 10,
+    // 2,000 25 / 19 / 10, 20,000 35 / 30, 65,536 67 / 74).  The Gaussian core's costly
+    // pairs ask for small unions of boxes: four points however many (2M plume on
+    // 128^3 8.74 against 9.14 ms, 133,613 ring on 160^3 0.43 against 0.59), but
+    // for K = 0, whose waves are mostly set-up.
     const bool wide = a.nsrc >= (1u << 28);
-    if (t8 && wide) launch_near_sized<KERNEL, SEGMENT, true, 8>(a, nc, st);
-    else if (t8) launch_near_sized<KERNEL, SEGMENT, false, 8>(a, nc, st);
-    else if (wide) launch_near_sized<KERNEL, SEGMENT, true, 4>(a, nc, st);
-    else launch_near_sized<KERNEL, SEGMENT, false, 4>(a, nc, st);
+    auto run = [&](auto t) {
+        if (wide) launch_near_sized<KERNEL, SEGMENT, true, decltype(t)::value>(a, nc, st);
+        else launch_near_sized<KERNEL, SEGMENT, false, decltype(t)::value>(a, nc, st);
+    };
+    if (a.m > kNearMany && (KERNEL != PPPM_KERNEL_GAUSSIAN || a.K < 1)) run(std::integral_constant<int, 8>());
+    else if (a.m > 3u << 12) run(std::integral_constant<int, 4>());
+    else if (a.m > 1u << 11) run(std::integral_constant<int, 2>());
+    else run(std::integral_constant<int, 1>());
 }
 
 template <int KERNEL, bool WIDE>
