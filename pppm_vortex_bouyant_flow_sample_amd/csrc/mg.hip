@@ -1983,7 +1983,9 @@ bool MGHier<T>::has_temp(const int (*d)[3], int L, int l) {
     if (sizeof(T) == 4) return true;
     const size_t n = (size_t)d[l][0] * d[l][1] * d[l][2];
     const bool tail = l == L - 2 && L >= 3 && n <= (size_t)kTailMax && tail_fits<T>(d[l]);
-    return n <= (size_t)1 << 24 && l < L - 1 && !tail;
+    const bool tiles = n < kTileCells && d[l][0] > 1 && d[l][1] > 1 && d[l][2] > 1;
+    const bool wide = n <= (size_t)1 << 24 && !(d[l][0] & 1);
+    return l < L - 1 && !tail && (tiles || wide);
 }
 
 template <typename T>
@@ -1992,8 +1994,8 @@ size_t MGHier<T>::bytes_for(int nx, int ny, int nz, int ncomp) {
     const int L = level_dims(nx, ny, nz, d);
     size_t b = 0;
     for (int l = 0; l < L; l++) {
-        const size_t n = (size_t)d[l][0] * d[l][1] * d[l][2] * ncomp * sizeof(T);
-        b += (l > 0 ? 2 : 0) * n + (has_temp(d, L, l) ? n : 0);
+        const size_t n = (size_t)d[l][0] * d[l][1] * d[l][2] * ncomp;
+        b += ((l > 0 ? 2 : 0) * n + (has_temp(d, L, l) ? (n + 63) & ~(size_t)63 : 0)) * sizeof(T);
     }
     const int x = d[L - 1][0], y = d[L - 1][1], z = d[L - 1][2];
     // coarse tables (two bases, <= 3 * 512^2 doubles each at most) and norm partials
@@ -2021,16 +2023,35 @@ pppm_status MGHier<T>::init(int nx, int ny, int nz, int ncomp) {
     {
         if (std::is_same<T, float>::value) rbc_prime();
         else (void)cu_count();
-        // out-of-place targets of the blocked passes
-        for (int l = 0; l < L_; l++) {
-            if (!has_temp(d_, L_, l)) continue;
-            size_t n = cells(l) * ncomp_;
-            if (hipMalloc(&t_[l], n * sizeof(T)) != hipSuccess) {
-                release_locked();
-                return PPPM_ERR_NOMEM;
-            }
-            bytes_ += n * sizeof(T);
+    }
+    // out-of-place targets; the FP64 passes run in place without (the same
+    // values, more launches), so a card that has no room for them serves the
+    // hierarchy all the same
+    auto temps = [&]() {
+        // one allocation (each takes about 40 us)
+        size_t all = 0;
+        auto each = [&](auto f) {
+            for (int l = 0; l < L_; l++)
+                if (has_temp(d_, L_, l)) f(l, (cells(l) * ncomp_ + 63) & ~(size_t)63);
+        };
+        each([&](int, size_t n) { all += n; });
+        if (all == 0) return true;
+        if (hipMalloc(&tbase_, all * sizeof(T)) != hipSuccess) {
+            (void)hipGetLastError();
+            tbase_ = nullptr;
+            return false;
         }
+        bytes_ += all * sizeof(T);
+        T* p = tbase_;
+        each([&](int l, size_t n) {
+            t_[l] = p;
+            p += n;
+        });
+        return true;
+    };
+    if (std::is_same<T, float>::value && !temps()) {
+        release_locked();
+        return PPPM_ERR_NOMEM;
     }
     for (int l = 1; l < L_; l++) {
         size_t n = cells(l) * ncomp_;
@@ -2055,6 +2076,7 @@ pppm_status MGHier<T>::init(int nx, int ny, int nz, int ncomp) {
               2 * (size_t)ncomp_ * sizeof(double);
     PPPM_HIP_TRY(hipMemcpy(tab_cons_, tc.data(), tc.size() * sizeof(double), hipMemcpyHostToDevice));
     PPPM_HIP_TRY(hipMemcpy(tab_ref_, tr.data(), tr.size() * sizeof(double), hipMemcpyHostToDevice));
+    if (std::is_same<T, double>::value) (void)temps();
     return PPPM_OK;
 }
 
@@ -2070,8 +2092,8 @@ void MGHier<T>::release_locked() {
         if (p) (void)hipFree(p);
     for (T* p : b_)
         if (p) (void)hipFree(p);
-    for (T* p : t_)
-        if (p) (void)hipFree(p);
+    if (tbase_) (void)hipFree(tbase_);
+    tbase_ = nullptr;
     x_.clear();
     b_.clear();
     t_.clear();

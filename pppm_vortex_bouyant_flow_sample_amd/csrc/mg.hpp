@@ -77,8 +77,9 @@ class MGHier {
     // has_temp is false)
     T* temp(int l) { return t_[l]; }
     // whether level l of L has an out-of-place target: every float level
-    // (blocked smoother, tile passes), the double ones up to 256^3 (tile
-    // passes, k_rb4) but those of the small levels' one launch
+    // (blocked smoother, tile passes), the double ones that take tile passes
+    // (below kTileCells) or k_rb4 (even nx, up to 256^3) but not the small
+    // levels' one launch.  +134 MB a component at 256^3 in FP64.
     static bool has_temp(const int (*d)[3], int L, int l);
     double* partials() { return part_; }
     // the reduced norms, 2 per component (||r||^2, ||b||^2), after the partials
@@ -138,7 +139,8 @@ class MGHier {
     int L_ = 0, ncomp_ = 1, cap_ = 1;
     int d_[16][3];
     std::vector<T*> x_, b_;       // levels >= 1
-    std::vector<T*> t_;           // all levels: blocked-smoother ping-pong (float)
+    std::vector<T*> t_;           // out-of-place targets (has_temp), in tbase_
+    T* tbase_ = nullptr;
     double* tab_cons_ = nullptr;  // coarse eigenbasis, consistent ghosts
     double* tab_ref_ = nullptr;   // coarse eigenbasis, zero ghosts
     double* part_ = nullptr;      // norm partial sums
