@@ -2244,8 +2244,16 @@ static pppm_status launch_rb2(const TbArgs& a, int ncomp, int kind, hipStream_t 
     const bool beta = a.beta != 0.f;
     if (two_iter && (kind < 4 || (a.nx & 1) != 0)) return PPPM_ERR_INVALID;
     if (two_iter) {
-        if (beta) launch_rb4<float, R, P, Z, true>(a, ncomp, st);
-        else launch_rb4<float, R, P, Z, false>(a, ncomp, st);
+        // from zero only with the residual, and with it from an iterate only
+        // on the finest level, which has no ghost factor
+        if constexpr (!R && Z) return PPPM_ERR_INVALID;
+        else if constexpr (R && !Z) {
+            if (beta) return PPPM_ERR_INVALID;
+            launch_rb4<float, R, P, Z, false>(a, ncomp, st);
+        } else {
+            if (beta) launch_rb4<float, R, P, Z, true>(a, ncomp, st);
+            else launch_rb4<float, R, P, Z, false>(a, ncomp, st);
+        }
     } else if (kind >= 2 && (a.nx & 1) == 0) {
         if (R || kind == 3) {
             if (beta) launch_rbc<R, P, Z, true, 6>(a, ncomp, st);
