@@ -50,7 +50,9 @@ def test_component_equals_alone(native, dims, ncomp, dtype, nu, sched):
 
 
 @pytest.mark.parametrize("dims,nu", [((64, 64, 64), (2, 2)), ((64, 64, 64), (1, 1)), ((96, 72, 80), (2, 1)),
-                                     ((80, 112, 72), (1, 2)), ((128, 64, 64), (2, 2))])
+                                     ((80, 112, 72), (1, 2)), ((128, 64, 64), (2, 2)),
+                                     ((62, 58, 60), (2, 2)), ((62, 58, 60), (2, 1)),  # partial tiles of 16^3
+                                     ((46, 62, 30), (2, 2))])                         # ... and of 8^3
 def test_blocked_kinds_equal_half_sweeps(native, dims, nu):
     """FP32 V-cycles of one launch per half-sweep and in blocked passes (kinds 1
     to 4) and tiles, three components."""
