@@ -1994,8 +1994,8 @@ size_t MGHier<T>::bytes_for(int nx, int ny, int nz, int ncomp) {
     const int L = level_dims(nx, ny, nz, d);
     size_t b = 0;
     for (int l = 0; l < L; l++) {
-        const size_t n = (size_t)d[l][0] * d[l][1] * d[l][2] * ncomp;
-        b += ((l > 0 ? 2 : 0) * n + (has_temp(d, L, l) ? (n + 63) & ~(size_t)63 : 0)) * sizeof(T);
+        const size_t n = ((size_t)d[l][0] * d[l][1] * d[l][2] * ncomp + 63) & ~(size_t)63;
+        b += ((l > 0 ? 2 : 0) + (has_temp(d, L, l) ? 1 : 0)) * n * sizeof(T);
     }
     const int x = d[L - 1][0], y = d[L - 1][1], z = d[L - 1][2];
     // coarse tables (two bases, <= 3 * 512^2 doubles each at most) and norm partials
@@ -2053,13 +2053,22 @@ pppm_status MGHier<T>::init(int nx, int ny, int nz, int ncomp) {
         release_locked();
         return PPPM_ERR_NOMEM;
     }
-    for (int l = 1; l < L_; l++) {
-        size_t n = cells(l) * ncomp_;
-        if (hipMalloc(&x_[l], n * sizeof(T)) != hipSuccess || hipMalloc(&b_[l], n * sizeof(T)) != hipSuccess) {
+    if (L_ > 1) {
+        auto room = [&](int l) { return (cells(l) * ncomp_ + 63) & ~(size_t)63; };
+        size_t all = 0;
+        for (int l = 1; l < L_; l++) all += 2 * room(l);
+        if (hipMalloc(&xbase_, all * sizeof(T)) != hipSuccess) {
+            xbase_ = nullptr;
             release_locked();
             return PPPM_ERR_NOMEM;
         }
-        bytes_ += 2 * n * sizeof(T);
+        bytes_ += all * sizeof(T);
+        T* p = xbase_;
+        for (int l = 1; l < L_; l++) {
+            x_[l] = p;
+            b_[l] = p + room(l);
+            p += 2 * room(l);
+        }
     }
     const int* dc = d_[L_ - 1];
     std::vector<double> tc = coarse_tables(dc[0], dc[1], dc[2], mg_beta(L_ - 1));
@@ -2088,12 +2097,9 @@ void MGHier<T>::release() {
 
 template <typename T>
 void MGHier<T>::release_locked() {
-    for (T* p : x_)
-        if (p) (void)hipFree(p);
-    for (T* p : b_)
-        if (p) (void)hipFree(p);
+    if (xbase_) (void)hipFree(xbase_);
     if (tbase_) (void)hipFree(tbase_);
-    tbase_ = nullptr;
+    xbase_ = tbase_ = nullptr;
     x_.clear();
     b_.clear();
     t_.clear();

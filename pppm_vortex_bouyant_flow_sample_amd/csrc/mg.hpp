@@ -138,7 +138,8 @@ class MGHier {
     void release_locked();  // release() with runtime_mutex() already held
     int L_ = 0, ncomp_ = 1, cap_ = 1;
     int d_[16][3];
-    std::vector<T*> x_, b_;       // levels >= 1
+    std::vector<T*> x_, b_;       // levels >= 1, in xbase_
+    T* xbase_ = nullptr;
     std::vector<T*> t_;           // out-of-place targets (has_temp), in tbase_
     T* tbase_ = nullptr;
     double* tab_cons_ = nullptr;  // coarse eigenbasis, consistent ghosts
