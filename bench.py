@@ -400,11 +400,12 @@ def run_multigrid(N, g, cycles=10, nu1=2, nu2=2):
     """The multigrid alone, as every evaluation runs it: V(nu1,nu2) cycles of
     the tolerance-driven form on three FP32 components of a g^3 grid (random
     right-hand side), `cycles` cycles back to back after two untimed ones,
-    timed with HIP events on the stream they are launched on.  Algorithmic
-    bytes per cycle: 3 [12 (nu1 + nu2) + 17] (8/7) g^3 (each smoothing
-    iteration reads x and b and writes x once, 4 bytes each; 17 bytes per
-    cell for residual, restriction and prolongation; the coarser levels add
-    1/7)."""
+    timed with HIP events on the stream they are launched on.  Bytes are those
+    that the passes have to move: a pass of two iterations reads x and b and
+    writes x once, 4 bytes each, and takes the residual's restriction or the
+    prolongation along (half a byte a cell each way); with p = ceil(nu1 / 2) +
+    ceil(nu2 / 2) passes that is 12 p + 1 bytes a cell on the finest level and 4
+    less on the coarser ones (1/7 of the cells), which start from zero."""
     G = g ** 3
     rng = np.random.default_rng(7)
     b = N.DeviceBuffer.from_array(rng.standard_normal(3 * G).astype(np.float32))
@@ -418,7 +419,8 @@ def run_multigrid(N, g, cycles=10, nu1=2, nu2=2):
     t.stop(None)
     N.synchronize()
     ms = t.ms() / cycles
-    algo = 3 * (12 * (nu1 + nu2) + 17) * (8 / 7) * G
+    p = -(-nu1 // 2) - (-nu2 // 2)
+    algo = 3 * ((12 * p + 1) + (12 * p - 3) / 7) * G
     return {"bound": "hbm", "kernel": f"V({nu1},{nu2}) cycle, 3 x {g}^3 FP32", "ms_per_cycle": ms,
             "algorithmic_bytes": algo, "achieved": algo / (ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": algo / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "cycles_timed": cycles}
