@@ -311,9 +311,11 @@ pppm_status pppm_mg_vcycles(pppm_mg *mg, void *x, const void *b, int32_t nu1, in
 /* iters red-black SOR iterations (odd colour first, MultiGrid_kernel.cu:722-820)
  * on the finest level, in place on x.  blocked (PPPM_F32 only): 0 one launch
  * per half-sweep; 1 temporally blocked LDS passes; 2 colour-split blocked
- * passes (four-plane ring); 3 the same with a six-plane ring; 4 kind 3 with
- * two iterations per pass while two remain.  Kinds 2 to 4 take kind 1's
- * kernel when nx is odd. */
+ * passes (four-plane ring); 3 the same with a six-plane ring; 4 passes of two
+ * iterations, an odd one by kind 2.  Kinds 2 to 4 take kind 1's kernel when nx
+ * is odd.  The results are the same, bit for bit, whichever it is.  Kinds 1 to
+ * 4 pass through the handle's buffers: their calls on one handle must not
+ * overlap.  Kind 0 touches x and b alone, in PPPM_F64 always. */
 pppm_status pppm_mg_smooth(pppm_mg *mg, void *x, const void *b, int32_t iters, double omega, int32_t blocked,
                            void *hip_stream);
 /* PPPM_F32 V-cycles on levels at or above the blocked threshold (below):
@@ -337,7 +339,7 @@ pppm_status pppm_mg_set_blocked_min_cells(pppm_mg *mg, uint64_t cells);
  * 16^3) with the coarsest solve in one launch, one workgroup per component
  * with the iterates in LDS; 0 runs them as one launch per half-sweep,
  * residual, restriction, coarsest solve and prolongation.  Both give the
- * same results, bit for bit. */
+ * same results, bit for bit.  PPPM_F64 cycles always take the one launch. */
 pppm_status pppm_mg_set_small_levels(pppm_mg *mg, int32_t one_launch);
 
 /* ---- device memory (MemoryOperation.cuh:13-29 semantics) -------------------- */

@@ -440,7 +440,7 @@ static void launch_curl_far_k(const TP* psi, const float* wgrid, float* far, con
                               float h3, TC half_invh, float cd, hipStream_t st) {
     constexpr int TY = kCfThreads / (TX / 2);
     const uint32_t tiles = div_up(g, TX) * div_up(g, TY);
-    // planes per workgroup: about three workgroups per CU in all; longer runs
+    // planes per workgroup: about three workgroups per CU (of 256) in all; longer runs
     // (up to 32) repeat fewer of the 2K planes around them, shorter ones (down
     // to 2) keep the chip busy on small grids
     const int zc = std::max(2, std::min(32, (int)div_up(g * tiles, 768)));
@@ -451,8 +451,8 @@ static void launch_curl_far_k(const TP* psi, const float* wgrid, float* far, con
         case 2: hipLaunchKernelGGL((k_curl_far<TP, TC, 2, TX, EVEN>), grid, blk, 0, st, psi, wgrid, far, dir, g, h3, half_invh, cd, zc); break;
         case 3:
         case 4: {
-            // as many workgroups as fit the chip's LDS at once: three of 45 KB
-            // a CU (K = 3), two of 69 KB (K = 4)
+            // as many workgroups as fit the LDS of 256 CUs at once: three of
+            // 45 KB a CU (K = 3), two of 69 KB (K = 4)
             const uint32_t tp = div_up(g, kCfTX) * div_up(g, kCfTY);
             const int zp = std::max(2, std::min(16, (int)div_up(g * tp, K == 3 ? 768 : 512)));
             const dim3 gp(tp, div_up(g, zp));
@@ -470,8 +470,9 @@ pppm_status launch_curl_far_impl(const void* psi, int psi_dtype, const float* wg
     const double half_invh = 0.5 * (1.0 / h);
     // vortex-in-cell (K < 0): the far-field buffer is the grid velocity itself
     const float cd = K < 0 ? 0.0f : (float)(kRefDiagPsi * h * h * half_invh);
-    // 64-cell tiles along x, or 32 where they would leave a third of the
-    // threads or more without cells
+    // 64-cell tiles along x, or 32 where the last of 64 would be partial and
+    // they are two at most (96^3: a quarter of the threads without cells); past
+    // 128 cells a partial tile costs less than the halo of twice as many
     const bool t64 = g % 64 == 0 || g > 128;
     auto run = [&](auto* ps, auto hi, auto t64_, auto even) {
         using TP = std::remove_const_t<std::remove_pointer_t<decltype(ps)>>;

@@ -412,7 +412,8 @@ __global__ void __launch_bounds__(256) k_rb2(TbArgs a) {
 
 // Colour-split blocked smoother: the pass of k_rb2 (z planes streamed through
 // LDS rings, halos recomputed, out of place; one red-black iteration) with
-// each LDS plane split by colour.  Row ly of colour c holds at index m the colour-c cell of the cell pair (2m, 2m + 1) of that row.  Every
+// each LDS plane split by colour.  Row ly of colour c holds at index m the
+// colour-c cell of the cell pair (2m, 2m + 1) of that row.  Every
 // neighbour of a colour-c cell is of colour 1 - c: at index m in the rows
 // above and below and in the planes before and after, and at m + s - 1 and
 // m + s in its own row (s = 1 if the cell is the pair's second), so the reads
@@ -1213,9 +1214,9 @@ __global__ void __launch_bounds__(256) k_prolong(T* __restrict__ x, const T* __r
 //
 // us of one V(2,2) cycle's level, three components, before -> here: 32^3 50
 // (11 launches) -> 16.5 (2), 64^3 51 (k_rbc) -> 34; FP64, one component: V(4,4)
-// at 64^3 and below 19 launches of 4.2 -> 4 of 11.  In FP32 the blocked passes
-// (k_rb4) are the faster from 72^3 (tb_min_cells_).  1024 threads take a 16^3
-// tile, 576 an 8^3 one.
+// at 64^3 and below 19 launches of 4.2 -> 4 of 11.  Where the FP32 blocked
+// passes (k_rb4) are the faster: MGHier::blocked_level.  1024 threads take a
+// 16^3 tile, 576 an 8^3 one.
 template <typename T>
 struct TileArgs {
     const T* xin;  // level before the pass (null: zero)

@@ -120,7 +120,7 @@ extern "C" void sortParticles(uint32_t* dGridParticleHash, uint32_t* dGridPartic
 // the process.  Host code never passes `scratch` itself to a kernel: its address
 // on a device comes from hipGetSymbolAddress, looked up once per device with that
 // device current, and only that address is used.  The sort writes every scratch
-// word it later reads (histograms, scan partials, ping-pong halves), so nothing
+// word it later reads (histograms, digit totals, ping-pong halves), so nothing
 // needs clearing between calls.  Calls that overlap on one device share the array
 // and race.
 namespace {
