@@ -470,9 +470,10 @@ pppm_status launch_curl_far_impl(const void* psi, int psi_dtype, const float* wg
     const double half_invh = 0.5 * (1.0 / h);
     // vortex-in-cell (K < 0): the far-field buffer is the grid velocity itself
     const float cd = K < 0 ? 0.0f : (float)(kRefDiagPsi * h * h * half_invh);
-    // 64-cell tiles along x, or 32 where the last of 64 would be partial and
-    // they are two at most (96^3: a quarter of the threads without cells); past
-    // 128 cells a partial tile costs less than the halo of twice as many
+    // 64-cell tiles along x, or 32 where one of two would be partial (us, FP64
+    // psi, 64 / 32: 66^3 38 / 25, 80^3 44 / 39, 96^3 47 / 45, 120^3 61 / 62).  Past
+    // 128 cells 64 throughout: even where the last is well filled (200^3 253 /
+    // 253), behind where it is not (160^3 129 / 114, 288^3 580 / 486)
     const bool t64 = g % 64 == 0 || g > 128;
     auto run = [&](auto* ps, auto hi, auto t64_, auto even) {
         using TP = std::remove_const_t<std::remove_pointer_t<decltype(ps)>>;
