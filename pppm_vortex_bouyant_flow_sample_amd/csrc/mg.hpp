@@ -149,7 +149,10 @@ class MGHier {
     size_t bytes_ = 0;
     int tb_ = 4;
     // Tile passes below kTileCells cells a component, in 16^3 tiles from
-    // kTile16Cells cells over all components.
+    // kTile16Cells cells over all components: fewer cells leave CUs without a
+    // workgroup, more are worth the smaller halo (us of a V(2,2) cycle, all
+    // levels in 8^3 / 16^3 tiles: 48^3 43 / 58, x 3 59 / 70, x 6 76 / 72; 64^3 55 /
+    // 74, x 2 79 / 75, x 6 151 / 105; 32^3 x 6 36 / 39, x 16 61 / 41).
     static constexpr size_t kTileCells = (size_t)1 << 19;
     static constexpr size_t kTile16Cells = (size_t)1 << 19;
     // FP32 blocked passes (blocked_level) from kBlockedMin cells (us down and up,
